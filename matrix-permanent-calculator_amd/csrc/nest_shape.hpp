@@ -19,6 +19,17 @@ constexpr int kMinPairN = 16;
 // Smallest n with nested variants (tails of Gray columns 1 and 2 shared too).
 constexpr int kMinNestN = 24;
 
+// Orders whose FP64 pass is the class walk (ryser_class_impl.hpp) when its
+// instruction count per subset is below kClassGain of the plain walk's 2n + 2.
+// Measured, one call: n = 20 51 -> 55 us and n = 23 58 -> 60 us (its host
+// preparation costs what the kernel gains), n = 27 137 -> 122 us; full
+// matrices, where both walks execute the same instructions and the Gray
+// kernels issue them at 97 % of the cycles: n = 24 67 -> 90 us, n = 28 266 ->
+// 308 us.  Above kMaxNestN no walk of every subset finishes.
+constexpr int kMinClassN = 24;
+constexpr int kMaxClassN = kMaxNestN;
+constexpr double kClassGain = 0.75;
+
 // Walk shape: Gray column l < 3 touches rows [0, k_l) only (k0 <= k1 <= k2).
 struct NestShape {
   int k0, k1, k2;

@@ -25,6 +25,7 @@
 
 #include "../../include/perman_hip.h"
 #include "perman_internal.hpp"
+#include "ryser_class.hpp"
 #include "ryser_host.hpp"
 #include "ryser_kernels.hpp"
 
@@ -63,6 +64,11 @@ struct perm_plan {
   perm::DenseLaunch L{};
   int unroll_bits = 0;
   int walk_bits = 0, high_bits = 0;  // split of the n-1 Gray columns
+  // split the FP64 error estimate is stated for (error_estimate)
+  int est_walk_bits = 0, est_high_bits = 0;
+  bool classed = false;  // the FP64 pass is the class walk
+  size_t table_doubles = 0;  // ClassTables::data
+  perm::ClassMatrix cls{};
   int nu = 0;             // rows touched by Gray column 0 for the FP64 kernel (n: none)
   int nu1 = 0, nu2 = 0;   // rows touched by Gray columns 0-1 and 0-2 (n: not nested)
   bool integral = false;  // every entry an integer of magnitude < 2^31
@@ -105,12 +111,12 @@ DeviceCache& device_cache(int dev) {
   return *table[dev];
 }
 
-// Device layout of a plan: column store, x0, result record, sample ids and
-// records, then the workgroup records and their weights (the last two are a
-// separate arena in owning plans).
+// Device layout of a plan: column store, x0, the class walk's tables (these
+// three uploaded as one), result record, sample ids and records, then the workgroup records and their
+// weights (the last two are a separate arena in owning plans).
 struct PlanLayout {
-  size_t col, x, res, ids, vrec, part, z;
-  size_t fixed() const { return col + x + res + ids + vrec; }
+  size_t col, x, cls, res, ids, vrec, part, z;
+  size_t fixed() const { return col + x + cls + res + ids + vrec; }
   size_t total() const { return fixed() + part + z; }
 };
 
@@ -118,8 +124,10 @@ using perm::kVerifyUnits;
 
 uint64_t blocks_of(uint64_t lanes) { return (lanes + 255) / 256; }
 
-PlanLayout plan_layout(const perm_plan* P, size_t col_doubles) {
+PlanLayout plan_layout(const perm_plan* P) {
   PlanLayout l;
+  const size_t col_doubles = (size_t)(2 * (P->n - 1) + 1) * P->n;
+  l.cls = align_up(P->table_doubles * sizeof(double), 256);
   l.col = align_up(col_doubles * sizeof(double), 256);
   l.x = align_up(2 * (size_t)P->n * sizeof(double), 256);  // start vector and its low parts
   l.part = align_up(blocks_of(1ull << P->high_bits) * sizeof(perm::Partial), 256);
@@ -132,26 +140,42 @@ PlanLayout plan_layout(const perm_plan* P, size_t col_doubles) {
 
 // Fill the geometry of a plan for order n and return the device bytes it
 // needs.
-size_t layout_plan(perm_plan* P, int n, size_t col_doubles) {
+size_t layout_plan(perm_plan* P, int n, const Prepared& prep) {
   P->n = n;
+  P->classed = prep.classed;
+  P->table_doubles = prep.classed ? prep.tables.data.size() : 0;
   P->unroll_bits = perm::dense_unroll_bits(n);
   const perm::Split sp = perm::choose_split(n, P->unroll_bits, env_int("PERMAN_WALK_BITS", 0));
-  P->walk_bits = sp.walk_bits;
-  P->high_bits = sp.high_bits;
+  P->walk_bits = P->est_walk_bits = sp.walk_bits;
+  P->high_bits = P->est_high_bits = sp.high_bits;
+  if (P->classed) {
+    // a class walk workgroup covers the subsets of 256 Gray lanes; the
+    // estimate keeps the Gray split's drift (the class walk has less)
+    P->walk_bits = perm::class_walk_bits(n) + perm::kClassBits + perm::kClassLaneBits - 8;
+    P->high_bits = n - 1 - P->walk_bits;
+  }
   P->L.n = n;
-  return plan_layout(P, col_doubles).total();
+  return plan_layout(P).total();
 }
 
 // Bind the fixed regions at `base`; with `records`, also the workgroup
 // records of all 2^h lanes and their weights right after them.
-void bind_plan_memory(perm_plan* P, void* base, size_t col_doubles, bool records = true) {
-  const PlanLayout l = plan_layout(P, col_doubles);
+void bind_plan_memory(perm_plan* P, const Prepared& prep, void* base, bool records = true) {
+  const PlanLayout l = plan_layout(P);
   char* b = (char*)base;
   P->L.colpm = (const double*)b;
   P->L.x0 = (const double*)(b + l.col);
-  P->L.result = (perm::Partial*)(b + l.col + l.x);
-  P->ids = (uint32_t*)(b + l.col + l.x + l.res);
-  P->vrec = (perm::Partial*)(b + l.col + l.x + l.res + l.ids);
+  char* r = b + l.col + l.x + l.cls;
+  P->L.result = (perm::Partial*)r;
+  P->ids = (uint32_t*)(r + l.res);
+  P->vrec = (perm::Partial*)(r + l.res + l.ids);
+  if (prep.classed) {
+    const perm::ClassTables& t = prep.tables;
+    const double* d = (const double*)(b + l.col + l.x);
+    P->cls = {d, d + t.lane, d + t.block, d + t.walk, prep.plan.live, P->n,
+              perm::class_walk_bits(P->n), 0};
+    P->cls.block_bits = P->n - 1 - perm::kClassBits - P->cls.walk_bits - perm::kClassLaneBits;
+  }
   if (records) {
     P->L.partials = (perm::Partial*)(b + l.fixed());
     P->zdev = (double*)(b + l.fixed() + l.part);
@@ -206,28 +230,41 @@ void configure_passes(perm_plan* P, int mode) {
   L.total_blocks = L.main.blocks;
 }
 
-int upload_plan(perm_plan* P, const std::vector<double>& colstore, const std::vector<double>& x0) {
-  HIP_TRY(hipMemcpyAsync((void*)P->L.colpm, colstore.data(), colstore.size() * sizeof(double),
+// Enqueue the upload of the column store, start vector and class tables.
+int upload_plan(perm_plan* P, const Prepared& prep) {
+  HIP_TRY(hipMemcpyAsync((void*)P->L.colpm, prep.cs.data(), prep.cs.size() * sizeof(double),
                          hipMemcpyHostToDevice, P->stream));
-  HIP_TRY(hipMemcpyAsync((void*)P->L.x0, x0.data(), x0.size() * sizeof(double),
+  HIP_TRY(hipMemcpyAsync((void*)P->L.x0, prep.x0.data(), prep.x0.size() * sizeof(double),
                          hipMemcpyHostToDevice, P->stream));
-  // the host vectors die on return: wait for the copies
-  HIP_TRY(hipStreamSynchronize(P->stream));
+  if (prep.classed)
+    HIP_TRY(hipMemcpyAsync((void*)P->cls.records, prep.tables.data.data(),
+                           prep.tables.data.size() * sizeof(double), hipMemcpyHostToDevice,
+                           P->stream));
   return PERM_OK;
+}
+
+// Enqueue the walk of P->L.main's workgroups [b0, b1) in P->L.mode: the
+// class walk in FP64 for a classed plan, else the Gray kernels.  Record of
+// workgroup b to L.partials[b - record_begin].
+hipError_t launch_walk(perm_plan* P, uint64_t b0, uint64_t b1, uint64_t record_begin) {
+  if (P->classed && P->L.mode == 0)
+    return perm::launch_class({P->cls, P->L.partials + (b0 - record_begin), b0, b1}, P->stream);
+  perm::DenseLaunch L = P->L;
+  L.main.block_begin = b0;
+  L.main.block_end = b1;
+  L.main.record_begin = record_begin;
+  return perm::launch_dense_pass_only(L, P->stream);
 }
 
 // Create an owning plan (its own stream, events and device memory).
 int make_plan(int n, const Prepared& prep, perm_plan** out) {
-  const std::vector<double>& colstore = prep.cs;
-  const std::vector<double>& x0 = prep.x0;
-  const bool integral = prep.integral;
   if (int s = select_device()) return s;
   auto* P = new perm_plan();
   P->device = perm::current_device();
   set_shape(P, n, prep);
-  P->integral = integral;
-  layout_plan(P, n, colstore.size());
-  P->mem.bytes = plan_layout(P, colstore.size()).fixed();  // records: ensure_records
+  P->integral = prep.integral;
+  layout_plan(P, n, prep);
+  P->mem.bytes = plan_layout(P).fixed();  // records: ensure_records
   auto cleanup = [&](int code, const std::string& msg) {
     perm_plan_destroy(P);
     return fail(code, msg);
@@ -240,12 +277,11 @@ int make_plan(int n, const Prepared& prep, perm_plan** out) {
     return cleanup(PERM_ERR_HIP, std::string("hipEventCreate: ") + hipGetErrorString(e));
   if ((e = hipMalloc(&P->mem.base, P->mem.bytes)) != hipSuccess)
     return cleanup(PERM_ERR_HIP, std::string("hipMalloc: ") + hipGetErrorString(e));
-  bind_plan_memory(P, P->mem.base, colstore.size(), false);
-  if (upload_plan(P, colstore, x0) != PERM_OK ||
-      (e = hipStreamSynchronize(P->stream)) != hipSuccess) {
-    std::string msg = *perm::last_error() ? std::string(perm::last_error()) : hipGetErrorString(e);
-    return cleanup(PERM_ERR_HIP, "upload: " + msg);
-  }
+  bind_plan_memory(P, prep, P->mem.base, false);
+  if (upload_plan(P, prep) != PERM_OK)
+    return cleanup(PERM_ERR_HIP, "upload: " + std::string(perm::last_error()));
+  if ((e = hipStreamSynchronize(P->stream)) != hipSuccess)
+    return cleanup(PERM_ERR_HIP, std::string("upload: ") + hipGetErrorString(e));
   *out = P;
   return ok();
 }
@@ -257,7 +293,11 @@ int run_pass(perm_plan* P, int mode, perm::Partial& r, float& ms, float& main_ms
   // one workgroup (n <= 19): its record is the sum, the walk the only kernel
   const bool single = P->L.total_blocks <= 1;
   HIP_TRY(hipEventRecord(P->ev0, P->stream));
-  HIP_TRY(perm::launch_dense(P->L, P->stream, single ? nullptr : P->evm));
+  HIP_TRY(launch_walk(P, 0, P->L.total_blocks, 0));
+  if (!single) {
+    HIP_TRY(hipEventRecord(P->evm, P->stream));
+    HIP_TRY(perm::launch_reduce(P->L.partials, P->L.total_blocks, P->L.result, P->stream));
+  }
   HIP_TRY(hipEventRecord(P->ev1, P->stream));
   HIP_TRY(hipMemcpyAsync(&r, single ? P->L.partials : P->L.result, sizeof(r),
                          hipMemcpyDeviceToHost, P->stream));
@@ -280,7 +320,8 @@ void fill_result(const perm_plan* P, const perm::Partial& r, int mode, perm_resu
                                          P->unroll_bits, P->integral, mode);
   out->subsets = std::ldexp(1.0, n - 1);
   out->err_est = perm::error_estimate(scale * scale * r.sq_sum, scale * scale * r.sq_run,
-                                      out->value, n, P->walk_bits, P->high_bits, mode,
+                                      out->value, n, mode == 0 ? P->est_walk_bits : P->walk_bits,
+                                      mode == 0 ? P->est_high_bits : P->high_bits, mode,
                                       P->integral);
   if (perm::integer_sum_exact(P->integral, P->product_bits, out->abs_sum, scale, n))
     out->err_bound = out->err_est = 0.0;  // exact arithmetic throughout
@@ -317,7 +358,7 @@ int verify_sampled(perm_plan* P, perm_result* out, uint32_t& units_out, float& m
   const uint64_t blocks = P->L.total_blocks;
   // variance weights of the FP64 pass's workgroup records, formed on the
   // device (8 bytes per record come back instead of the record)
-  const double run_weight = std::ldexp(1.0, P->walk_bits - 1) + (double)P->high_bits;
+  const double run_weight = std::ldexp(1.0, P->est_walk_bits - 1) + (double)P->est_high_bits;
   HIP_TRY(perm::launch_unit_weights(P->L.partials, blocks, run_weight, P->zdev, P->stream));
   P->zhost.resize(blocks);
   HIP_TRY(hipMemcpyAsync(P->zhost.data(), P->zdev, blocks * sizeof(double),
@@ -413,7 +454,6 @@ int plan_run_impl(perm_plan* P, int mode, perm_result* out) {
 // Bind a borrowed plan to the per-device cache and upload a prepared
 // matrix (caller holds C.mu).
 int bind_oneshot(int n, const Prepared& prep, DeviceCache& C, perm_plan& P) {
-  const std::vector<double>& cs = prep.cs;
   if (!C.stream) {
     HIP_TRY(hipStreamCreateWithFlags(&C.stream, hipStreamNonBlocking));
     HIP_TRY(hipEventCreate(&C.ev0));
@@ -428,7 +468,7 @@ int bind_oneshot(int n, const Prepared& prep, DeviceCache& C, perm_plan& P) {
   P.evm = C.evm;
   P.integral = prep.integral;
   set_shape(&P, n, prep);
-  const size_t need = layout_plan(&P, n, cs.size());
+  const size_t need = layout_plan(&P, n, prep);
   if (need > C.bytes) {
     if (C.base) HIP_TRY(hipFree(C.base));
     C.base = nullptr;
@@ -436,12 +476,14 @@ int bind_oneshot(int n, const Prepared& prep, DeviceCache& C, perm_plan& P) {
     HIP_TRY(hipMalloc(&C.base, need));
     C.bytes = need;
   }
-  bind_plan_memory(&P, C.base, cs.size());
+  bind_plan_memory(&P, prep, C.base);
   // one asynchronous copy from pinned staging in the device layout; the
   // stream orders the kernels after it, and the staging is reused only by
   // the next call under C.mu, after this call's final synchronisation
   const size_t col_bytes = (const char*)P.L.x0 - (const char*)P.L.colpm;
-  const size_t up = col_bytes + prep.x0.size() * sizeof(double);
+  const size_t x_end = col_bytes + prep.x0.size() * sizeof(double);
+  const size_t cls_off = (const char*)P.cls.records - (const char*)P.L.colpm;
+  const size_t up = prep.classed ? cls_off + prep.tables.data.size() * sizeof(double) : x_end;
   if (up > C.stage_bytes) {
     if (C.stage) HIP_TRY(hipHostFree(C.stage));
     C.stage = nullptr;
@@ -450,8 +492,11 @@ int bind_oneshot(int n, const Prepared& prep, DeviceCache& C, perm_plan& P) {
     C.stage_bytes = up;
   }
   HIP_TRY(hipStreamSynchronize(P.stream));  // idle unless an earlier call failed midway
-  std::memcpy(C.stage, cs.data(), cs.size() * sizeof(double));
+  std::memcpy(C.stage, prep.cs.data(), prep.cs.size() * sizeof(double));
   std::memcpy(C.stage + col_bytes, prep.x0.data(), prep.x0.size() * sizeof(double));
+  if (prep.classed)
+    std::memcpy(C.stage + cls_off, prep.tables.data.data(),
+                prep.tables.data.size() * sizeof(double));
   HIP_TRY(hipMemcpyAsync((void*)P.L.colpm, C.stage, up, hipMemcpyHostToDevice, P.stream));
   return PERM_OK;
 }
@@ -528,10 +573,7 @@ int run_chunked(int n, const Prepared& prep, bool use_cpu, int threads, perm_res
     const uint64_t c0 = next.fetch_add(gpu_take);
     if (c0 >= n_chunks) break;
     const uint64_t c1 = std::min(n_chunks, c0 + gpu_take);
-    perm::DenseLaunch Lc = L;
-    Lc.main.block_begin = c0 * chunk_blocks;
-    Lc.main.block_end = std::min(mb, c1 * chunk_blocks);
-    e = perm::launch_dense_pass_only(Lc, P.stream);
+    e = launch_walk(&P, c0 * chunk_blocks, std::min(mb, c1 * chunk_blocks), 0);
   }
   if (cpu.joinable()) cpu.join();
   if (e == hipSuccess) e = hipEventRecord(P.ev1, P.stream);
@@ -683,12 +725,10 @@ int perm_plan_run_blocks(perm_plan* P, int mode, unsigned long long block_begin,
   HIP_TRY(hipSetDevice(P->device));
   if (int s = ensure_records(P, block_end - block_begin)) return s;
   configure_passes(P, mode);
-  perm::DenseLaunch L = P->L;
-  L.main.block_begin = block_begin;
-  L.main.block_end = block_end;
-  L.main.record_begin = block_begin;  // the range's records from partials[0]
+  perm::DenseLaunch& L = P->L;
   HIP_TRY(hipEventRecord(P->ev0, P->stream));
-  HIP_TRY(perm::launch_dense_pass_only(L, P->stream));
+  // the range's records from partials[0]
+  HIP_TRY(launch_walk(P, block_begin, block_end, block_begin));
   HIP_TRY(hipEventRecord(P->ev1, P->stream));
   HIP_TRY(perm::launch_reduce(L.partials, block_end - block_begin, L.result, P->stream));
   perm::Partial r;
@@ -757,18 +797,15 @@ int perm_dense_noalloc(int dtype, const void* mat, int nov, int algo_id, perm_re
   P.evm = D.evm;
   P.integral = p.integral;
   set_shape(&P, nov, p);
-  const size_t need = layout_plan(&P, nov, p.cs.size());
+  const size_t need = layout_plan(&P, nov, p);
   if (need > kScratchBytes)
     return fail(PERM_ERR_SIZE, "nov=" + std::to_string(nov) + " needs " + std::to_string(need) +
                                    " bytes of device scratch; perm_dense_noalloc has " +
                                    std::to_string(kScratchBytes) + " (n <= 35)");
-  bind_plan_memory(&P, D.ptr, p.cs.size());
+  bind_plan_memory(&P, p, D.ptr);
   // pageable sources: plan_run_impl waits for the stream before returning,
   // and p outlives the call
-  HIP_TRY(hipMemcpyAsync((void*)P.L.colpm, p.cs.data(), p.cs.size() * sizeof(double),
-                         hipMemcpyHostToDevice, P.stream));
-  HIP_TRY(hipMemcpyAsync((void*)P.L.x0, p.x0.data(), p.x0.size() * sizeof(double),
-                         hipMemcpyHostToDevice, P.stream));
+  if (int st = upload_plan(&P, p)) return st;
   return plan_run_impl(&P, -1, out);
 }
 

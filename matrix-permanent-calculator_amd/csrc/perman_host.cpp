@@ -107,25 +107,25 @@ int select_device() {
 // rows [0, K_l).  Row and column permutations leave the permanent unchanged.
 // `menu`: the shapes the kernels that will run the matrix provide.
 // PERMAN_PAIR=0 keeps the natural order; PERMAN_NEST=0 only pair shapes.
-void nest_order(int n, perm::NestMenu menu, std::vector<double>& x0, std::vector<double>& cols,
+// sup[k]: rows with a nonzero in walked column k.  cp: a column order on
+// entry, whose first `pool` columns are the candidates; the order chosen
+// (the candidates taken first, the others in the order given) on return.
+// rp: the row order chosen.
+void nest_order(int n, perm::NestMenu menu, const uint64_t* sup, int pool, int* cp, int* rp,
                 int& nu, int& nu1, int& nu2) {
   nu = nu1 = nu2 = n;
+  for (int k = 0; k < n; ++k) rp[k] = k;
   if (n < perm::kMinPairN || n > perm::kMaxNestN || env_int("PERMAN_PAIR", 1) == 0) return;
   if (env_int("PERMAN_NEST", 1) == 0) menu.mask &= 1u;
   const bool nested = (menu.mask & ~1u) != 0 && n >= perm::kMinNestN;
   const int B = n - 1;
-  std::vector<uint64_t> sup(B, 0);
-  for (int k = 0; k < B; ++k)
-    for (int j = 0; j < n; ++j)
-      if (cols[(size_t)k * n + j] != 0.0) sup[k] |= 1ull << j;
-  std::vector<int> by_count(B);
-  for (int k = 0; k < B; ++k) by_count[k] = k;
+  std::vector<int> by_count(cp, cp + pool);
   std::stable_sort(by_count.begin(), by_count.end(), [&](int a, int b) {
     return __builtin_popcountll(sup[a]) < __builtin_popcountll(sup[b]);
   });
   // pair shapes only: the cost grows with column 0's support, so the
   // sparsest column (first in by_count) is the choice
-  const int n0 = std::min(B, nested ? 8 : 1), n12 = nested ? std::min(B, 12) : 0;
+  const int n0 = std::min(pool, nested ? 8 : 1), n12 = nested ? std::min(pool, 12) : 0;
   int best_cost = perm::nest_cost(n, {n, n, n});
   perm::NestShape best{n, n, n};
   int bc[3] = {-1, -1, -1};
@@ -189,29 +189,24 @@ void nest_order(int n, perm::NestMenu menu, std::vector<double>& x0, std::vector
   }
   if (bc[0] < 0) return;
   // rows: column 0's, then column 1's new ones, then column 2's, then the rest
-  std::vector<int> rp, cp;
+  int nr = 0;
   uint64_t taken = 0;
   for (int l = 0; l < 3; ++l) {
     if (bc[l] < 0) continue;
     for (int j = 0; j < n; ++j)
       if (((sup[bc[l]] >> j) & 1) && !((taken >> j) & 1)) {
-        rp.push_back(j);
+        rp[nr++] = j;
         taken |= 1ull << j;
       }
   }
   for (int j = 0; j < n; ++j)
-    if (!((taken >> j) & 1)) rp.push_back(j);
+    if (!((taken >> j) & 1)) rp[nr++] = j;
+  int nc = 0, old[64];
+  std::copy(cp, cp + B, old);
   for (int l = 0; l < 3; ++l)
-    if (bc[l] >= 0) cp.push_back(bc[l]);
+    if (bc[l] >= 0) cp[nc++] = bc[l];
   for (int k = 0; k < B; ++k)
-    if (k != bc[0] && k != bc[1] && k != bc[2]) cp.push_back(k);
-  std::vector<double> x2(x0.size()), c2(cols.size());
-  for (int j = 0; j < n; ++j) x2[j] = x0[rp[j]];
-  for (int j = 0; j + n < (int)x0.size(); ++j) x2[n + j] = x0[n + rp[j]];  // low parts
-  for (int k = 0; k < B; ++k)
-    for (int j = 0; j < n; ++j) c2[(size_t)k * n + j] = cols[(size_t)cp[k] * n + rp[j]];
-  x0.swap(x2);
-  cols.swap(c2);
+    if (old[k] != bc[0] && old[k] != bc[1] && old[k] != bc[2]) cp[nc++] = old[k];
   nu = best.k0;
   nu1 = best.k1;
   nu2 = best.k2;
@@ -394,10 +389,57 @@ bool integral_matrix(const std::vector<double>& a) {
   return true;
 }
 
+// Groups per lane: a workgroup's table of the lane columns (built from the
+// block columns at its start) is used by 2^t groups of 32 subsets.  Few
+// groups while the whole walk is a few microseconds, so that it spreads over
+// the chip; 2^5 to 2^8 beyond.  Measured at density 0.5 (ms, t): n = 24 0.025
+// (1) 0.0148 (3) 0.0185 (4); n = 28 0.138 (3) 0.108 (5) 0.121 (7); n = 32 1.83
+// (4) 1.58 (7) 1.57 (8); n = 40 343 (7) 336 (8) 334 (9).  A workgroup's
+// subsets, 2^(11 + t), are those of 256 lanes of 2^(t + 3) steps of the Gray
+// kernels.
+int class_walk_bits(int n) {
+  if (n >= 37) return std::max(8, n - 34);  // at most 2^22 workgroups
+  return std::min(7, std::max(1, n / 2 - 9));
+}
+
+// The class walk takes the FP64 pass of the single-matrix paths unless a
+// walk order or split is asked for.
+static bool class_order(int n, const NestMenu& menu) {
+  return n >= kMinClassN && n <= kMaxClassN && menu.mask == kMenuSingle.mask &&
+         env_int("PERMAN_PAIR", 1) != 0 && env_int("PERMAN_NEST", 1) != 0 &&
+         env_int("PERMAN_WALK_BITS", 0) == 0;
+}
+
 void finish_prepare(int n, const NestMenu& menu, std::vector<double>& cols, Prepared& p) {
-  nest_order(n, menu, p.x0, cols, p.nu, p.nu1, p.nu2);
+  uint64_t sup[64];
+  for (int k = 0; k < n - 1; ++k) {
+    sup[k] = 0;
+    for (int j = 0; j < n; ++j)
+      if (cols[(size_t)k * n + j] != 0.0) sup[k] |= 1ull << j;
+  }
   if (p.integral) p.product_bits = perm::integer_product_bits(p.x0.data(), cols.data(), n);
-  perm::build_column_store(n, [&](int k, int j) { return cols[(size_t)k * n + j]; }, p.cs);
+  int cp[64], rp[64];
+  p.classed = class_order(n, menu);
+  if (p.classed) {
+    plan_classes(n, sup, p.plan);
+    p.classed = p.plan.cost < kClassGain * (1 << kClassBits) * (2 * n + 2);
+  }
+  if (p.classed) {
+    build_class_tables(p.plan, p.x0.data(), cols.data(), class_walk_bits(n), p.tables);
+    std::copy(p.plan.cols, p.plan.cols + n - 1, cp);
+  } else {
+    for (int k = 0; k < n - 1; ++k) cp[k] = k;
+  }
+  // the Gray walk takes its first columns among the class columns, so that
+  // its workgroups cover the class walk's subsets
+  nest_order(n, menu, sup, p.classed ? kClassBits : n - 1, cp, rp, p.nu, p.nu1, p.nu2);
+  std::vector<double> x0(2 * (size_t)n);
+  for (int j = 0; j < n; ++j) {
+    x0[j] = p.x0[rp[j]];
+    x0[n + j] = p.x0[n + rp[j]];  // low parts
+  }
+  p.x0.swap(x0);
+  perm::build_column_store(n, [&](int k, int j) { return cols[(size_t)cp[k] * n + rp[j]]; }, p.cs);
 }
 
 int prepare_dense(int dtype, const void* mat, int n, Prepared& p, const NestMenu& menu) {

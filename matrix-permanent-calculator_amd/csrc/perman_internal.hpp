@@ -6,6 +6,7 @@
 #include <string>
 #include <vector>
 
+#include "class_plan.hpp"
 #include "nest_shape.hpp"
 
 struct perm_result;
@@ -35,6 +36,12 @@ struct Prepared {
   int nu = 0, nu1 = 0, nu2 = 0;
   bool integral = false;
   double product_bits = 1e9;  // integer_product_bits (integer matrices)
+  // Class walk (single-matrix FP64 pass, orders kMinClassN..kMaxClassN): its
+  // plan and tables.  The store above then has the class columns first, so
+  // the Gray kernels' workgroups cover the same subsets as the class walk's.
+  bool classed = false;
+  ClassPlan plan;
+  ClassTables tables;
   // no perfect matching in the matrix's nonzero pattern: every term of the
   // permanent vanishes, the result is exactly 0 and no walk is run
   bool zero = false;
@@ -50,8 +57,11 @@ bool has_perfect_matching(int n, const uint64_t* rowsup);
 bool sparse_pattern_zero(int dtype, const void* mat, const std::vector<double>& cols, int n);
 // The result of a permanent whose pattern has no perfect matching: exactly 0.
 void fill_zero_result(int n, bool integral, perm_result& out);
+// log2 of the class walk's groups per lane for order n.
+int class_walk_bits(int n);
 // menu: the walk shapes the kernels that will run the matrix are compiled
 // for (kMenuSingle: single-matrix paths; kMenuBatch: batch and server).
+// With kMenuSingle, orders of the class walk are prepared for it.
 int prepare_dense(int dtype, const void* mat, int n, Prepared& p,
                   const NestMenu& menu = kMenuSingle);
 int prepare_sparse(int dtype, const void* mat, const int* cptrs, const int* rows,

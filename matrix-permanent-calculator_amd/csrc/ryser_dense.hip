@@ -5,20 +5,20 @@
 
 namespace perm {
 
-hipError_t launch_dense_range_a(const DenseLaunch& L, hipStream_t s, hipEvent_t ev);
-hipError_t launch_dense_range_b(const DenseLaunch& L, hipStream_t s, hipEvent_t ev);
-hipError_t launch_dense_range_c(const DenseLaunch& L, hipStream_t s, hipEvent_t ev);
-hipError_t launch_dense_range_d(const DenseLaunch& L, hipStream_t s, hipEvent_t ev);
-hipError_t launch_dense_range_e(const DenseLaunch& L, hipStream_t s, hipEvent_t ev);
-hipError_t launch_dense_range_f(const DenseLaunch& L, hipStream_t s, hipEvent_t ev);
-hipError_t launch_dense_range_g(const DenseLaunch& L, hipStream_t s, hipEvent_t ev);
-hipError_t launch_dense_range_h(const DenseLaunch& L, hipStream_t s, hipEvent_t ev);
-hipError_t launch_dense_range_i(const DenseLaunch& L, hipStream_t s, hipEvent_t ev);
-hipError_t launch_dense_range_j(const DenseLaunch& L, hipStream_t s, hipEvent_t ev);
-hipError_t launch_dense_range_k(const DenseLaunch& L, hipStream_t s, hipEvent_t ev);
-hipError_t launch_dense_range_l(const DenseLaunch& L, hipStream_t s, hipEvent_t ev);
-hipError_t launch_dense_range_m(const DenseLaunch& L, hipStream_t s, hipEvent_t ev);
-hipError_t launch_dense_range_o(const DenseLaunch& L, hipStream_t s, hipEvent_t ev);
+hipError_t launch_dense_range_a(const DenseLaunch& L, hipStream_t s);
+hipError_t launch_dense_range_b(const DenseLaunch& L, hipStream_t s);
+hipError_t launch_dense_range_c(const DenseLaunch& L, hipStream_t s);
+hipError_t launch_dense_range_d(const DenseLaunch& L, hipStream_t s);
+hipError_t launch_dense_range_e(const DenseLaunch& L, hipStream_t s);
+hipError_t launch_dense_range_f(const DenseLaunch& L, hipStream_t s);
+hipError_t launch_dense_range_g(const DenseLaunch& L, hipStream_t s);
+hipError_t launch_dense_range_h(const DenseLaunch& L, hipStream_t s);
+hipError_t launch_dense_range_i(const DenseLaunch& L, hipStream_t s);
+hipError_t launch_dense_range_j(const DenseLaunch& L, hipStream_t s);
+hipError_t launch_dense_range_k(const DenseLaunch& L, hipStream_t s);
+hipError_t launch_dense_range_l(const DenseLaunch& L, hipStream_t s);
+hipError_t launch_dense_range_m(const DenseLaunch& L, hipStream_t s);
+hipError_t launch_dense_range_o(const DenseLaunch& L, hipStream_t s);
 
 // Grid-level reduction of `count` partials into out[0] (one workgroup of
 // 256 threads, fixed order).
@@ -91,9 +91,9 @@ hipError_t launch_skip(const SkipLaunch& L, hipStream_t stream) {
   return hipGetLastError();
 }
 
-static hipError_t launch_passes(const DenseLaunch& L, hipStream_t stream, hipEvent_t main_done) {
+hipError_t launch_dense_pass_only(const DenseLaunch& L, hipStream_t stream) {
   if (L.n < 1 || L.n > kMaxDenseN) return hipErrorInvalidValue;
-  using RangeFn = hipError_t (*)(const DenseLaunch&, hipStream_t, hipEvent_t);
+  using RangeFn = hipError_t (*)(const DenseLaunch&, hipStream_t);
   static const struct {
     int hi;
     RangeFn fn;
@@ -105,23 +105,12 @@ static hipError_t launch_passes(const DenseLaunch& L, hipStream_t stream, hipEve
                  {48, launch_dense_range_k}, {53, launch_dense_range_l},
                  {58, launch_dense_range_m}, {63, launch_dense_range_o}};
   for (const auto& r : kRanges)
-    if (L.n <= r.hi) return r.fn(L, stream, main_done);
+    if (L.n <= r.hi) return r.fn(L, stream);
   return hipErrorInvalidValue;
-}
-
-hipError_t launch_dense_pass_only(const DenseLaunch& L, hipStream_t stream) {
-  return launch_passes(L, stream, nullptr);
 }
 
 hipError_t launch_reduce(const Partial* in, uint64_t count, Partial* out, hipStream_t stream) {
   reduce_partials_kernel<<<1, 256, 0, stream>>>(in, count, out);
-  return hipGetLastError();
-}
-
-hipError_t launch_dense(const DenseLaunch& L, hipStream_t stream, hipEvent_t main_done) {
-  hipError_t e = launch_passes(L, stream, main_done);
-  if (e != hipSuccess || L.total_blocks <= 1) return e;  // one record: it is the sum
-  reduce_partials_kernel<<<1, 256, 0, stream>>>(L.partials, L.total_blocks, L.result);
   return hipGetLastError();
 }
 

@@ -485,15 +485,13 @@ hipError_t launch_pass(const DenseLaunch& L, const LanePass& P, hipStream_t stre
 
 // One run: the kernel of mode MODE and shape S.
 template <int N, int MODE, class S>
-hipError_t launch_mode(const DenseLaunch& L, hipStream_t stream, hipEvent_t main_done) {
-  hipError_t e = launch_pass<N, MODE, S>(L, L.main, stream);
-  if (e == hipSuccess && main_done) e = hipEventRecord(main_done, stream);
-  return e;
+hipError_t launch_mode(const DenseLaunch& L, hipStream_t stream) {
+  return launch_pass<N, MODE, S>(L, L.main, stream);
 }
 
 // Shape j of K0 = 4(q+1) in the compiled menu (nest_menu_shape).
 template <int N, int MODE, int Q, int J>
-hipError_t launch_shape(const DenseLaunch& L, hipStream_t stream, hipEvent_t main_done,
+hipError_t launch_shape(const DenseLaunch& L, hipStream_t stream,
                         bool& hit) {
   constexpr int K0 = 4 * (Q + 1);
   constexpr NestShape sh = nest_menu_shape(N, K0, J);
@@ -502,25 +500,25 @@ hipError_t launch_shape(const DenseLaunch& L, hipStream_t stream, hipEvent_t mai
   } else {
     if (L.nu != sh.k0 || L.nu1 != sh.k1 || L.nu2 != sh.k2) return hipErrorInvalidValue;
     hit = true;
-    return launch_mode<N, MODE, Nest<sh.k0, sh.k1, sh.k2>>(L, stream, main_done);
+    return launch_mode<N, MODE, Nest<sh.k0, sh.k1, sh.k2>>(L, stream);
   }
 }
 
 template <int N, int MODE, int Q, int... J>
-hipError_t launch_k0(const DenseLaunch& L, hipStream_t stream, hipEvent_t main_done, bool& hit,
+hipError_t launch_k0(const DenseLaunch& L, hipStream_t stream, bool& hit,
                      std::integer_sequence<int, J...>) {
   hipError_t e = hipErrorInvalidValue;
-  ((hit ? 0 : (e = launch_shape<N, MODE, Q, J>(L, stream, main_done, hit), 0)), ...);
+  ((hit ? 0 : (e = launch_shape<N, MODE, Q, J>(L, stream, hit), 0)), ...);
   return e;
 }
 
 template <int N, int MODE, int... Q>
-hipError_t launch_nested(const DenseLaunch& L, hipStream_t stream, hipEvent_t main_done,
+hipError_t launch_nested(const DenseLaunch& L, hipStream_t stream,
                          std::integer_sequence<int, Q...>) {
   hipError_t e = hipErrorInvalidValue;
   bool hit = false;
   ((L.nu == 4 * (Q + 1) && !hit
-        ? (e = launch_k0<N, MODE, Q>(L, stream, main_done, hit,
+        ? (e = launch_k0<N, MODE, Q>(L, stream, hit,
                                      std::make_integer_sequence<int, kNestShapesPerK0>{}),
            0)
         : 0),
@@ -529,11 +527,11 @@ hipError_t launch_nested(const DenseLaunch& L, hipStream_t stream, hipEvent_t ma
 }
 
 template <int N, int MODE>
-hipError_t launch_shaped(const DenseLaunch& L, hipStream_t stream, hipEvent_t main_done) {
-  if (L.nu == N || L.nu <= 0) return launch_mode<N, MODE, Nest<N, N, N>>(L, stream, main_done);
+hipError_t launch_shaped(const DenseLaunch& L, hipStream_t stream) {
+  if (L.nu == N || L.nu <= 0) return launch_mode<N, MODE, Nest<N, N, N>>(L, stream);
   if constexpr (N >= kMinPairN && N <= kMaxNestN) {
     if (L.nu % 4 == 0 && L.nu < N)
-      return launch_nested<N, MODE>(L, stream, main_done,
+      return launch_nested<N, MODE>(L, stream,
                                     std::make_integer_sequence<int, (N - 1) / 4>{});
   }
   return hipErrorInvalidValue;
@@ -542,10 +540,10 @@ hipError_t launch_shaped(const DenseLaunch& L, hipStream_t stream, hipEvent_t ma
 // kFast and kDDProd run the walk shape in L (nu, nu1, nu2); kDDAll the plain
 // walk.
 template <int N>
-hipError_t launch_n(const DenseLaunch& L, hipStream_t stream, hipEvent_t main_done) {
-  if (L.mode == kDDAll) return launch_mode<N, kDDAll, Nest<N, N, N>>(L, stream, main_done);
-  if (L.mode == kDDProd) return launch_shaped<N, kDDProd>(L, stream, main_done);
-  if (L.mode == kFast) return launch_shaped<N, kFast>(L, stream, main_done);
+hipError_t launch_n(const DenseLaunch& L, hipStream_t stream) {
+  if (L.mode == kDDAll) return launch_mode<N, kDDAll, Nest<N, N, N>>(L, stream);
+  if (L.mode == kDDProd) return launch_shaped<N, kDDProd>(L, stream);
+  if (L.mode == kFast) return launch_shaped<N, kFast>(L, stream);
   return hipErrorInvalidValue;
 }
 
@@ -556,13 +554,13 @@ hipError_t launch_n(const DenseLaunch& L, hipStream_t stream, hipEvent_t main_do
 #define PERM_DENSE_RANGE(TAG, LO, HI)                                                         \
   namespace perm {                                                                            \
   template <int... I>                                                                         \
-  static hipError_t dispatch_##TAG(const DenseLaunch& L, hipStream_t s, hipEvent_t ev,        \
+  static hipError_t dispatch_##TAG(const DenseLaunch& L, hipStream_t s,                       \
                                    std::integer_sequence<int, I...>) {                        \
     hipError_t e = hipErrorInvalidValue;                                                      \
-    ((L.n == LO + I ? (e = launch_n<LO + I>(L, s, ev), 0) : 0), ...);                         \
+    ((L.n == LO + I ? (e = launch_n<LO + I>(L, s), 0) : 0), ...);                         \
     return e;                                                                                 \
   }                                                                                           \
-  hipError_t launch_dense_range_##TAG(const DenseLaunch& L, hipStream_t s, hipEvent_t ev) {   \
-    return dispatch_##TAG(L, s, ev, std::make_integer_sequence<int, HI - LO + 1>{});          \
+  hipError_t launch_dense_range_##TAG(const DenseLaunch& L, hipStream_t s) {                  \
+    return dispatch_##TAG(L, s, std::make_integer_sequence<int, HI - LO + 1>{});          \
   }                                                                                           \
   }

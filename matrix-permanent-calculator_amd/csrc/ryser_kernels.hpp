@@ -66,16 +66,10 @@ constexpr int kMinSkipN = 16;
 // Enqueue the skipping kernel and the grid reduction on `stream`.
 hipError_t launch_skip(const SkipLaunch& L, hipStream_t stream);
 
-// Enqueue the passes of the dense kernel and the grid reduction of all
-// partials on `stream` (with a single workgroup record, no reduction: the
-// sum is partials[0]).
-// `main_done`, if not null, is recorded on `stream` after the main pass.
-hipError_t launch_dense(const DenseLaunch& L, hipStream_t stream, hipEvent_t main_done = nullptr);
 // Only the walk of L (its block range), no reduction (the caller sums the
 // partial records).
 hipError_t launch_dense_pass_only(const DenseLaunch& L, hipStream_t stream);
-// The grid reduction alone: the DD sum of in[0, count) into *out (the same
-// order as launch_dense's).
+// The grid reduction: the DD sum of in[0, count) into *out, in a fixed order.
 hipError_t launch_reduce(const Partial* in, uint64_t count, Partial* out, hipStream_t stream);
 // z[i] = rec[i].sq_sum + run_weight * rec[i].sq_run for i < units: the
 // modelled variance weights of a walk's workgroup records.

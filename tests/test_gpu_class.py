@@ -1,0 +1,89 @@
+"""The class walk (FP64 pass of the single-matrix paths, n = 24..48): its
+column classes, records and splits at the orders where they change, against
+exact values and the double-double oracle, and against the double-double X
+mode over the same workgroups where no oracle finishes."""
+import numpy as np
+import pytest
+
+import oracle as O
+import permanent_amd as P
+from conftest import assert_target
+
+pytestmark = pytest.mark.gpu
+
+
+def patterns(n):
+    """0/1 matrices whose rows fall into few, many, or one-sided classes:
+    name -> (matrix, its permanent)."""
+    eye = np.eye(n, dtype=np.int32)
+    band = eye + np.roll(eye, 1, axis=1)          # circulant, two ones per row: 2
+    tri = np.triu(np.ones((n, n), dtype=np.int32))
+    hat = eye.copy()                               # a full first row and column
+    hat[0, :] = hat[:, 0] = 1                      # 1 + (n - 1)
+    pairs = np.kron(np.eye(n // 2, dtype=np.int32), np.ones((2, 2), dtype=np.int32))
+    return {"identity": (eye, 1), "circulant": (band, 2), "triangular": (tri, 1),
+            "arrow": (hat, n), "pairs": (pairs, 2 ** (n // 2))}
+
+
+@pytest.mark.parametrize("name", ["identity", "circulant", "triangular", "arrow", "pairs"])
+@pytest.mark.parametrize("n", [24, 30])
+def test_structured_patterns_exact(n, name):
+    a, want = patterns(n)[name]
+    g = np.random.default_rng(n)
+    for m in (a, a[g.permutation(n)][:, g.permutation(n)], 3 * a):
+        m = np.ascontiguousarray(m, dtype=np.int32)
+        scale = 3 ** n if m.max() == 3 else 1
+        r = P.dense(m)
+        # within the stated error; exact where that is below one half (the
+        # sum of |terms| of 3 a, n = 30, is 4e26 times its permanent: there
+        # no double-double product sum is)
+        assert abs(r.value - float(want * scale)) <= r.stated, (n, name, r)
+        if r.stated < 0.5:
+            assert r.value == want * scale, (n, name, r)
+        assert r.stated < 0.5 or scale > 1, (n, name, r)
+
+
+@pytest.mark.parametrize("n,density,signed", [(24, 0.15, False), (24, 0.6, True), (25, 0.35, False),
+                                              (25, 0.8, False), (26, 0.5, False),
+                                              (26, 0.25, True)])
+def test_against_exact_and_natural_order(monkeypatch, n, density, signed):
+    a = P.synthetic_matrix(n, density, 90 + n, full_support=True)
+    if signed:
+        a = a * np.where(P.uniforms(7, n * n).reshape(n, n) < 0.5, -1.0, 1.0)
+    hi, lo = O.ryser_dd(a)
+    ex = hi + lo
+    r = P.dense(a)
+    assert_target(r, ex, ctx=(n, density, signed))
+    with monkeypatch.context() as m:
+        m.setenv("PERMAN_PAIR", "0")
+        plain = P.dense(a)
+    assert abs(r.value - plain.value) <= r.stated + plain.stated
+    # the sum of |terms| does not depend on the walk: n roundings of a term, at
+    # most 2^10 of a lane's sum
+    assert abs(r.abs_sum - plain.abs_sum) <= (n + 1024) * 2.0 ** -52 * plain.abs_sum
+    if not signed:
+        s = P.sparse(a)
+        assert (s.value, s.abs_sum) == (r.value, r.abs_sum)
+
+
+@pytest.mark.parametrize("n,density", [(27, 0.1), (28, 0.7), (31, 0.3), (32, 0.5), (36, 0.2),
+                                       (37, 0.6), (42, 0.45), (43, 0.2), (48, 0.5)])
+def test_workgroups_cover_the_same_subsets_in_every_mode(n, density):
+    """One workgroup of the class walk against the double-double X mode over
+    the same subsets (the first, one in the middle, the last)."""
+    plan = P.Plan(P.synthetic_matrix(n, density, 300 + n, full_support=True))
+    try:
+        w, h, blocks = plan.geometry()
+        assert blocks == 1 << (n - 1 - w - 8)
+        for b in (0, blocks // 3, blocks - 1):
+            fp = plan.run_blocks(b, b + 1, mode=0)
+            dd = plan.run_blocks(b, b + 1, mode=2)
+            diff = abs((fp.sum_hi - dd.sum_hi) + (fp.sum_lo - dd.sum_lo))
+            # n + 9 roundings of a term (product and row sums) and at most 256
+            # of a run's sum
+            assert diff <= min(fp.err_est / 2.0, (n + 9 + 256) * 2.0 ** -53 * fp.abs_sum / 2.0), \
+                (n, b, fp, dd)
+            # a lane's sum of |terms| is not folded: a rounding per subset
+            assert abs(fp.abs_sum - dd.abs_sum) <= (n + 9 + 2.0 ** w) * 2.0 ** -52 * dd.abs_sum
+    finally:
+        plan.close()
