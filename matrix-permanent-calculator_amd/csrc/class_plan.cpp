@@ -228,12 +228,11 @@ void plan_classes(int n, const uint64_t* sup, ClassPlan& p) {
 void build_class_tables(const ClassPlan& p, const double* x0, const double* cols, int walk_bits,
                         ClassTables& out) {
   const int n = p.n, B = n - 1;
-  const int block_bits = B - kClassBits - walk_bits - kClassLaneBits;
   auto entry = [&](int r, int i) { return cols[(size_t)p.cols[i] * n + p.rows[r]]; };
   std::vector<double>& d = out.data;
   d.clear();
+  d.reserve(class_tables_bound(n) + (walk_bits < 0 ? 0 : class_split_doubles(n, walk_bits)));
   // records: 7 offsets and the control word, then 8 offsets each
-  const int walk0 = kClassBits, lane0 = walk0 + walk_bits, block0 = lane0 + kClassLaneBits;
   auto add_row = [&](int r, double* o) {  // the 2^m - 1 offsets of row r
     const int t = p.classes[r];
     double hi[kClasses] = {0.0}, lo[kClasses] = {0.0};
@@ -269,15 +268,19 @@ void build_class_tables(const ClassPlan& p, const double* x0, const double* cols
     }
   }
   d.resize(d.size() + 8, 0.0);  // read ahead by one record
+  out.cols = d.size();
+  for (int b = kClassBits; b < B; ++b)
+    for (int r = 0; r < n; ++r) d.push_back(entry(r, b));
+  for (int part = 0; part < 2; ++part)
+    for (int r = 0; r < n; ++r) d.push_back(x0[part * n + p.rows[r]]);
+  if (walk_bits < 0) return;
+  const int walk0 = kClassBits, lane0 = walk0 + walk_bits;
   out.lane = d.size();
   for (int r = 0; r < n; ++r) {
     for (int b = 0; b < kClassLaneBits; ++b) d.push_back(entry(r, lane0 + b));
     d.push_back(x0[p.rows[r]]);
     d.push_back(x0[n + p.rows[r]]);
   }
-  out.block = d.size();
-  for (int b = 0; b < block_bits; ++b)
-    for (int r = 0; r < n; ++r) d.push_back(entry(r, block0 + b));
   // offsets of the walk columns' subsets, each the rounded double-double sum
   out.walk = d.size();
   const size_t subsets = (size_t)1 << walk_bits;

@@ -31,17 +31,27 @@ struct ClassPlan {
 // kClassBits.
 void plan_classes(int n, const uint64_t* sup, ClassPlan& p);
 
-// What the kernel reads, as one array: the rows' records at 0, the lane
-// columns with the start vector, the block columns and the walk offsets.
+// What the kernel reads, as one array: the rows' records at 0; the columns
+// after the class columns and the start vector (x0, then its low parts), n
+// doubles each, rows in the plan's order; and, for a given split, the lane
+// columns by row and the walk offsets (ClassMatrix in ryser_class.hpp).
 struct ClassTables {
   std::vector<double> data;
-  size_t lane = 0, block = 0, walk = 0;  // where the parts begin
+  size_t cols = 0, lane = 0, walk = 0;  // where the parts begin
 };
 
 // x0: 2n doubles (start vector, its low parts); cols[k * n + j] = a[j][k] of
-// the walked columns.  2^walk_bits groups of 2^kClassBits subsets per lane;
-// n - 1 >= kClassBits + walk_bits + kClassLaneBits.
+// the walked columns.  walk_bits >= 0: the last two parts for 2^walk_bits
+// groups of 2^kClassBits subsets per lane (n - 1 >= kClassBits + walk_bits +
+// kClassLaneBits); < 0: without them (the device expands them).
 void build_class_tables(const ClassPlan& p, const double* x0, const double* cols, int walk_bits,
                         ClassTables& out);
+// Doubles of the last two parts, and a bound of the first ones'.
+inline size_t class_split_doubles(int n, int walk_bits) {
+  return 8 * (size_t)n + ((size_t)n << walk_bits) + 2;
+}
+inline size_t class_tables_bound(int n) {
+  return 32 * (size_t)n + 8 + (size_t)(n + 1) * n;
+}
 
 }  // namespace perm

@@ -28,6 +28,9 @@ constexpr int kMinNestN = 24;
 // 308 us.  Above kMaxNestN no walk of every subset finishes.
 constexpr int kMinClassN = 24;
 constexpr int kMaxClassN = kMaxNestN;
+// In a batch a matrix pays no launch of its own: from the smallest order with
+// class and lane columns on.
+constexpr int kMinBatchClassN = 12;
 constexpr double kClassGain = 0.75;
 
 // Walk shape: Gray column l < 3 touches rows [0, k_l) only (k0 <= k1 <= k2).
@@ -58,9 +61,12 @@ constexpr NestShape nest_menu_shape(int n, int k0, int j) {
 struct NestMenu {
   int max_k0;
   unsigned mask;
+  int min_class_n;  // the class walk's smallest order for these kernels (0: none)
 };
-constexpr NestMenu kMenuSingle = {kMaxDenseN, 0x1fu};  // single-matrix kernels: all
-constexpr NestMenu kMenuBatch = {kMaxDenseN, 0x19u};  // batch kernels: shapes j = 0, 3, 4
+constexpr NestMenu kMenuSingle = {kMaxDenseN, 0x1fu, kMinClassN};  // single matrices: all
+// batch and served kernels: shapes j = 0, 3, 4
+constexpr NestMenu kMenuBatch = {kMaxDenseN, 0x19u, kMinBatchClassN};
+constexpr NestMenu kMenuServe = {kMaxDenseN, 0x19u, 0};
 constexpr bool nest_menu_has(const NestMenu& m, int n, int k0, int j) {
   return k0 <= m.max_k0 && ((m.mask >> j) & 1u) && nest_menu_shape(n, k0, j).k0 != 0;
 }

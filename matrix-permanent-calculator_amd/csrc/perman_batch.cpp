@@ -8,7 +8,9 @@
 // what else is in the batch.  Items are grouped by kernel variant (n and
 // walk shape);
 // one persistent kernel per variant drains its group, the groups running
-// concurrently on several streams.  The whole launch sequence (counter reset,
+// concurrently on several streams.  The FP64 pass of all matrices of the
+// class walk is one group whatever their orders (ryser_class.hip; an item is
+// a workgroup there, over the same subsets).  The whole launch sequence (counter reset,
 // variant kernels, per-matrix reduction, result copy) is captured once in a
 // hipGraph at the second run and replayed from then on (the first run after a
 // build launches directly: a batch computed once pays no capture).
@@ -27,6 +29,7 @@
 #include "../../include/perman_hip.h"
 #include "perman_internal.hpp"
 #include "ryser_batch.hpp"
+#include "ryser_class.hpp"
 #include "ryser_host.hpp"
 #include "ryser_kernels.hpp"
 
@@ -37,6 +40,7 @@ using perm::BatchMatrix;
 using perm::Partial;
 
 constexpr int kMaxStreams = 8;
+constexpr int kClassGroup = -2;
 
 struct Entry {
   int n = 0, variant = -1, walk_bits = 0, high_bits = 0;
@@ -45,6 +49,12 @@ struct Entry {
   bool zero = false;  // no perfect matching: exactly 0, no items
   double product_bits = 1e9;
   size_t col_off = 0, x0_off = 0;  // offsets (doubles) into the data buffer
+  // class walk of the FP64 pass: where its records and columns are in the
+  // data buffer, its lane columns and walk offsets in the expanded tables
+  bool classed = false;
+  uint32_t live = 0;
+  size_t rec_off = 0, ccol_off = 0, split_off = 0;
+  int cost = 0;  // FP64 instructions per 32 subsets
   uint32_t first_item = 0, item_count = 0;
 };
 
@@ -55,19 +65,23 @@ struct perm_batch {
   int item_log2 = 17;   // subsets per item (64 lanes x 2^(item_log2-6) steps)
   int streams = 8;
   int max_grid = 1024;  // workgroups per variant kernel
+  uint32_t max_grid_u() const { return (uint32_t)max_grid; }
   std::vector<double> data;
   std::vector<Entry> ents;
   std::vector<BatchItem> items;
   struct Group {
-    int vid;
+    int vid;      // batch variant, or kClassGroup
     uint32_t begin, end;
     double work;
+    int max_n;  // kClassGroup: largest order
   };
   std::vector<Group> groups;
   // device
   void* dmem = nullptr;
   size_t dbytes = 0;
   double* d_data = nullptr;
+  double* d_split = nullptr;  // lane columns and walk offsets of the class walk
+  perm::ClassMatrix* d_cls = nullptr;
   BatchMatrix* d_mats = nullptr;
   BatchItem* d_items = nullptr;
   Partial* d_partials = nullptr;
@@ -125,6 +139,15 @@ int fill_entry(perm_batch* B, Entry& e, int n, perm::Prepared& p) {
   B->data.insert(B->data.end(), p.cs.begin(), p.cs.end());
   e.x0_off = B->data.size();
   B->data.insert(B->data.end(), p.x0.begin(), p.x0.end());
+  e.classed = p.classed;
+  if (p.classed) {
+    e.live = p.plan.live;
+    e.cost = p.plan.cost;
+    while (B->data.size() % 8) B->data.push_back(0.0);  // records are 64 bytes
+    e.rec_off = B->data.size();
+    e.ccol_off = e.rec_off + p.tables.cols;
+    B->data.insert(B->data.end(), p.tables.data.begin(), p.tables.data.end());
+  }
   while (B->data.size() % 32) B->data.push_back(0.0);  // 256-B alignment of the next store
   return PERM_OK;
 }
@@ -150,6 +173,19 @@ int add_prepared(perm_batch* B, int n, perm::Prepared& p, int* index) {
 
 size_t align256(size_t v) { return (v + 255) / 256 * 256; }
 
+// The group's kernel on `stream`.
+hipError_t launch_group(perm_batch* B, size_t gi, hipStream_t stream) {
+  const perm_batch::Group& G = B->groups[gi];
+  const uint32_t items = G.end - G.begin;
+  if (G.vid == kClassGroup)
+    return perm::launch_class_batch(B->d_cls, B->d_items, G.begin, G.end, B->d_counters + gi,
+                                    B->d_partials, G.max_n, std::min(items, B->max_grid_u()),
+                                    stream);
+  const uint32_t grid = std::max(1u, std::min<uint32_t>((items + 3) / 4, B->max_grid_u()));
+  return perm::launch_batch_variant(G.vid, B->d_mats, B->d_items, G.begin, G.end,
+                                    B->d_counters + gi, B->d_partials, grid, stream);
+}
+
 // Enqueue one run of the batch on its streams: reset -> fork -> variant
 // kernels over streams -> join -> reduce -> result copy.  Groups come in
 // decreasing work; each goes to the stream with the least work so far
@@ -165,13 +201,10 @@ int enqueue_run(perm_batch* B) {
   for (int i = 1; i < ns; ++i) HIP_TRYB(hipStreamWaitEvent(B->s[i], B->ev_fork, 0));
   for (size_t gi = 0; gi < B->groups.size(); ++gi) {
     const auto& G = B->groups[gi];
-    const uint32_t waves = G.end - G.begin;
-    const uint32_t grid = std::max(1u, std::min<uint32_t>((waves + 3) / 4, B->max_grid));
     const int si = (int)(std::min_element(stream_work.begin(), stream_work.end()) -
                          stream_work.begin());
     stream_work[si] += G.work;
-    HIP_TRYB(perm::launch_batch_variant(G.vid, B->d_mats, B->d_items, G.begin, G.end,
-                                        B->d_counters + gi, B->d_partials, grid, B->s[si]));
+    HIP_TRYB(launch_group(B, gi, B->s[si]));
   }
   for (int i = 1; i < ns; ++i) {
     HIP_TRYB(hipEventRecord(B->ev_join[i], B->s[i]));
@@ -203,9 +236,17 @@ int capture(perm_batch* B) {
   return PERM_OK;
 }
 
-// Plan items and upload.
-// Append the items of entries `idx` to B->items, grouped by variant, the
-// groups in decreasing work, each group a contiguous item range.
+// The class walk takes an entry's FP64 pass when its items have a group of
+// class subsets per lane, and at most 2^10 of them (the table of walk offsets
+// is as long).
+bool class_split_ok(int walk_bits) {
+  return walk_bits >= perm::kClassBits && walk_bits <= perm::kClassBits + 10;
+}
+bool runs_classed(const Entry& e) { return e.classed && class_split_ok(e.walk_bits); }
+
+// Append the items of entries `idx` to B->items, grouped by variant (the
+// class walk's entries as one group, decreasing n), the groups in decreasing
+// work, each group a contiguous item range.
 void plan_items(perm_batch* B, const std::vector<uint32_t>& idx) {
   std::vector<std::vector<uint32_t>> by_var;
   std::vector<int> var_ids;
@@ -215,9 +256,10 @@ void plan_items(perm_batch* B, const std::vector<uint32_t>& idx) {
     e.first_item = 0;
     e.item_count = 0;
     if (e.zero) continue;  // no walk: its result is exactly 0
-    auto it = std::find(var_ids.begin(), var_ids.end(), e.variant);
+    const int vid = runs_classed(e) ? kClassGroup : e.variant;
+    auto it = std::find(var_ids.begin(), var_ids.end(), vid);
     if (it == var_ids.end()) {
-      var_ids.push_back(e.variant);
+      var_ids.push_back(vid);
       by_var.emplace_back();
       it = var_ids.end() - 1;
     }
@@ -229,18 +271,27 @@ void plan_items(perm_batch* B, const std::vector<uint32_t>& idx) {
     order[v] = v;
     for (uint32_t m : by_var[v]) {
       const Entry& e = B->ents[m];
-      work[v] += std::ldexp((double)perm::nest_cost(e.n, e.shape), e.n - 4);
+      work[v] += var_ids[v] == kClassGroup
+                     ? std::ldexp((double)e.cost, e.n - 1 - perm::kClassBits)
+                     : std::ldexp((double)perm::nest_cost(e.n, e.shape), e.n - 4);
     }
+    // the longest items first: the last ones drain quickly
+    if (var_ids[v] == kClassGroup)
+      std::stable_sort(by_var[v].begin(), by_var[v].end(), [&](uint32_t a, uint32_t b) {
+        const Entry &x = B->ents[a], &y = B->ents[b];
+        return std::ldexp(x.cost, x.walk_bits) > std::ldexp(y.cost, y.walk_bits);
+      });
   }
   std::sort(order.begin(), order.end(), [&](size_t a, size_t b) { return work[a] > work[b]; });
   for (size_t oi : order) {
-    perm_batch::Group g{var_ids[oi], (uint32_t)B->items.size(), 0, work[oi]};
+    perm_batch::Group g{var_ids[oi], (uint32_t)B->items.size(), 0, work[oi], 0};
     for (uint32_t m : by_var[oi]) {
       Entry& e = B->ents[m];
       const uint64_t lanes = 1ull << e.high_bits;
       const uint64_t cnt = (lanes + perm::kItemLanes - 1) / perm::kItemLanes;
       e.first_item = (uint32_t)B->items.size();
       e.item_count = (uint32_t)cnt;
+      g.max_n = std::max(g.max_n, e.n);
       for (uint64_t i = 0; i < cnt; ++i) B->items.push_back({m, 0u, i * perm::kItemLanes});
     }
     g.end = (uint32_t)B->items.size();
@@ -248,18 +299,38 @@ void plan_items(perm_batch* B, const std::vector<uint32_t>& idx) {
   }
 }
 
-// Device memory for `data` doubles, nm matrices, `items` items and `groups`
-// variant groups: data, matrices, items, item records, results, counters
+// Places the expanded tables of entry e at `at` (doubles into d_split);
+// returns where the next one's may begin.
+size_t place_split(Entry& e, size_t at) {
+  if (!runs_classed(e)) return at;
+  e.split_off = at;
+  at += perm::class_split_doubles(e.n, e.walk_bits - perm::kClassBits);
+  return (at + 7) / 8 * 8;
+}
+
+// The class walk's descriptor of entry e (n = 0: it runs a variant kernel).
+perm::ClassMatrix class_entry(const perm_batch* B, const Entry& e) {
+  if (!runs_classed(e)) return {};
+  const double* lane = B->d_split + e.split_off;
+  return perm::class_matrix(e.n, e.live, e.walk_bits - perm::kClassBits, B->d_data + e.rec_off,
+                            B->d_data + e.ccol_off, lane, lane + 8 * (size_t)e.n);
+}
+
+// Device memory for `data` doubles, `split` doubles of expanded tables, nm
+// matrices, `items` items and `groups` variant groups: data, tables, matrices, items, item records, results, counters
 // (one per group, then one per matrix for double-double passes), and the
 // pinned result copy.
-int alloc_device(perm_batch* B, size_t data, size_t nm, size_t items, size_t groups) {
+int alloc_device(perm_batch* B, size_t data, size_t split, size_t nm, size_t items,
+                 size_t groups) {
   const size_t data_b = align256(data * sizeof(double));
+  const size_t split_b = align256(split * sizeof(double));
+  const size_t cls_b = align256(nm * sizeof(perm::ClassMatrix));
   const size_t mats_b = align256(nm * sizeof(BatchMatrix));
   const size_t items_b = align256(items * sizeof(BatchItem));
   const size_t part_b = align256(items * sizeof(Partial));
   const size_t res_b = align256(nm * sizeof(Partial));
   const size_t ctr_b = align256((groups + nm) * sizeof(uint32_t));
-  B->dbytes = data_b + mats_b + items_b + part_b + res_b + ctr_b;
+  B->dbytes = data_b + mats_b + items_b + part_b + res_b + ctr_b + split_b + cls_b;
   HIP_TRYB(hipMalloc(&B->dmem, B->dbytes));
   char* p = (char*)B->dmem;
   B->d_data = (double*)p;
@@ -268,6 +339,9 @@ int alloc_device(perm_batch* B, size_t data, size_t nm, size_t items, size_t gro
   B->d_partials = (Partial*)(p + data_b + mats_b + items_b);
   B->d_results = (Partial*)(p + data_b + mats_b + items_b + part_b);
   B->d_counters = (uint32_t*)(p + data_b + mats_b + items_b + part_b + res_b);
+  p += data_b + mats_b + items_b + part_b + res_b + ctr_b;
+  B->d_split = (double*)p;
+  B->d_cls = (perm::ClassMatrix*)(p + split_b);
   HIP_TRYB(hipHostMalloc((void**)&B->h_results, nm * sizeof(Partial), hipHostMallocDefault));
   return PERM_OK;
 }
@@ -290,9 +364,16 @@ int build(perm_batch* B) {
     plan_items(B, all);
   }
   if (B->items.size() > 0xffffffffull) return perm::fail(PERM_ERR_SIZE, "too many items");
-  if (int st = alloc_device(B, B->data.size(), nm, B->items.size(), B->groups.size())) return st;
+  size_t split = 0;
+  for (Entry& e : B->ents) split = place_split(e, split);
+  if (int st = alloc_device(B, B->data.size(), split, nm, B->items.size(), B->groups.size()))
+    return st;
   std::vector<BatchMatrix> mats(nm);
-  for (size_t m = 0; m < nm; ++m) mats[m] = device_matrix(B, B->ents[m]);
+  std::vector<perm::ClassMatrix> cls(nm);
+  for (size_t m = 0; m < nm; ++m) {
+    mats[m] = device_matrix(B, B->ents[m]);
+    cls[m] = class_entry(B, B->ents[m]);
+  }
   hipStream_t s0 = B->s[0];
   HIP_TRYB(hipMemcpyAsync(B->d_data, B->data.data(), B->data.size() * sizeof(double),
                           hipMemcpyHostToDevice, s0));
@@ -300,6 +381,11 @@ int build(perm_batch* B) {
                           s0));
   HIP_TRYB(hipMemcpyAsync(B->d_items, B->items.data(), B->items.size() * sizeof(BatchItem),
                           hipMemcpyHostToDevice, s0));
+  if (split) {
+    HIP_TRYB(hipMemcpyAsync(B->d_cls, cls.data(), nm * sizeof(perm::ClassMatrix),
+                            hipMemcpyHostToDevice, s0));
+    HIP_TRYB(perm::launch_class_expand(B->d_cls, (uint32_t)nm, s0));
+  }
   HIP_TRYB(hipStreamSynchronize(s0));
   B->built = true;  // the graph is captured at the second run (a batch run once needs none)
   return perm::ok();
@@ -873,13 +959,17 @@ int perm_batch_compute_dense(perm_batch* B, int count, const int* dtypes,
   }
   // device memory from the orders alone (upper bounds: column store, start
   // vector and padding per matrix; every matrix's items)
-  size_t data_ub = 0, items_ub = 0;
+  size_t data_ub = 0, items_ub = 0, split_ub = 0;
   for (int i = 0; i < count; ++i) {
     const size_t n = (size_t)novs[i];
     data_ub += (2 * n - 1) * n + 2 * n + 32;
     int w = 0, h = 0;
     perm::batch_split(novs[i], B->item_log2, w, h);
     items_ub += ((1ull << h) + perm::kItemLanes - 1) / perm::kItemLanes;
+    if (novs[i] >= perm::kMinBatchClassN && class_split_ok(w)) {
+      data_ub += perm::class_tables_bound(novs[i]) + 8;
+      split_ub += perm::class_split_doubles(novs[i], w - perm::kClassBits) + 8;
+    }
   }
   if (items_ub > 0xffffffffull) return perm::fail(PERM_ERR_SIZE, "too many items");
   B->ents.assign((size_t)count, Entry{});
@@ -899,7 +989,7 @@ int perm_batch_compute_dense(perm_batch* B, int count, const int* dtypes,
     B->groups.clear();
     return st;
   };
-  if (int st = alloc_device(B, data_ub, (size_t)count, items_ub, 3 * (size_t)count))
+  if (int st = alloc_device(B, data_ub, split_ub, (size_t)count, items_ub, 3 * (size_t)count))
     return undo(st);
   mark("allocated");
   hipStream_t s0 = B->s[0];
@@ -917,6 +1007,8 @@ int perm_batch_compute_dense(perm_batch* B, int count, const int* dtypes,
   std::vector<int> status((size_t)count, PERM_OK);
   std::vector<std::string> msg((size_t)count);
   std::vector<BatchMatrix> dm((size_t)count);
+  std::vector<perm::ClassMatrix> dc((size_t)count);
+  size_t split = 0;
   const size_t phases[4] = {0, cut[0], std::max(cut[0], cut[1]), (size_t)count};
   for (int ph = 0; ph < 3; ++ph) {
     const size_t p0 = phases[ph], p1 = phases[ph + 1];
@@ -949,7 +1041,11 @@ int perm_batch_compute_dense(perm_batch* B, int count, const int* dtypes,
     }
     if (B->data.size() > data_ub) return undo(perm::fail(PERM_ERR_SIZE, "batch data bound"));
     plan_items(B, idx);
-    for (size_t k = p0; k < p1; ++k) dm[k] = device_matrix(B, B->ents[k]);
+    for (size_t k = p0; k < p1; ++k) {
+      split = place_split(B->ents[k], split);
+      dm[k] = device_matrix(B, B->ents[k]);
+      dc[k] = class_entry(B, B->ents[k]);
+    }
     mark("planned");
     // this phase's data, matrices and items, then its variant kernels
     HIP_TRYB(hipMemcpyAsync(B->d_data + d0, B->data.data() + d0,
@@ -960,17 +1056,19 @@ int perm_batch_compute_dense(perm_batch* B, int count, const int* dtypes,
       HIP_TRYB(hipMemcpyAsync(B->d_items + i0, B->items.data() + i0,
                               (B->items.size() - i0) * sizeof(BatchItem), hipMemcpyHostToDevice,
                               s0));
+    if (split_ub) {
+      HIP_TRYB(hipMemcpyAsync(B->d_cls + p0, dc.data() + p0,
+                              (p1 - p0) * sizeof(perm::ClassMatrix), hipMemcpyHostToDevice, s0));
+      HIP_TRYB(perm::launch_class_expand(B->d_cls + p0, (uint32_t)(p1 - p0), s0));
+    }
     HIP_TRYB(hipEventRecord(B->ev_fork, s0));
     for (int i = k0; i < ke; ++i) HIP_TRYB(hipStreamWaitEvent(B->s[i], B->ev_fork, 0));
     for (size_t gi = g0; gi < B->groups.size(); ++gi) {
       const auto& G = B->groups[gi];
-      const uint32_t waves = G.end - G.begin;
-      const uint32_t grid = std::max(1u, std::min<uint32_t>((waves + 3) / 4, B->max_grid));
       const int si = (int)(std::min_element(stream_work.begin() + k0, stream_work.end()) -
                            stream_work.begin());  // in [k0, ke)
       stream_work[(size_t)si] += G.work;
-      HIP_TRYB(perm::launch_batch_variant(G.vid, B->d_mats, B->d_items, G.begin, G.end,
-                                          B->d_counters + gi, B->d_partials, grid, B->s[si]));
+      HIP_TRYB(launch_group(B, gi, B->s[si]));
     }
     mark("launched");
   }

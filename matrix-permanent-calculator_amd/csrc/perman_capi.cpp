@@ -172,9 +172,8 @@ void bind_plan_memory(perm_plan* P, const Prepared& prep, void* base, bool recor
   if (prep.classed) {
     const perm::ClassTables& t = prep.tables;
     const double* d = (const double*)(b + l.col + l.x);
-    P->cls = {d, d + t.lane, d + t.block, d + t.walk, prep.plan.live, P->n,
-              perm::class_walk_bits(P->n), 0};
-    P->cls.block_bits = P->n - 1 - perm::kClassBits - P->cls.walk_bits - perm::kClassLaneBits;
+    P->cls = perm::class_matrix(P->n, prep.plan.live, perm::class_walk_bits(P->n), d, d + t.cols,
+                                d + t.lane, d + t.walk);
   }
   if (records) {
     P->L.partials = (perm::Partial*)(b + l.fixed());

@@ -402,10 +402,10 @@ int class_walk_bits(int n) {
   return std::min(7, std::max(1, n / 2 - 9));
 }
 
-// The class walk takes the FP64 pass of the single-matrix paths unless a
-// walk order or split is asked for.
+// The class walk takes the FP64 pass unless a walk order or split is asked
+// for.
 static bool class_order(int n, const NestMenu& menu) {
-  return n >= kMinClassN && n <= kMaxClassN && menu.mask == kMenuSingle.mask &&
+  return menu.min_class_n > 0 && n >= menu.min_class_n && n <= kMaxClassN &&
          env_int("PERMAN_PAIR", 1) != 0 && env_int("PERMAN_NEST", 1) != 0 &&
          env_int("PERMAN_WALK_BITS", 0) == 0;
 }
@@ -425,7 +425,10 @@ void finish_prepare(int n, const NestMenu& menu, std::vector<double>& cols, Prep
     p.classed = p.plan.cost < kClassGain * (1 << kClassBits) * (2 * n + 2);
   }
   if (p.classed) {
-    build_class_tables(p.plan, p.x0.data(), cols.data(), class_walk_bits(n), p.tables);
+    // (a batch chooses its split later, and its tables are expanded on the
+    // device)
+    build_class_tables(p.plan, p.x0.data(), cols.data(),
+                       menu.mask == kMenuSingle.mask ? class_walk_bits(n) : -1, p.tables);
     std::copy(p.plan.cols, p.plan.cols + n - 1, cp);
   } else {
     for (int k = 0; k < n - 1; ++k) cp[k] = k;

@@ -36,8 +36,8 @@ struct Prepared {
   int nu = 0, nu1 = 0, nu2 = 0;
   bool integral = false;
   double product_bits = 1e9;  // integer_product_bits (integer matrices)
-  // Class walk (single-matrix FP64 pass, orders kMinClassN..kMaxClassN): its
-  // plan and tables.  The store above then has the class columns first, so
+  // Class walk (the FP64 pass; see kMinClassN): its plan and tables.  The
+  // store above then has the class columns first, so
   // the Gray kernels' workgroups cover the same subsets as the class walk's.
   bool classed = false;
   ClassPlan plan;
@@ -60,8 +60,8 @@ void fill_zero_result(int n, bool integral, perm_result& out);
 // log2 of the class walk's groups per lane for order n.
 int class_walk_bits(int n);
 // menu: the walk shapes the kernels that will run the matrix are compiled
-// for (kMenuSingle: single-matrix paths; kMenuBatch: batch and server).
-// With kMenuSingle, orders of the class walk are prepared for it.
+// for (kMenuSingle: single-matrix paths, kMenuBatch: batches, kMenuServe: the
+// server) and the orders prepared for the class walk.
 int prepare_dense(int dtype, const void* mat, int n, Prepared& p,
                   const NestMenu& menu = kMenuSingle);
 int prepare_sparse(int dtype, const void* mat, const int* cptrs, const int* rows,

@@ -940,8 +940,8 @@ int prepare_request(perm_server* S, Request* r) {
   perm::Prepared p;
   int st = in.sparse ? perm::prepare_sparse(in.dtype, in.mat.data(), in.cptrs.data(),
                                             in.rows.data(), in.cvals.data(), n, p,
-                                            perm::kMenuBatch)
-                     : perm::prepare_dense(in.dtype, in.mat.data(), n, p, perm::kMenuBatch);
+                                            perm::kMenuServe)
+                     : perm::prepare_dense(in.dtype, in.mat.data(), n, p, perm::kMenuServe);
   if (st != PERM_OK) {
     r->error = perm::last_error();
     return st;

@@ -1,5 +1,6 @@
-// ryser_class.hip -- kernel of the class walk (ryser_class_impl.hpp) for one
-// matrix.
+// ryser_class.hip -- kernels of the class walk (ryser_class_impl.hpp): one
+// matrix, and the items of a batch.
+#include "ryser_batch.hpp"
 #include "ryser_class_impl.hpp"
 
 namespace perm {
@@ -32,6 +33,76 @@ hipError_t launch_class(const ClassLaunch& L, hipStream_t stream) {
   const size_t lds = (size_t)(m.n + 2) * kWave * sizeof(double);
   ryser_class_kernel<<<dim3((unsigned)(L.block_end - L.block_begin)), dim3(256), lds, stream>>>(
       m, L.partials, L.block_begin);
+  return hipGetLastError();
+}
+
+// Lane columns and walk offsets of one matrix per workgroup, the offsets as
+// build_class_tables forms them (double-double sums in ascending column
+// order).
+__global__ __launch_bounds__(256) void class_expand_kernel(const ClassMatrix* __restrict__ mats) {
+  const ClassMatrix m = mats[blockIdx.x];
+  const int n = m.n;
+  if (n == 0) return;
+  const double* cols = m.blockcols - (size_t)(m.walk_bits + kClassLaneBits) * n;
+  const double* x0 = m.blockcols + (size_t)m.block_bits * n;
+  const double* lane0 = cols + (size_t)m.walk_bits * n;
+  double* lane = const_cast<double*>(m.lanecols);
+  for (int i = threadIdx.x; i < 8 * n; i += blockDim.x) {
+    const int r = i >> 3, b = i & 7;
+    lane[i] = b < kClassLaneBits ? lane0[(size_t)b * n + r] : x0[(b - kClassLaneBits) * n + r];
+  }
+  double* walk = const_cast<double*>(m.walk);
+  const uint32_t entries = (uint32_t)n << m.walk_bits;
+  for (uint32_t i = threadIdx.x; i < entries; i += blockDim.x) {
+    const uint32_t t = i / (uint32_t)n, r = i - t * (uint32_t)n;
+    double hi = 0.0, lo = 0.0;
+    for (int b = 0; b < m.walk_bits; ++b) {
+      if (!((t >> b) & 1)) continue;
+      const DD e = two_sum(hi, cols[(size_t)b * n + r]);
+      hi = e.hi;
+      lo += e.lo;
+    }
+    walk[i] = hi + lo;
+  }
+}
+
+hipError_t launch_class_expand(const ClassMatrix* mats, uint32_t count, hipStream_t stream) {
+  if (count == 0) return hipSuccess;
+  class_expand_kernel<<<count, 256, 0, stream>>>(mats);
+  return hipGetLastError();
+}
+
+// Persistent: every workgroup takes items from the counter until they are
+// drained.
+__global__ __launch_bounds__(256)
+__attribute__((amdgpu_waves_per_eu(3)))
+void ryser_class_batch_kernel(const ClassMatrix* __restrict__ mats,
+                              const BatchItem* __restrict__ items, uint32_t begin, uint32_t end,
+                              uint32_t* __restrict__ counter, Partial* __restrict__ partials) {
+  extern __shared__ double lds[];
+  __shared__ Partial scratch[256 / kWave];
+  __shared__ uint32_t ticket;
+  for (;;) {
+    if (threadIdx.x == 0) ticket = atomicAdd(counter, 1u);
+    __syncthreads();
+    const uint32_t it = (uint32_t)__builtin_amdgcn_readfirstlane((int)ticket) + begin;
+    if (it >= end) break;
+    const BatchItem d = items[it];
+    const ClassMatrix m = mats[d.matrix];
+    DD s;
+    Moments mo;
+    class_walk(m, d.lane_base / kItemLanes, lds, s, mo);
+    block_reduce_store(s, mo, scratch, partials + it);
+    __syncthreads();  // (the tables, the records and the ticket are reused)
+  }
+}
+
+hipError_t launch_class_batch(const ClassMatrix* mats, const BatchItem* items, uint32_t begin,
+                              uint32_t end, uint32_t* counter, Partial* partials, int max_n,
+                              uint32_t grid, hipStream_t stream) {
+  if (end <= begin || max_n < 1 || max_n > 64 || grid == 0) return hipErrorInvalidValue;
+  const size_t lds = (size_t)(max_n + 2) * kWave * sizeof(double);
+  ryser_class_batch_kernel<<<grid, 256, lds, stream>>>(mats, items, begin, end, counter, partials);
   return hipGetLastError();
 }
 

@@ -87,3 +87,37 @@ def test_workgroups_cover_the_same_subsets_in_every_mode(n, density):
             assert abs(fp.abs_sum - dd.abs_sum) <= (n + 9 + 2.0 ** w) * 2.0 ** -52 * dd.abs_sum
     finally:
         plan.close()
+
+
+@pytest.mark.parametrize("item_log2", [8, 10, 11, 12, 15, 21, 22])
+def test_batch_splits(item_log2):
+    """Batches at every kind of split: items too small for a group of class
+    subsets per lane (8, 10: the variant kernels), one group (11), fewer
+    groups than waves (12), more (15), the longest walk table (21: 2^10
+    groups) and past it (22), for orders from below the class walk's smallest
+    on, full matrices (which keep the variant kernels) and empty columns
+    among them.  Every result within the stated errors of the single-matrix
+    path, and the same bits alone and among the others."""
+    mats = [P.synthetic_matrix(n, d, 500 + 10 * n + k, full_support=True)
+            for n in (11, 12, 13, 15, 18, 23, 28) for k, d in enumerate((0.2, 0.5, 1.0))]
+    mats.append((P.synthetic_matrix(22, 0.4, 3, binary=True)).astype(np.int32))
+    mats.append(P.synthetic_matrix(20, 0.05, 9))
+    b = P.Batch(item_log2=item_log2)
+    b.add_many(mats)
+    first, _ = b.run()
+    again, _ = b.run()
+    b.close()
+    for m, r, r2 in zip(mats, first, again):
+        one = P.dense(m)
+        n = m.shape[0]
+        assert abs(r.value - one.value) <= r.stated + one.stated, (n, item_log2, r, one)
+        assert r.certified and r.zero_pattern == one.zero_pattern
+        assert (r.value, r.sum_lo, r.abs_sum, r.err_est) == (r2.value, r2.sum_lo, r2.abs_sum,
+                                                             r2.err_est)
+    for i in (1, 7, 13, 19):
+        b = P.Batch(item_log2=item_log2)
+        b.add(mats[i])
+        (alone,), _ = b.run()
+        b.close()
+        assert (alone.value, alone.sum_lo, alone.abs_sum) == (first[i].value, first[i].sum_lo,
+                                                              first[i].abs_sum), i
