@@ -4,10 +4,10 @@
 // Each wave of the kernel loops:
 //   1. claim: first from its workgroup's current pass (kept in LDS, so the
 //      waves of a CU tend to run one variant and the instruction cache holds
-//      few walk loops), else from its cursor (>= the device head of its kind)
-//      over the published passes of its kind, one atomic increment of a
-//      pass's item counter per pass tried; the first pass with an unclaimed
-//      item gives the wave that item and becomes the workgroup's pass;
+//      few walk loops), else from the 64 passes at its cursor (>= the device
+//      head of its kind), read at once, one lane per pass: an atomic increment
+//      of the item counter of one that had items left, a different one per
+//      wave; the pass that gives the wave an item becomes the workgroup's;
 //   2. walk it: the item's 64-lane groups with the lane walk of the
 //      single-matrix kernel (ryser_dense_impl.hpp) for the pass's variant,
 //      called through one non-inlined function per variant, so each body is
@@ -19,18 +19,22 @@
 //      i+64, ... in order, then the fixed butterfly) and appends the
 //      completion record to the queue in host memory: the sum depends only
 //      on the pass, never on which waves ran which items;
-//   4. with nothing to claim: one wave at a time (at most once per 0.5 us)
-//      reads the host's tail into device memory; idle waves take up to 16
-//      published passes at a time, copy their ranges from the host mirror
+//   4. with nothing to claim: one idle wave of the workgroup, the poller,
+//      watches the device state (one line, one load per round) while the
+//      others sleep on a word in LDS.  Among the pollers one at a time (at
+//      most once per 0.5 us) reads the host's tail into device memory; they
+//      take up to 16 published passes at a time, copy their ranges from the host mirror
 //      into the arena (many waves in parallel: each GPU read of host memory
 //      is a PCIe round trip), mark them copied and advance `pub` over the
 //      passes copied so far, in publication order.  All waves of a launch
 //      leave together (a device stop flag of their kind) on the host's stop
-//      (read by each wave at most once per ms), or when the kind's activity
-//      count (claims, publications) has not moved for the idle time on the
-//      deciding wave's own clock and nothing published waits to be copied.
-// Every wait is bounded by the idle time measured on the 100 MHz real-time
-// counter, so the kernel always ends once work stops arriving.
+//      (read by each wave at most once per ms), or when every pass of the
+//      kind has completed, its activity count (claims, publications,
+//      completions) has not moved for the idle time on the deciding wave's own
+//      clock and nothing published waits to be copied.
+// Every wait ends with the items being walked and the idle time after them,
+// measured on the 100 MHz real-time counter, so the kernel always ends once
+// work stops arriving.
 #include "ryser_dense_impl.hpp"
 #include "ryser_serve.hpp"
 
@@ -44,6 +48,11 @@ __device__ __forceinline__ uint64_t uni64(uint64_t v) {
 }
 __device__ __forceinline__ uint32_t uni32(uint32_t v) {
   return (uint32_t)__builtin_amdgcn_readfirstlane((int)v);
+}
+// Lane `at`'s value (at wave-uniform).
+__device__ __forceinline__ uint64_t lane64(uint64_t v, int at) {
+  return ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(v >> 32), at) << 32) |
+         (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)v, at);
 }
 
 // Cross-wave data (counters, ring copies, item records) is read and written
@@ -76,6 +85,23 @@ __device__ __forceinline__ void store_dev_d(double* p, double v) {
 // acknowledged at the scope they were issued with) before any later one
 // issues; the compiler moves no memory access across it.
 __device__ __forceinline__ void wait_mem() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+
+// Words of the device state (one 128-byte line) as the waves read it.
+constexpr uint32_t kStateWords = 16;
+constexpr int kPub = offsetof(ServeState, pub) / 8, kPoll = offsetof(ServeState, poll) / 8,
+              kHostTail = offsetof(ServeState, host_tail) / 8,
+              kCopyClaim = offsetof(ServeState, copy_claim) / 8,
+              kHead0 = offsetof(ServeState, head) / 8, kStop0 = offsetof(ServeState, stop) / 8,
+              kActivity0 = offsetof(ServeState, activity) / 8,
+              kOpen0 = offsetof(ServeState, open) / 8;
+static_assert(kOpen0 + 2 <= (int)kStateWords, "state line");
+__device__ __forceinline__ uint32_t lds_load(const uint32_t* p) {
+  return uni32(__hip_atomic_load(const_cast<uint32_t*>(p), __ATOMIC_RELAXED,
+                                 __HIP_MEMORY_SCOPE_WORKGROUP));
+}
+__device__ __forceinline__ void lds_store(uint32_t* p, uint32_t v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
 
 // A 64-bit word of a pass header, wave-uniform.  Header fields are read
 // with device-scope loads: a launch's waves scan past completed passes'
@@ -148,7 +174,8 @@ __device__ __forceinline__ ItemSum dispatch(int vid, const ServeHeader* h, uint3
 
 // The last item of pass H is done: sum its records in item order and append
 // the completion record (lane 0) at the next queue position, tag last.
-__device__ void finish_pass(const ServeHeader* H, ServeState* st, ServeDone* done, uint32_t lane) {
+__device__ void finish_pass(const ServeHeader* H, ServeState* st, ServeDone* done, int k,
+                            uint32_t lane) {
   const uint64_t vi = HDR(H, variant);  // variant, items
   // (an export pass's sum is zero: its records are the walk's, not its own)
   const uint32_t items = ((uint32_t)vi & kServeExportFlag) ? 0u : (uint32_t)(vi >> 32);
@@ -175,6 +202,8 @@ __device__ void finish_pass(const ServeHeader* H, ServeState* st, ServeDone* don
     store_sys(&d->seq, seq);
     wait_mem();  // the record is in host memory before its tag
     store_sys(&d->tag, slot + 1);
+    atomicAdd((unsigned long long*)&st->open[k], ~0ull);  // one fewer
+    atomicAdd((unsigned long long*)&st->activity[k], 1ull);
   }
 }
 
@@ -246,13 +275,31 @@ __device__ void export_item(const ServeHeader* H, uint32_t item, uint32_t lane) 
   }
 }
 
-// Passes one wave tries per claim round.
-constexpr uint64_t kScan = 64;
+// Open passes one wave tries to take an item of per claim round.
+constexpr int kClaimTries = 4;
 // Least real-time ticks (10 ns) between two reads of the host's tail.
 constexpr uint64_t kPollTicks = 50;
 // Most passes one idle wave takes to copy in at a time (many waves copy in
 // parallel: a GPU read of host memory is a PCIe round trip).
 constexpr uint64_t kCopyBatch = 16;
+
+// The host's tail is read by one idle wave in kPollShare, unless the last
+// read is kPollLate ticks old.
+constexpr uint32_t kPollShare = 32;
+constexpr uint64_t kPollLate = 8 * kPollTicks;
+// A draw in [0, 2^16) that changes with the workgroup and every 0.64 us.
+__device__ __forceinline__ uint32_t draw_turn(uint64_t now) {
+  uint32_t h = blockIdx.x * 0x9e3779b1u + (uint32_t)(now >> 6) * 0x85ebca77u;
+  h ^= h >> 15;
+  h *= 0xc2b2ae3du;
+  return h >> 16;
+}
+// The share, of 2^16, of `pollers` that makes four tries per batch of `passes`.
+__device__ __forceinline__ uint32_t copy_share(uint64_t passes, uint32_t pollers) {
+  const uint64_t batches = (passes + kCopyBatch - 1) / kCopyBatch;
+  const uint64_t share = (batches << 18) / pollers + 1;
+  return share < (1u << 16) ? (uint32_t)share : 1u << 16;
+}
 
 // Advance `pub` over the passes whose copies are complete (64 flags per
 // round, one per lane); a wave that advanced it bumps the kind's activity.
@@ -274,7 +321,8 @@ __device__ void advance_pub(ServeControl* ctl, ServeState* st, int k, uint32_t l
   }
 }
 // Least real-time ticks between two reads of the host's stop flag by one wave
-// (1 ms: a few million reads per second over the whole launch).
+// (1 ms: a few million reads per second over the whole launch, when every
+// wave has items; an idle workgroup's poller reads it for all of them).
 constexpr uint64_t kStopTicks = 100000;
 // Most real-time ticks between two increments of the activity count by a
 // wave that keeps claiming (and at most a quarter of the idle time).
@@ -297,7 +345,14 @@ void serve_kernel(ServeControl* ctl, ServeState* st, ServeDone* done, const char
   __shared__ uint32_t copy_pre[256 / kWave][kWave + 1];  // each wave's copy plan
   __shared__ uint64_t copy_from[256 / kWave][kWave];
   __shared__ uint64_t copy_to[256 / kWave][kWave];
-  if (threadIdx.x == 0) wg_pass = 0ull;
+  // One idle wave of the workgroup at a time, the poller (wave + 1; 0: none),
+  // looks at the device state; the others sleep on wg_wake, which it moves
+  // when it finds work, and on wg_stop.
+  __shared__ uint32_t wg_poller, wg_wake, wg_stop;
+  if (threadIdx.x == 0) {
+    wg_pass = 0ull;
+    wg_poller = wg_wake = wg_stop = 0u;
+  }
   __syncthreads();
   const uint32_t lane = threadIdx.x & (kWave - 1);
   const uint32_t wave = threadIdx.x / kWave;
@@ -307,20 +362,32 @@ void serve_kernel(ServeControl* ctl, ServeState* st, ServeDone* done, const char
   // wave's own clock
   uint64_t idle_seen = ~0ull, idle_since = 0, last_activity = 0, last_stop = 0;
   uint32_t idle_rounds = 0;  // rounds in a row without work (longer sleeps after a few)
+  const uint32_t me = uni32(wave + 1);
+  uint32_t turn = 0;       // claim attempts so far
+  uint32_t woken = 0;      // wg_wake when this wave last looked for work
+  bool look = true;        // look for work without waiting for the poller (after an item)
   const uint64_t activity_ticks = idle_ticks / 4 < kActivityTicks ? idle_ticks / 4 : kActivityTicks;
   for (;;) {
     const uint64_t now = __builtin_amdgcn_s_memrealtime();
-    if (uni64(load_dev(&st->stop[k])) != 0) break;  // the host's stop, or the launch went idle
-    if (now - last_stop >= kStopTicks) {
+    if (lds_load(&wg_stop)) break;
+    bool poller = lds_load(&wg_poller) == me;
+    // the host's stop (read by a poller, or by a wave between two items), or
+    // the launch went idle (a poller sees that in the state it reads below)
+    bool stop = look && uni64(load_dev(&st->stop[k])) != 0;
+    if ((look || poller) && now - last_stop >= kStopTicks) {
       last_stop = now;
       if (uni64(load_sys(&ctl->stop)) != 0) {
+        stop = true;
         if (lane == 0) {
           atomicMax((unsigned long long*)&st->stop[k], 1ull);
           store_sys(&ctl->why[k], 2ull);
           store_sys(&ctl->ended[k], epoch);
         }
-        break;
       }
+    }
+    if (stop) {
+      if (lane == 0) lds_store(&wg_stop, 1u);
+      break;
     }
     ServeHeader* H = nullptr;
     uint32_t item = 0, items = 0;
@@ -346,31 +413,81 @@ void serve_kernel(ServeControl* ctl, ServeState* st, ServeDone* done, const char
         }
       }
     }
+    uint64_t state = 0;  // lane i: word i of the device state
     if (!H) {
-      const uint64_t pub = uni64(load_dev(&st->pub));
-      const uint64_t head = uni64(load_dev(&st->head[k]));
-      if (cursor < head) cursor = head;
-      const uint64_t scan_end = pub < cursor + kScan ? pub : cursor + kScan;
-      for (uint64_t q = cursor; q < scan_end; ++q) {
-        ServeHeader* h = (ServeHeader*)uni64(load_dev(&st->dring[q & (kServeRing - 1)]));
-        const uint64_t vi = HDR(h, variant);  // variant, items
-        if ((((uint32_t)vi & kServeDDFlag) != 0) != DD) {
-          if (q == cursor) ++cursor;  // the other kernel's pass
-          continue;
+      if (!poller) {
+        const uint32_t w = lds_load(&wg_wake);
+        if (w != woken || look) {
+          woken = w;
+          look = false;
+        } else {
+          uint32_t got = 0;
+          if (lane == 0) got = atomicCAS(&wg_poller, 0u, me) == 0u ? 1u : 0u;
+          poller = uni32(got) != 0;
+          if (!poller) {
+            __builtin_amdgcn_s_sleep(16);  // about 0.4 us
+            continue;
+          }
         }
-        const uint32_t n_items = (uint32_t)(vi >> 32);
-        uint32_t t = 0;
-        if (lane == 0) t = atomicAdd(&h->next_item, 1u);
-        t = uni32(t);
-        if (t < n_items) {
-          H = h;
-          item = t;
-          items = n_items;
-          break;
-        }
-        if (q == cursor) ++cursor;  // every item of pass q is claimed
       }
-      if (cursor > head) atomicMax((unsigned long long*)&st->head[k], (unsigned long long)cursor);
+      // one request for the whole state: thousands of waves reading its words
+      // one by one, round after round, queued every access to the line for
+      // hundreds of microseconds (first result of a burst of 2000 after 5 ms
+      // on a grid of 1024 workgroups, 1.3 ms on 256)
+      state = lane < kStateWords ? load_dev((const uint64_t*)st + lane) : 0ull;
+      if (lane64(state, kStop0 + k) != 0) {
+        if (lane == 0) lds_store(&wg_stop, 1u);
+        break;
+      }
+      const uint64_t pub = lane64(state, kPub);
+      const uint64_t head = lane64(state, kHead0 + k);
+      if (cursor < head) cursor = head;
+      if (cursor < pub) {
+        // lane i looks at pass cursor + i: two loads for 64 passes, and an
+        // atomic only on a pass that had items left (one pass per step, each
+        // tried by its atomic, took ~3 us a step and put every wave of the
+        // grid on the counters of the passes it found claimed: 4-5 us per
+        // one-item pass)
+        const uint64_t q = cursor + lane;
+        const bool in = q < pub;
+        uint64_t h = 0, vi = 0;
+        uint32_t next = 0;
+        if (in) {
+          h = load_dev(&st->dring[q & (kServeRing - 1)]);
+          const ServeHeader* hp = (const ServeHeader*)h;
+          vi = load_dev((const uint64_t*)&hp->variant);  // variant, items
+          next = __hip_atomic_load(const_cast<uint32_t*>(&hp->next_item), __ATOMIC_RELAXED,
+                                   __HIP_MEMORY_SCOPE_AGENT);
+        }
+        const bool mine = in && (((uint32_t)vi & kServeDDFlag) != 0) == DD;
+        const bool open = mine && next < (uint32_t)(vi >> 32);
+        // leading passes of the other kind, or with every item claimed
+        const uint64_t wait = __builtin_amdgcn_ballot_w64(!in || open);
+        cursor += wait ? (uint64_t)__builtin_ctzll(wait) : (uint64_t)kWave;
+        uint64_t left = __builtin_amdgcn_ballot_w64(open);
+        // the waves spread over the open passes, starting at different ones
+        for (int tries = 0; tries < kClaimTries && left && !H; ++tries) {
+          uint32_t skip = (4u * blockIdx.x + wave + turn++) %
+                          (uint32_t)__builtin_popcountll(left);
+          skip = uni32(skip);
+          uint64_t b = left;
+          for (; skip > 0; --skip) b &= b - 1;
+          const int at = __builtin_ctzll(b);
+          left &= ~(1ull << at);
+          ServeHeader* c = (ServeHeader*)lane64(h, at);
+          const uint32_t n_items = (uint32_t)(lane64(vi, at) >> 32);
+          uint32_t t = 0;
+          if (lane == 0) t = atomicAdd(&c->next_item, 1u);
+          t = uni32(t);
+          if (t < n_items) {
+            H = c;
+            item = t;
+            items = n_items;
+          }
+        }
+      }
+      if (cursor > head && lane == 0)
+        atomicMax((unsigned long long*)&st->head[k], (unsigned long long)cursor);
       if (H && lane == 0)
         __hip_atomic_store(&wg_pass, (unsigned long long)(uintptr_t)H, __ATOMIC_RELAXED,
                            __HIP_MEMORY_SCOPE_WORKGROUP);
@@ -378,6 +495,11 @@ void serve_kernel(ServeControl* ctl, ServeState* st, ServeDone* done, const char
     if (H) {
       idle_seen = ~0ull;
       idle_rounds = 0;
+      look = true;
+      if (poller && lane == 0) {  // another wave may poll, and there may be more work
+        lds_store(&wg_poller, 0u);
+        atomicAdd(&wg_wake, 1u);
+      }
       // the kind's activity count moves at least every activity_ticks while
       // this wave claims items (not on every claim: one counter per kind)
       if (now - last_activity >= activity_ticks) {
@@ -391,7 +513,7 @@ void serve_kernel(ServeControl* ctl, ServeState* st, ServeDone* done, const char
         uint32_t d = 0;
         if (lane == 0) d = atomicAdd(&H->done_items, 1u);
         d = uni32(d);
-        if (d + 1 == items) finish_pass(H, st, done, lane);
+        if (d + 1 == items) finish_pass(H, st, done, k, lane);
         continue;
       }
       uint32_t* ids = (uint32_t*)HDR(H, ids);
@@ -425,18 +547,22 @@ void serve_kernel(ServeControl* ctl, ServeState* st, ServeDone* done, const char
       d = uni32(d);
       if (d + 1 == items) {
         wait_mem();  // every record is read after the last count
-        finish_pass(H, st, done, lane);
+        finish_pass(H, st, done, k, lane);
       }
       continue;
     }
+    if (!poller) continue;
     // nothing to claim: (a) one wave per kPollTicks reads the host's tail
     // into device memory; (b) idle waves take up to kCopyBatch of the passes
     // the host published, copy their ranges from the host mirror into the
     // arena and their ring entries into dring, mark them copied, and
     // advance `pub` over the passes copied so far (in order)
+    uint64_t ht = lane64(state, kHostTail);
     {
-      const uint64_t last = uni64(load_dev(&st->poll));
-      if (now - last >= kPollTicks) {
+      const uint64_t last = lane64(state, kPoll);
+      // (one wave in kPollShare, by turns, while the reads are on time)
+      if (now - last >= kPollTicks && (now - last >= kPollLate ||
+                                       draw_turn(now) < (1u << 16) / kPollShare)) {
         unsigned long long old = 0;
         if (lane == 0)
           old = atomicCAS((unsigned long long*)&st->poll, (unsigned long long)last,
@@ -444,13 +570,16 @@ void serve_kernel(ServeControl* ctl, ServeState* st, ServeDone* done, const char
         if (uni64(old) == last) {
           const uint64_t tail = uni64(load_sys(&ctl->tail));
           if (lane == 0) atomicMax((unsigned long long*)&st->host_tail, (unsigned long long)tail);
+          if (tail > ht) ht = tail;
         }
       }
     }
     {
-      const uint64_t ht = uni64(load_dev(&st->host_tail));
-      const uint64_t c = uni64(load_dev(&st->copy_claim));
-      if (c < ht) {
+      const uint64_t c = lane64(state, kCopyClaim);
+      // About four pollers try for every batch there is to copy, taking
+      // turns; one idle for long tries one time in 8 anyway (few may be idle)
+      if (c < ht && draw_turn(now) < ((idle_rounds >= 20 ? 1u << 13 : 0u) |
+                                      copy_share(ht - c, gridDim.x))) {
         const uint64_t n = ht - c < kCopyBatch ? ht - c : kCopyBatch;
         unsigned long long old = ~0ull;
         if (lane == 0)
@@ -474,6 +603,15 @@ void serve_kernel(ServeControl* ctl, ServeState* st, ServeDone* done, const char
                       mine ? words : 0u, lane, copy_pre[wave], copy_from[wave], copy_to[wave]);
           if (lane < m) store_dev(&st->dring[q], entry);
           wait_mem();  // the copies and entries land before they are marked
+          // counted as open, by kind, before any wave can see them
+          uint64_t vi = 0;
+          if (lane < m) vi = load_dev((const uint64_t*)&((const ServeHeader*)entry)->variant);
+          const uint32_t dd = (uint32_t)__builtin_popcountll(
+              __builtin_amdgcn_ballot_w64(lane < m && ((uint32_t)vi & kServeDDFlag) != 0));
+          if (lane < 2)
+            atomicAdd((unsigned long long*)&st->open[lane],
+                      (unsigned long long)(lane == 1 ? dd : m - dd));
+          wait_mem();
           if (lane < m) store_dev(&st->copied[q], c + lane + 1);
           wait_mem();
           advance_pub(ctl, st, k, lane);
@@ -486,7 +624,7 @@ void serve_kernel(ServeControl* ctl, ServeState* st, ServeDone* done, const char
     // idle_ticks: the wave that sees it stops every wave of the launch, so a
     // launch never lingers with a few waves (the host launches again for
     // anything published meanwhile)
-    const uint64_t act = uni64(load_dev(&st->activity[k]));
+    const uint64_t act = lane64(state, kActivity0 + k);
     if (act != idle_seen) {
       idle_seen = act;
       idle_since = now;
@@ -494,13 +632,18 @@ void serve_kernel(ServeControl* ctl, ServeState* st, ServeDone* done, const char
                // never while the host has published passes not yet copied in
                // (a slow first touch of the host mirror must not end the
                // launch)
-               uni64(load_sys(&ctl->tail)) > uni64(load_dev(&st->pub))) {
+               uni64(load_sys(&ctl->tail)) > lane64(state, kPub)) {
       idle_since = now;
-    } else if (now - idle_since > idle_ticks) {
+    } else if (now - idle_since > idle_ticks && lane64(state, kOpen0 + k) == 0) {
+      // (never while a pass of the kind is being walked: a launch that ended
+      // behind one long item was launched again for the next burst, 1.5 ms
+      // on a grid of 1024 workgroups, whose scratch memory the runtime
+      // allocates per launch)
       if (lane == 0) {
         atomicMax((unsigned long long*)&st->stop[k], 1ull);
         store_sys(&ctl->why[k], 1ull | (act << 8));
         store_sys(&ctl->ended[k], epoch);  // the host may launch again (after this one)
+        lds_store(&wg_stop, 1u);
       }
       break;
     }

@@ -17,9 +17,9 @@
 // finishes a pass's last item sums the records in item order and appends
 // the pass's sum to a completion queue in pinned host memory (ServeDone),
 // which the host reads in order.  A launch ends when the host sets `stop`,
-// or when no wave of its kind has claimed an item or seen a new pass for
-// `idle` ticks: its waves leave together, never one by one while work may
-// still come.  The host launches it again (one captured graph) when it
+// or when every pass of its kind has completed and none of its waves has
+// claimed an item or seen a new pass for `idle` ticks: its waves leave
+// together, never one by one while work may still come.  The host launches it again (one captured graph) when it
 // publishes work and no launch of that kind is live.
 //
 // Orders are served by kernels of padded orders: a request of order n runs
@@ -109,7 +109,8 @@ struct ServeState {
   uint64_t head[2];      // passes of kind k before head[k] have every item claimed
   uint64_t stop[2];      // all waves of kind k leave (zeroed before each launch)
   uint64_t activity[2];  // kind k's claims and publications (idle: it stands still)
-  uint64_t pad[5];
+  uint64_t open[2];      // passes of kind k copied in and not yet completed
+  uint64_t pad[3];
   uint64_t dring[kServeRing];   // device copy of ServeControl::ring
   uint64_t copied[kServeRing];  // q + 1 once pass q's range and ring entry are in
 };
