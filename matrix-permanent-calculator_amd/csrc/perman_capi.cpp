@@ -4,7 +4,7 @@
 //
 // Host flow of one permanent (reference wrapper gpu_exact_dense.cu:640-699):
 // x-init + column store on the host, upload, Ryser kernel, grid reduction,
-// download of one 32-byte record, scale by 4(n&1)-2.  Unlike the reference,
+// one record written by the last kernel into host memory, scale by 4(n&1)-2.  Unlike the reference,
 // device buffers come from a per-device cache (no cudaMalloc/cudaFree per
 // call), the launch geometry is chosen here, and every HIP status is
 // checked.
@@ -17,6 +17,7 @@
 #include <cstring>
 #include <array>
 #include <atomic>
+#include <chrono>
 #include <limits>
 #include <mutex>
 #include <string>
@@ -59,7 +60,7 @@ struct perm_plan {
   int device = 0;
   int n = 0;
   hipStream_t stream = nullptr;
-  hipEvent_t ev0 = nullptr, ev1 = nullptr, evm = nullptr;  // evm: after the main pass
+  hipEvent_t ev0 = nullptr, ev1 = nullptr;
   DeviceBuffers mem;
   perm::DenseLaunch L{};
   int unroll_bits = 0;
@@ -83,6 +84,8 @@ struct perm_plan {
   void* rec_base = nullptr;
   uint64_t rec_cap = 0;
   double* zdev = nullptr;   // device: one variance weight per workgroup record
+  perm::HostRecord* rec = nullptr;  // pinned: where a run's last kernel reports
+  uint64_t* begin = nullptr;        // device: begin tick of the run
   perm::Partial* vrec = nullptr;  // device: 2 kVerifyUnits records (FP64, then mode 2)
   std::vector<double> zhost;      // host copy of zdev (kept between runs)
 };
@@ -94,8 +97,10 @@ namespace {
 // device buffer, reused call after call under a mutex.
 struct DeviceCache {
   std::mutex mu;
+  bool busy = false;  // a call left the stream with work it did not wait for
+  perm::HostRecord* rec = nullptr;
   hipStream_t stream = nullptr;
-  hipEvent_t ev0 = nullptr, ev1 = nullptr, evm = nullptr;
+  hipEvent_t ev0 = nullptr, ev1 = nullptr;
   void* base = nullptr;
   size_t bytes = 0;
   char* stage = nullptr;  // pinned upload staging: [column store | pad | x0]
@@ -109,6 +114,63 @@ DeviceCache& device_cache(int dev) {
   if ((int)table.size() <= dev) table.resize(dev + 1, nullptr);
   if (!table[dev]) table[dev] = new DeviceCache();  // lives until process exit
   return *table[dev];
+}
+
+// Host records of the runs (pinned): taken and given back one by one, in
+// slabs kept until the process ends (one record per plan alive, at most).
+struct RecordPool {
+  std::mutex mu;
+  std::vector<perm::HostRecord*> free;
+};
+RecordPool& record_pool() {
+  static RecordPool* pool = new RecordPool();  // (plans may outlive statics)
+  return *pool;
+}
+int take_record(perm::HostRecord** out) {
+  constexpr size_t kSlab = 64;
+  RecordPool& pool = record_pool();
+  std::lock_guard<std::mutex> g(pool.mu);
+  if (pool.free.empty()) {
+    perm::HostRecord* slab = nullptr;
+    HIP_TRY(hipHostMalloc((void**)&slab, kSlab * sizeof(perm::HostRecord),
+                          hipHostMallocPortable));
+    for (size_t i = 0; i < kSlab; ++i) {
+      slab[i].seq = 0;
+      pool.free.push_back(slab + i);
+    }
+  }
+  *out = pool.free.back();
+  pool.free.pop_back();
+  return PERM_OK;
+}
+void give_record(perm::HostRecord* r) {
+  if (!r) return;
+  RecordPool& pool = record_pool();
+  std::lock_guard<std::mutex> g(pool.mu);
+  pool.free.push_back(r);
+}
+// A number no earlier run carries.
+uint64_t next_seq() {
+  static std::atomic<uint64_t> seq{0};
+  return seq.fetch_add(1, std::memory_order_relaxed) + 1;
+}
+
+// Wait for the run `seq` to report: polled for a while (a short walk's report
+// arrives within microseconds of its last store), then waited for on the
+// stream.
+int wait_record(hipStream_t stream, const perm::HostRecord* rec, uint64_t seq) {
+  const auto arrived = [&] { return __atomic_load_n(&rec->seq, __ATOMIC_ACQUIRE) == seq; };
+  const auto t0 = std::chrono::steady_clock::now();
+  for (;;) {
+    for (int i = 0; i < 64; ++i) {
+      if (arrived()) return PERM_OK;
+      __builtin_ia32_pause();
+    }
+    if (std::chrono::steady_clock::now() - t0 > std::chrono::microseconds(400)) break;
+  }
+  HIP_TRY(hipStreamSynchronize(stream));
+  if (!arrived()) return fail(PERM_ERR_HIP, "a run ended without its record");
+  return PERM_OK;
 }
 
 // Device layout of a plan: column store, x0, the class walk's tables (these
@@ -131,7 +193,7 @@ PlanLayout plan_layout(const perm_plan* P) {
   l.col = align_up(col_doubles * sizeof(double), 256);
   l.x = align_up(2 * (size_t)P->n * sizeof(double), 256);  // start vector and its low parts
   l.part = align_up(blocks_of(1ull << P->high_bits) * sizeof(perm::Partial), 256);
-  l.res = align_up(sizeof(perm::Partial), 256);
+  l.res = align_up(sizeof(perm::Partial) + sizeof(uint64_t), 256);  // and the begin tick
   l.ids = align_up(kVerifyUnits * sizeof(uint32_t), 256);
   l.z = align_up(blocks_of(1ull << P->high_bits) * sizeof(double), 256);
   l.vrec = align_up(2 * kVerifyUnits * sizeof(perm::Partial), 256);
@@ -167,6 +229,7 @@ void bind_plan_memory(perm_plan* P, const Prepared& prep, void* base, bool recor
   P->L.x0 = (const double*)(b + l.col);
   char* r = b + l.col + l.x + l.cls;
   P->L.result = (perm::Partial*)r;
+  P->begin = (uint64_t*)(P->L.result + 1);
   P->ids = (uint32_t*)(r + l.res);
   P->vrec = (perm::Partial*)(r + l.res + l.ids);
   if (prep.classed) {
@@ -229,16 +292,30 @@ void configure_passes(perm_plan* P, int mode) {
   L.total_blocks = L.main.blocks;
 }
 
-// Enqueue the upload of the column store, start vector and class tables.
-int upload_plan(perm_plan* P, const Prepared& prep) {
-  HIP_TRY(hipMemcpyAsync((void*)P->L.colpm, prep.cs.data(), prep.cs.size() * sizeof(double),
-                         hipMemcpyHostToDevice, P->stream));
-  HIP_TRY(hipMemcpyAsync((void*)P->L.x0, prep.x0.data(), prep.x0.size() * sizeof(double),
-                         hipMemcpyHostToDevice, P->stream));
+// Bytes of the column store, start vector and class tables as they lie on the
+// device, from colpm on; packed: written there (one copy uploads them).
+size_t packed_bytes(const perm_plan* P, const Prepared& prep) {
+  const char* b = (const char*)P->L.colpm;
+  return prep.classed
+             ? (size_t)((const char*)P->cls.records - b) + prep.tables.data.size() * sizeof(double)
+             : (size_t)((const char*)P->L.x0 - b) + prep.x0.size() * sizeof(double);
+}
+void pack_matrix(const perm_plan* P, const Prepared& prep, char* packed) {
+  const char* b = (const char*)P->L.colpm;
+  std::memcpy(packed, prep.cs.data(), prep.cs.size() * sizeof(double));
+  std::memcpy(packed + ((const char*)P->L.x0 - b), prep.x0.data(),
+              prep.x0.size() * sizeof(double));
   if (prep.classed)
-    HIP_TRY(hipMemcpyAsync((void*)P->cls.records, prep.tables.data.data(),
-                           prep.tables.data.size() * sizeof(double), hipMemcpyHostToDevice,
-                           P->stream));
+    std::memcpy(packed + ((const char*)P->cls.records - b), prep.tables.data.data(),
+                prep.tables.data.size() * sizeof(double));
+}
+
+// Enqueue the upload of the prepared matrix; `packed` is its source.
+int upload_plan(perm_plan* P, const Prepared& prep, std::vector<char>& packed) {
+  packed.resize(packed_bytes(P, prep));
+  pack_matrix(P, prep, packed.data());
+  HIP_TRY(hipMemcpyAsync((void*)P->L.colpm, packed.data(), packed.size(), hipMemcpyHostToDevice,
+                         P->stream));
   return PERM_OK;
 }
 
@@ -247,7 +324,8 @@ int upload_plan(perm_plan* P, const Prepared& prep) {
 // workgroup b to L.partials[b - record_begin].
 hipError_t launch_walk(perm_plan* P, uint64_t b0, uint64_t b1, uint64_t record_begin) {
   if (P->classed && P->L.mode == 0)
-    return perm::launch_class({P->cls, P->L.partials + (b0 - record_begin), b0, b1}, P->stream);
+    return perm::launch_class(
+        {P->cls, P->L.partials + (b0 - record_begin), b0, b1, P->L.report.begin}, P->stream);
   perm::DenseLaunch L = P->L;
   L.main.block_begin = b0;
   L.main.block_end = b1;
@@ -271,13 +349,15 @@ int make_plan(int n, const Prepared& prep, perm_plan** out) {
   hipError_t e;
   if ((e = hipStreamCreateWithFlags(&P->stream, hipStreamNonBlocking)) != hipSuccess)
     return cleanup(PERM_ERR_HIP, std::string("hipStreamCreate: ") + hipGetErrorString(e));
-  if ((e = hipEventCreate(&P->ev0)) != hipSuccess || (e = hipEventCreate(&P->ev1)) != hipSuccess ||
-      (e = hipEventCreate(&P->evm)) != hipSuccess)
+  if ((e = hipEventCreate(&P->ev0)) != hipSuccess || (e = hipEventCreate(&P->ev1)) != hipSuccess)
     return cleanup(PERM_ERR_HIP, std::string("hipEventCreate: ") + hipGetErrorString(e));
+  if (take_record(&P->rec) != PERM_OK)
+    return cleanup(PERM_ERR_HIP, std::string(perm::last_error()));
   if ((e = hipMalloc(&P->mem.base, P->mem.bytes)) != hipSuccess)
     return cleanup(PERM_ERR_HIP, std::string("hipMalloc: ") + hipGetErrorString(e));
   bind_plan_memory(P, prep, P->mem.base, false);
-  if (upload_plan(P, prep) != PERM_OK)
+  std::vector<char> packed;
+  if (upload_plan(P, prep, packed) != PERM_OK)
     return cleanup(PERM_ERR_HIP, "upload: " + std::string(perm::last_error()));
   if ((e = hipStreamSynchronize(P->stream)) != hipSuccess)
     return cleanup(PERM_ERR_HIP, std::string("upload: ") + hipGetErrorString(e));
@@ -289,21 +369,20 @@ int make_plan(int n, const Prepared& prep, perm_plan** out) {
 // ms = device time of all its kernels, main_ms = of the main pass.
 int run_pass(perm_plan* P, int mode, perm::Partial& r, float& ms, float& main_ms) {
   configure_passes(P, mode);
-  // one workgroup (n <= 19): its record is the sum, the walk the only kernel
+  // one workgroup: its record is the sum, the walk the only kernel
   const bool single = P->L.total_blocks <= 1;
-  HIP_TRY(hipEventRecord(P->ev0, P->stream));
+  perm::RunReport& report = P->L.report;
+  report = {P->begin, P->rec, next_seq()};
   HIP_TRY(launch_walk(P, 0, P->L.total_blocks, 0));
-  if (!single) {
-    HIP_TRY(hipEventRecord(P->evm, P->stream));
-    HIP_TRY(perm::launch_reduce(P->L.partials, P->L.total_blocks, P->L.result, P->stream));
-  }
-  HIP_TRY(hipEventRecord(P->ev1, P->stream));
-  HIP_TRY(hipMemcpyAsync(&r, single ? P->L.partials : P->L.result, sizeof(r),
-                         hipMemcpyDeviceToHost, P->stream));
-  HIP_TRY(hipStreamSynchronize(P->stream));
-  HIP_TRY(hipEventElapsedTime(&ms, P->ev0, P->ev1));
-  if (single) main_ms = ms;
-  else HIP_TRY(hipEventElapsedTime(&main_ms, P->ev0, P->evm));
+  P->L.direct = nullptr;  // (the matrix is in place now)
+  if (!single)
+    HIP_TRY(perm::launch_reduce(P->L.partials, P->L.total_blocks, P->L.result, P->stream, report));
+  const uint64_t seq = report.seq;
+  report = {};
+  if (int s = wait_record(P->stream, P->rec, seq)) return s;
+  r = P->rec->sum;
+  ms = (float)(1e-5 * (double)(P->rec->end - P->rec->begin));  // 10 ns ticks
+  main_ms = (float)(1e-5 * (double)(P->rec->main_end - P->rec->begin));
   return PERM_OK;
 }
 
@@ -451,20 +530,23 @@ int plan_run_impl(perm_plan* P, int mode, perm_result* out) {
 }
 
 // Bind a borrowed plan to the per-device cache and upload a prepared
-// matrix (caller holds C.mu).
-int bind_oneshot(int n, const Prepared& prep, DeviceCache& C, perm_plan& P) {
+// matrix (caller holds C.mu).  direct: a walk of one workgroup may bring the
+// matrix in itself (the next launch is a run_pass).
+int bind_oneshot(int n, const Prepared& prep, DeviceCache& C, perm_plan& P, bool direct) {
   if (!C.stream) {
     HIP_TRY(hipStreamCreateWithFlags(&C.stream, hipStreamNonBlocking));
     HIP_TRY(hipEventCreate(&C.ev0));
     HIP_TRY(hipEventCreate(&C.ev1));
-    HIP_TRY(hipEventCreate(&C.evm));
+    if (int s = take_record(&C.rec)) return s;
   }
+  if (C.busy) HIP_TRY(hipStreamSynchronize(C.stream));  // an earlier call failed midway
+  C.busy = true;
   P.device = perm::current_device();
   P.borrowed = true;
+  P.rec = C.rec;
   P.stream = C.stream;
   P.ev0 = C.ev0;
   P.ev1 = C.ev1;
-  P.evm = C.evm;
   P.integral = prep.integral;
   set_shape(&P, n, prep);
   const size_t need = layout_plan(&P, n, prep);
@@ -478,11 +560,8 @@ int bind_oneshot(int n, const Prepared& prep, DeviceCache& C, perm_plan& P) {
   bind_plan_memory(&P, prep, C.base);
   // one asynchronous copy from pinned staging in the device layout; the
   // stream orders the kernels after it, and the staging is reused only by
-  // the next call under C.mu, after this call's final synchronisation
-  const size_t col_bytes = (const char*)P.L.x0 - (const char*)P.L.colpm;
-  const size_t x_end = col_bytes + prep.x0.size() * sizeof(double);
-  const size_t cls_off = (const char*)P.cls.records - (const char*)P.L.colpm;
-  const size_t up = prep.classed ? cls_off + prep.tables.data.size() * sizeof(double) : x_end;
+  // the next call under C.mu, after this call's last kernel has reported
+  const size_t up = packed_bytes(&P, prep);
   if (up > C.stage_bytes) {
     if (C.stage) HIP_TRY(hipHostFree(C.stage));
     C.stage = nullptr;
@@ -490,12 +569,12 @@ int bind_oneshot(int n, const Prepared& prep, DeviceCache& C, perm_plan& P) {
     HIP_TRY(hipHostMalloc((void**)&C.stage, up, hipHostMallocDefault));
     C.stage_bytes = up;
   }
-  HIP_TRY(hipStreamSynchronize(P.stream));  // idle unless an earlier call failed midway
-  std::memcpy(C.stage, prep.cs.data(), prep.cs.size() * sizeof(double));
-  std::memcpy(C.stage + col_bytes, prep.x0.data(), prep.x0.size() * sizeof(double));
-  if (prep.classed)
-    std::memcpy(C.stage + cls_off, prep.tables.data.data(),
-                prep.tables.data.size() * sizeof(double));
+  pack_matrix(&P, prep, C.stage);
+  if (direct && n <= perm::kMaxDirectN && !prep.classed) {
+    P.L.direct = (const double*)C.stage;
+    P.L.direct_doubles = (uint32_t)(up / sizeof(double));
+    return PERM_OK;
+  }
   HIP_TRY(hipMemcpyAsync((void*)P.L.colpm, C.stage, up, hipMemcpyHostToDevice, P.stream));
   return PERM_OK;
 }
@@ -510,8 +589,10 @@ int run_oneshot(int n, const Prepared& prep, int mode, perm_result* out) {
   DeviceCache& C = device_cache(perm::current_device());
   std::lock_guard<std::mutex> guard(C.mu);
   perm_plan P;
-  if (int s = bind_oneshot(n, prep, C, P)) return s;
-  return plan_run_impl(&P, mode, out);
+  if (int s = bind_oneshot(n, prep, C, P, true)) return s;
+  const int st = plan_run_impl(&P, mode, out);
+  C.busy = st != PERM_OK;
+  return st;
 }
 
 // The reference's chunked GPU+CPU scheduler (multigpucpu_chunks,
@@ -537,7 +618,7 @@ int run_chunked(int n, const Prepared& prep, bool use_cpu, int threads, perm_res
   DeviceCache& C = device_cache(perm::current_device());
   std::lock_guard<std::mutex> guard(C.mu);
   perm_plan P;
-  if (int s = bind_oneshot(n, prep, C, P)) return s;
+  if (int s = bind_oneshot(n, prep, C, P, false)) return s;
   configure_passes(&P, 0);
   perm::DenseLaunch& L = P.L;
   const uint64_t mb = L.main.blocks;
@@ -661,8 +742,9 @@ struct NoallocDevice {
   std::mutex mu;
   bool ready = false;
   char* ptr = nullptr;
+  perm::HostRecord* rec = nullptr;
   hipStream_t stream = nullptr;
-  hipEvent_t ev0 = nullptr, ev1 = nullptr, evm = nullptr;
+  hipEvent_t ev0 = nullptr, ev1 = nullptr;
 };
 NoallocDevice g_noalloc[kMaxNoallocDevices];
 
@@ -673,7 +755,7 @@ int noalloc_setup(NoallocDevice& D) {
   HIP_TRY(hipStreamCreateWithFlags(&D.stream, hipStreamNonBlocking));
   HIP_TRY(hipEventCreate(&D.ev0));
   HIP_TRY(hipEventCreate(&D.ev1));
-  HIP_TRY(hipEventCreate(&D.evm));
+  if (int s = take_record(&D.rec)) return s;
   D.ptr = (char*)p;
   D.ready = true;
   return PERM_OK;
@@ -754,8 +836,8 @@ void perm_plan_destroy(perm_plan* P) {
   if (P->rec_base) (void)hipFree(P->rec_base);
   if (P->ev0) (void)hipEventDestroy(P->ev0);
   if (P->ev1) (void)hipEventDestroy(P->ev1);
-  if (P->evm) (void)hipEventDestroy(P->evm);
   if (P->stream) (void)hipStreamDestroy(P->stream);
+  give_record(P->rec);
   delete P;
 }
 
@@ -791,9 +873,9 @@ int perm_dense_noalloc(int dtype, const void* mat, int nov, int algo_id, perm_re
   P.device = dev;
   P.borrowed = true;
   P.stream = D.stream;
+  P.rec = D.rec;
   P.ev0 = D.ev0;
   P.ev1 = D.ev1;
-  P.evm = D.evm;
   P.integral = p.integral;
   set_shape(&P, nov, p);
   const size_t need = layout_plan(&P, nov, p);
@@ -802,9 +884,10 @@ int perm_dense_noalloc(int dtype, const void* mat, int nov, int algo_id, perm_re
                                    " bytes of device scratch; perm_dense_noalloc has " +
                                    std::to_string(kScratchBytes) + " (n <= 35)");
   bind_plan_memory(&P, p, D.ptr);
-  // pageable sources: plan_run_impl waits for the stream before returning,
-  // and p outlives the call
-  if (int st = upload_plan(&P, p)) return st;
+  // a pageable source: plan_run_impl waits for a kernel after the copy
+  // before returning, and `packed` outlives it
+  std::vector<char> packed;
+  if (int st = upload_plan(&P, p, packed)) return st;
   return plan_run_impl(&P, -1, out);
 }
 

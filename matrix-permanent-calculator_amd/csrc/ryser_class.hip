@@ -8,12 +8,14 @@ namespace perm {
 // Workgroup b of the launch walks block block_begin + b.
 __global__ __launch_bounds__(256)
 __attribute__((amdgpu_waves_per_eu(3)))
-void ryser_class_kernel(ClassMatrix m, Partial* __restrict__ partials, uint64_t block_begin) {
+void ryser_class_kernel(ClassMatrix m, Partial* __restrict__ partials, uint64_t block_begin,
+                        uint64_t* __restrict__ begin_tick) {
   extern __shared__ double lds[];
   __shared__ Partial scratch[256 / kWave];
   // shader-clock and 100 MHz counters around the work (see ryser_dense_kernel)
   const uint64_t c0 = __builtin_amdgcn_s_memtime();
   const uint64_t r0 = __builtin_amdgcn_s_memrealtime();
+  if (begin_tick && blockIdx.x == 0 && threadIdx.x == 0) *begin_tick = r0;
   DD s;
   Moments mo;
   class_walk(m, block_begin + blockIdx.x, lds, s, mo);
@@ -32,7 +34,7 @@ hipError_t launch_class(const ClassLaunch& L, hipStream_t stream) {
     return hipErrorInvalidValue;
   const size_t lds = (size_t)(m.n + 2) * kWave * sizeof(double);
   ryser_class_kernel<<<dim3((unsigned)(L.block_end - L.block_begin)), dim3(256), lds, stream>>>(
-      m, L.partials, L.block_begin);
+      m, L.partials, L.block_begin, L.begin_tick);
   return hipGetLastError();
 }
 

@@ -6,6 +6,7 @@
 
 #include "class_plan.hpp"
 #include "ryser_device.hpp"
+#include "ryser_kernels.hpp"
 
 namespace perm {
 
@@ -36,6 +37,7 @@ struct ClassLaunch {
   ClassMatrix m;
   Partial* partials;
   uint64_t block_begin, block_end;
+  uint64_t* begin_tick = nullptr;  // device: the launch's begin (RunReport)
 };
 hipError_t launch_class(const ClassLaunch& L, hipStream_t stream);
 

@@ -24,7 +24,9 @@ hipError_t launch_dense_range_o(const DenseLaunch& L, hipStream_t s);
 // 256 threads, fixed order).
 __global__ __launch_bounds__(256) void reduce_partials_kernel(const Partial* __restrict__ in,
                                                               uint64_t count,
-                                                              Partial* __restrict__ out) {
+                                                              Partial* __restrict__ out,
+                                                              RunReport report) {
+  const uint64_t t0 = __builtin_amdgcn_s_memrealtime();
   __shared__ Partial scratch[256 / kWave];
   __shared__ double clk[256];
   DD s = {0.0, 0.0};
@@ -39,6 +41,9 @@ __global__ __launch_bounds__(256) void reduce_partials_kernel(const Partial* __r
   }
   clk[threadIdx.x] = c;
   block_reduce_store(s, m, scratch, out, 0.0, clk);  // (its first __syncthreads orders clk)
+  if (report.host && threadIdx.x == 0)
+    publish_record(report.host, scratch[0], *report.begin, t0, __builtin_amdgcn_s_memrealtime(),
+                   report.seq);
 }
 
 int dense_unroll_bits(int n) { return n - 1 < 3 ? n - 1 : 3; }
@@ -87,7 +92,7 @@ hipError_t launch_skip(const SkipLaunch& L, hipStream_t stream) {
                  : L.n <= 48 ? launch_skip_range_b(L, stream)
                              : launch_skip_range_c(L, stream);
   if (e != hipSuccess) return e;
-  reduce_partials_kernel<<<1, 256, 0, stream>>>(L.partials, L.blocks, L.result);
+  reduce_partials_kernel<<<1, 256, 0, stream>>>(L.partials, L.blocks, L.result, RunReport{});
   return hipGetLastError();
 }
 
@@ -109,8 +114,9 @@ hipError_t launch_dense_pass_only(const DenseLaunch& L, hipStream_t stream) {
   return hipErrorInvalidValue;
 }
 
-hipError_t launch_reduce(const Partial* in, uint64_t count, Partial* out, hipStream_t stream) {
-  reduce_partials_kernel<<<1, 256, 0, stream>>>(in, count, out);
+hipError_t launch_reduce(const Partial* in, uint64_t count, Partial* out, hipStream_t stream,
+                         const RunReport& report) {
+  reduce_partials_kernel<<<1, 256, 0, stream>>>(in, count, out, report);
   return hipGetLastError();
 }
 

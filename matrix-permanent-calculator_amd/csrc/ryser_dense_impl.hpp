@@ -428,12 +428,28 @@ __global__ __launch_bounds__(256)
 __attribute__((amdgpu_waves_per_eu(MODE == kFast ? kFastWavesPerEU : 1)))
 void ryser_dense_kernel(const double* __restrict__ colpm, const double* __restrict__ x0,
                         Partial* __restrict__ partials, uint64_t lane_base, uint64_t lanes,
-                        int n_walk_bits, int n_high_bits, const uint32_t* __restrict__ block_ids) {
+                        int n_walk_bits, int n_high_bits, const uint32_t* __restrict__ block_ids,
+                        RunReport report, const double* __restrict__ direct,
+                        uint32_t direct_doubles) {
   __shared__ Partial scratch[256 / kWave];
   // shader-clock and 100 MHz real-time counters around the workgroup's work:
   // their ratio is the clock the workgroup ran at (scalar reads, per wave)
   const uint64_t c0 = __builtin_amdgcn_s_memtime();
   const uint64_t r0 = __builtin_amdgcn_s_memrealtime();
+  if constexpr (N <= kMaxDirectN) {
+    // the only workgroup brings the matrix in from the caller's staging memory
+    // (a few KB, one PCIe round trip) instead of waiting for a copy before it
+    if (direct) {
+      for (uint32_t i = threadIdx.x; i < direct_doubles; i += blockDim.x)
+        const_cast<double*>(colpm)[i] = __hip_atomic_load(
+            const_cast<double*>(direct) + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      __syncthreads();
+      // (no load of the store moves above this)
+      asm volatile("" : "+s"(colpm), "+s"(x0)::"memory");
+    }
+  }
+  if (report.begin && blockIdx.x == 0 && threadIdx.x == 0) *report.begin = r0;
   // workgroup b walks lanes [lane_base + 256 b, +256); b = the listed index
   // when a list is given (the record still goes to slot blockIdx.x)
   const uint64_t b = block_ids ? (uint64_t)block_ids[blockIdx.x] : (uint64_t)blockIdx.x;
@@ -452,6 +468,10 @@ void ryser_dense_kernel(const double* __restrict__ colpm, const double* __restri
   const uint64_t r1 = __builtin_amdgcn_s_memrealtime();
   const double ratio = r1 > r0 ? (double)(c1 - c0) / (double)(r1 - r0) : 0.0;
   block_reduce_store(s, m, scratch, partials + blockIdx.x, ratio);
+  if (report.host && gridDim.x == 1 && threadIdx.x == 0) {  // one record: it is the sum
+    const uint64_t t = __builtin_amdgcn_s_memrealtime();
+    publish_record(report.host, scratch[0], r0, t, t, report.seq);
+  }
 }
 
 template <int N>
@@ -470,7 +490,8 @@ hipError_t launch_pass(const DenseLaunch& L, const LanePass& P, hipStream_t stre
   if (P.block_ids) {  // listed workgroups (indices checked by the caller)
     if (P.block_count == 0) return hipSuccess;
     ryser_dense_kernel<N, R, MODE, S><<<dim3(P.block_count), dim3(256), 0, stream>>>(
-        L.colpm, L.x0, P.partials, 0, P.lanes, P.walk_bits, P.high_bits, P.block_ids);
+        L.colpm, L.x0, P.partials, 0, P.lanes, P.walk_bits, P.high_bits, P.block_ids, RunReport{},
+        nullptr, 0);
     return hipGetLastError();
   }
   const uint64_t b0 = P.block_begin, b1 = P.block_end ? P.block_end : P.blocks;
@@ -479,7 +500,8 @@ hipError_t launch_pass(const DenseLaunch& L, const LanePass& P, hipStream_t stre
     return hipErrorInvalidValue;
   ryser_dense_kernel<N, R, MODE, S><<<dim3((unsigned)(b1 - b0)), dim3(256), 0, stream>>>(
       L.colpm, L.x0, P.partials + (b0 - P.record_begin), b0 * 256, P.lanes, P.walk_bits,
-      P.high_bits, nullptr);
+      P.high_bits, nullptr, b1 - b0 == P.blocks ? L.report : RunReport{}, L.direct,
+      L.direct_doubles);
   return hipGetLastError();
 }
 

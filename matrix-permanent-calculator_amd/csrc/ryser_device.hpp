@@ -27,6 +27,17 @@ struct Partial {
   double hi, lo, abs_sum, sq_sum, sq_run, pad;
 };
 
+// A run's result as the host receives it (pinned host memory): the grid sum,
+// real-time ticks (10 ns) of the walk's begin, its end and the end of the
+// reduction, and, stored last, the run's sequence number.  The host polls
+// `seq`: no copy, event or stream wait stands between the last kernel and the
+// caller.
+struct alignas(128) HostRecord {
+  Partial sum;
+  uint64_t begin, main_end, end;
+  uint64_t seq;
+};
+
 // The plain-summed statistics carried through every reduction.
 struct Moments {
   double a, q, r;  // abs_sum, sq_sum, sq_run
@@ -108,6 +119,24 @@ __device__ __forceinline__ void wave_reduce(DD& s, Moments& m) {
 
 __device__ __forceinline__ Partial make_partial(DD s, const Moments& m) {
   return {s.hi, s.lo, m.a, m.q, m.r, 0.0};
+}
+
+// One thread writes `sum` and the ticks, then the sequence number, past every
+// cache.
+__device__ __forceinline__ void publish_record(HostRecord* h, const Partial& sum, uint64_t begin,
+                                               uint64_t main_end, uint64_t end, uint64_t seq) {
+  auto put = [](uint64_t* p, uint64_t v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  };
+  const uint64_t* w = reinterpret_cast<const uint64_t*>(&sum);
+  uint64_t* d = reinterpret_cast<uint64_t*>(&h->sum);
+#pragma unroll
+  for (int i = 0; i < (int)(sizeof(Partial) / 8); ++i) put(d + i, w[i]);
+  put(&h->begin, begin);
+  put(&h->main_end, main_end);
+  put(&h->end, end);
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // all of it before the number
+  put(&h->seq, seq);
 }
 
 // Workgroup reduction of (s, m) into one Partial (thread 0 sums the waves).

@@ -25,6 +25,15 @@ struct LanePass {
   uint32_t block_count = 0;
 };
 
+// Where one run reports to (all null: nowhere): the begin tick of its walk in
+// device memory, for the reduction, and the host's record with the run's
+// sequence number, which the last kernel writes.
+struct RunReport {
+  uint64_t* begin = nullptr;
+  HostRecord* host = nullptr;
+  uint64_t seq = 0;
+};
+
 // One dense launch over all 2^(n-1) subsets of one matrix.
 struct DenseLaunch {
   const double* colpm;  // device: 2(n-1)+1 blocks of n doubles, [2k]=+a_k, [2k+1]=-a_k, zeros
@@ -37,7 +46,15 @@ struct DenseLaunch {
   int nu;               // rows touched by Gray column 0 (multiple of 4, < n) or n
   int nu1 = 0, nu2 = 0; // rows touched by Gray columns 0-1 and 0-2 (nested shape)
   LanePass main;        // the lanes of the walk
+  RunReport report;     // of a walk of all its workgroups
+  // n <= kMaxDirectN: where the store and start vector are in pinned host
+  // memory (as on the device, `direct_doubles` from colpm on); the walk's only
+  // workgroup copies them in first.  Null: they are in place.
+  const double* direct = nullptr;
+  uint32_t direct_doubles = 0;
 };
+// Largest order whose walk is one workgroup (2^8 lanes).
+constexpr int kMaxDirectN = 12;
 
 // One skipping walk (integer matrices; see ryser_skip_impl.hpp).
 struct SkipLaunch {
@@ -70,7 +87,8 @@ hipError_t launch_skip(const SkipLaunch& L, hipStream_t stream);
 // partial records).
 hipError_t launch_dense_pass_only(const DenseLaunch& L, hipStream_t stream);
 // The grid reduction: the DD sum of in[0, count) into *out, in a fixed order.
-hipError_t launch_reduce(const Partial* in, uint64_t count, Partial* out, hipStream_t stream);
+hipError_t launch_reduce(const Partial* in, uint64_t count, Partial* out, hipStream_t stream,
+                         const RunReport& report = {});
 // z[i] = rec[i].sq_sum + run_weight * rec[i].sq_run for i < units: the
 // modelled variance weights of a walk's workgroup records.
 hipError_t launch_unit_weights(const Partial* rec, uint64_t units, double run_weight, double* z,
