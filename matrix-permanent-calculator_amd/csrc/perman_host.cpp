@@ -410,6 +410,26 @@ static bool class_order(int n, const NestMenu& menu) {
          env_int("PERMAN_WALK_BITS", 0) == 0;
 }
 
+// The class walk multiplies the rows in another order than the Gray kernels,
+// and any subset of the rows may be one array's product: it runs only where
+// the rows' magnitudes let no such product leave the range (1022 binary
+// orders each way, 200 of them left for cancellation within the rows).  Rows
+// of +-2^400 in turn, which the Gray kernels' pairs survive, stay with them.
+static bool class_range(int n, const std::vector<double>& x0, const std::vector<double>& cols) {
+  double size[64];
+  for (int j = 0; j < n; ++j) size[j] = std::fabs(x0[j]);
+  for (int k = 0; k < n - 1; ++k)
+    for (int j = 0; j < n; ++j) size[j] += std::fabs(cols[(size_t)k * n + j]);
+  int up = 0, down = 0;
+  for (int j = 0; j < n; ++j) {
+    if (!(size[j] <= 1e300)) return false;
+    if (size[j] == 0.0) continue;
+    const int e = std::ilogb(size[j]) + 1;
+    (e > 0 ? up : down) += e;
+  }
+  return up <= 820 && down >= -820;
+}
+
 void finish_prepare(int n, const NestMenu& menu, std::vector<double>& cols, Prepared& p) {
   uint64_t sup[64];
   for (int k = 0; k < n - 1; ++k) {
@@ -419,7 +439,7 @@ void finish_prepare(int n, const NestMenu& menu, std::vector<double>& cols, Prep
   }
   if (p.integral) p.product_bits = perm::integer_product_bits(p.x0.data(), cols.data(), n);
   int cp[64], rp[64];
-  p.classed = class_order(n, menu);
+  p.classed = class_order(n, menu) && class_range(n, p.x0, cols);
   if (p.classed) {
     plan_classes(n, sup, p.plan);
     p.classed = p.plan.cost < kClassGain * (1 << kClassBits) * (2 * n + 2);

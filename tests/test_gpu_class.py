@@ -121,3 +121,20 @@ def test_batch_splits(item_log2):
         b.close()
         assert (alone.value, alone.sum_lo, alone.abs_sum) == (first[i].value, first[i].sum_lo,
                                                               first[i].abs_sum), i
+
+
+@pytest.mark.parametrize("n,exponent", [(24, 20), (24, 60), (24, 100), (24, 300), (30, 20),
+                                        (30, 60), (30, 100), (30, 300), (30, 450)])
+def test_rows_of_far_apart_magnitudes(n, exponent):
+    """Rows scaled by 2^e and 2^-e in turn: the permanent is the unscaled
+    one's, whichever walk the rows' range leaves (a class's product of twelve
+    rows of 2^100 is out of range).  The two runs' stated errors bound the
+    difference."""
+    a = P.synthetic_matrix(n, 0.6, n, full_support=True)
+    base = P.dense(a)
+    b = a.copy()
+    b[::2] *= 2.0 ** exponent
+    b[1::2] *= 2.0 ** -exponent
+    r = P.dense(b)
+    assert np.isfinite(r.value), (n, exponent, r)
+    assert abs(r.value - base.value) <= r.stated + base.stated, (n, exponent, r, base)
