@@ -10,7 +10,7 @@ namespace perm {
 namespace {
 
 constexpr int kClasses = 1 << kClassBits;
-constexpr int kRoot = kClasses - 1;
+constexpr int kHalf = kClasses / 2 - 1;  // the classes without the last column end here
 // Search effort: from kWideN on the walk takes a millisecond and more.
 constexpr int kWideN = 32;
 constexpr int kWidth = 6;
@@ -33,10 +33,10 @@ void split_rows(int n, const uint64_t* sup, const int* c, uint64_t (&rows)[kClas
     }
 }
 
-bool has_live_child(const uint64_t (&rows)[kClasses], int t) {
+bool has_live_child(const uint64_t (&rows)[kClasses], bool thin, int t) {
   for (int i = 0; i < kClassBits; ++i) {
     const int c = t & ~(1 << i);
-    if (c != t && rows[c] && class_parent(c) == t) return true;
+    if (c != t && rows[c] && class_parent(kClassBits, thin, c) == t) return true;
   }
   return false;
 }
@@ -44,23 +44,27 @@ bool has_live_child(const uint64_t (&rows)[kClasses], int t) {
 // Move rows up until every class with rows has a parent with rows (the
 // kernel starts an array from a row of its class).  A class may be computed
 // in any superset: the row's entries in the extra columns are zeros.
-void settle(uint64_t (&rows)[kClasses]) {
+// Returns false if the thin tree does not hold them.
+bool settle(uint64_t (&rows)[kClasses], bool thin) {
+  const int root = class_root(kClassBits, thin);
   auto count = [&](int t) { return __builtin_popcountll(rows[t]); };
+  auto leaf = [&](int t) { return !has_live_child(rows, thin, t); };
   auto move_one = [&](int from, int to) {
     const uint64_t one = rows[from] & -rows[from];
     rows[from] &= ~one;
     rows[to] |= one;
   };
+  for (int t = 0; t < kClasses; ++t)
+    if (rows[t] && !class_allowed(kClassBits, thin, t)) return false;
   for (int m = 0; m < kClassBits; ++m)
-    for (int t = 0; t < kRoot; ++t) {
-      if (class_popcount(t) != m || !rows[t]) continue;
-      const int p = class_parent(t);
+    for (int t = 0; t < kClasses; ++t) {
+      if (class_popcount(t) != m || !rows[t] || t == root || t == kHalf) continue;
+      const int p = class_parent(kClassBits, thin, t);
       if (rows[p]) continue;
-      const bool leaf = !has_live_child(rows, t);
       int other = -1;
       for (int i = 0; i < kClassBits; ++i)
         if (!((t >> i) & 1) && rows[t | 1 << i]) other = t | 1 << i;
-      if (leaf && other >= 0 && count(t) <= 2) {
+      if (other >= 0 && count(t) <= 2 && leaf(t)) {
         rows[other] |= rows[t];
         rows[t] = 0;
         continue;
@@ -68,33 +72,31 @@ void settle(uint64_t (&rows)[kClasses]) {
       // a row for the parent from a class inside it that can spare one
       int donor = -1;
       for (int c = 0; c < p; ++c)
-        if ((c & ~p) == 0 && rows[c] && (count(c) > 1 || !has_live_child(rows, c)) &&
+        if ((c & ~p) == 0 && rows[c] && (count(c) > 1 || leaf(c)) &&
             (donor < 0 || class_popcount(c) >= class_popcount(donor)))
           donor = c;
-      if (donor < 0) {  // (no class can spare a row: all in the root)
-        for (int c = 0; c < kRoot; ++c) {
-          rows[kRoot] |= rows[c];
+      if (donor < 0) {  // no class can spare a row
+        if (thin) return false;
+        for (int c = 0; c < root; ++c) {  // all in the root
+          rows[root] |= rows[c];
           rows[c] = 0;
         }
-        return;
+        return true;
       }
       move_one(donor, p);
     }
-  if (!rows[kRoot]) {  // no class of the last column: a row of the other half
-    for (int c = kRoot - 1; c >= 0; --c)
-      if (rows[c] && (count(c) > 1 || !has_live_child(rows, c))) {
-        move_one(c, kRoot);
-        break;
-      }
-  }
+  for (int c = kClasses - 1; !rows[root] && c >= 0; --c)  // (no row of the last column)
+    if ((c & ~root) == 0 && rows[c] && (count(c) > 1 || leaf(c))) move_one(c, root);
+  return rows[root] != 0;
 }
 
-int plan_cost(const uint64_t (&rows)[kClasses]) {
+int plan_cost(const uint64_t (&rows)[kClasses], bool thin) {
   int cost = 2 * kClasses;
   for (int t = 0; t < kClasses; ++t) {
     if (!rows[t]) continue;
     cost += (2 * __builtin_popcountll(rows[t]) - 1) << class_popcount(t);
-    if (t != kRoot && t != kRoot / 2) cost += 1 << class_popcount(class_parent(t));
+    if (t != class_root(kClassBits, thin) && t != kHalf)
+      cost += 1 << class_popcount(class_parent(kClassBits, thin, t));
   }
   return cost;
 }
@@ -105,7 +107,8 @@ void order_rows(const uint64_t (&rows)[kClasses], int t, int& at, ClassPlan& p) 
     p.rows[at++] = __builtin_ctzll(r);
   }
   for (int c = 0; c < t; ++c)
-    if (class_parent(c) == t && rows[c] && !(t == kRoot && c == kRoot / 2))
+    if (rows[c] && class_parent(kClassBits, p.thin, c) == t &&
+        !(t == class_root(kClassBits, p.thin) && c == kHalf))
       order_rows(rows, c, at, p);
 }
 
@@ -172,12 +175,14 @@ void plan_classes(int n, const uint64_t* sup, ClassPlan& p) {
   uint64_t rows[kClasses], best[kClasses];
   int best_cols[kClassBits];
   p.cost = -1;
-  auto consider = [&](const int* c) {
+  p.thin = false;
+  auto consider = [&](const int* c, bool thin) {
     split_rows(n, sup, c, rows);
-    settle(rows);
-    const int cost = plan_cost(rows);
+    if (!settle(rows, thin)) return;
+    const int cost = plan_cost(rows, thin);
     if (p.cost >= 0 && cost >= p.cost) return;
     p.cost = cost;
+    p.thin = thin;
     std::memcpy(best, rows, sizeof(rows));
     std::copy(c, c + kClassBits, best_cols);
   };
@@ -188,9 +193,23 @@ void plan_classes(int n, const uint64_t* sup, ClassPlan& p) {
       const int x = __builtin_popcountll(sup[a]), y = __builtin_popcountll(sup[b]);
       return x != y ? x < y : a < b;
     });
-    consider(c);
+    consider(c, false);
+    // the thin tree: two columns without a common row at its ends
+    for (int a = 0; a < kClassBits; ++a)
+      for (int b = a + 1; b < kClassBits; ++b) {
+        if (sup[c[a]] & sup[c[b]]) continue;
+        int d[kClassBits], at = 1;
+        d[0] = c[a];
+        d[kClassBits - 1] = c[b];
+        for (int k = 0; k < kClassBits; ++k)
+          if (k != a && k != b) d[at++] = c[k];
+        consider(d, true);
+        if (!wide) continue;
+        std::swap(d[0], d[kClassBits - 1]);
+        consider(d, true);
+      }
     std::reverse(c, c + kClassBits);
-    consider(c);
+    consider(c, false);
   }
   // Exchanges of two columns' places in the tree, while they help (2-3 % of
   // the walk for about 20 us here).
@@ -198,10 +217,11 @@ void plan_classes(int n, const uint64_t* sup, ClassPlan& p) {
     const int before = p.cost;
     int from[kClassBits];
     std::copy(best_cols, best_cols + kClassBits, from);
+    const bool thin = p.thin;
     for (int i = 0; i < kClassBits; ++i)
       for (int j = i + 1; j < kClassBits; ++j) {
         std::swap(from[i], from[j]);
-        consider(from);
+        consider(from, thin);
         std::swap(from[i], from[j]);
       }
     if (p.cost == before) break;
@@ -221,8 +241,8 @@ void plan_classes(int n, const uint64_t* sup, ClassPlan& p) {
     if (best[t]) p.live |= 1u << t;
   }
   at = 0;
-  order_rows(best, kRoot, at, p);
-  if (best[kRoot / 2]) order_rows(best, kRoot / 2, at, p);
+  order_rows(best, class_root(kClassBits, p.thin), at, p);
+  if (best[kHalf]) order_rows(best, kHalf, at, p);
 }
 
 void build_class_tables(const ClassPlan& p, const double* x0, const double* cols, int walk_bits,

@@ -24,6 +24,7 @@ struct ClassPlan {
   uint8_t classes[64];             // class of the i-th row
   uint8_t count[1 << kClassBits];  // rows in class T
   uint32_t live = 0;               // classes with rows
+  bool thin = false;               // which tree (class_tree.hpp)
   int cost = 0;                    // FP64 instructions per lane and group
 };
 

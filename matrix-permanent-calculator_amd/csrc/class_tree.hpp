@@ -12,6 +12,13 @@
 // The tree: a prefix class {0..i} hangs below {0..i+1}; any other class
 // below itself plus its lowest missing column.  (So the classes with largest
 // column i form a subtree below {0..i}.)
+//
+// Thin tree: when no row is touched by both the first and the last class
+// column, the classes of the last column are subsets of {1, .., K-1} and
+// their subtree ends in that class instead of {0, .., K-1}: its array is half
+// as long, and the final sum over the first and the last column is one factor
+// each.  Nearly every matrix of density up to 0.35 has such columns, two of
+// three at 0.4, one of thirty at 0.5 (n = 32).
 #pragma once
 #include <stdint.h>
 
@@ -22,11 +29,18 @@ constexpr int class_popcount(int t) {
   for (; t; t &= t - 1) ++c;
   return c;
 }
-// Parent class of T != 2^K - 1 (the root).
-constexpr int class_parent(int t) {
-  int i = 0;
+
+// The class whose array holds the product of all classes of the last column.
+constexpr int class_root(int k, bool thin) { return (1 << k) - (thin ? 2 : 1); }
+// Parent class of T (not the root).
+constexpr int class_parent(int k, bool thin, int t) {
+  int i = thin && (t >> (k - 1)) & 1 ? 1 : 0;
   while ((t >> i) & 1) ++i;  // lowest missing column
   return t | (1 << i);
+}
+// Classes that may hold rows.
+constexpr bool class_allowed(int k, bool thin, int t) {
+  return !thin || !((t & 1) && ((t >> (k - 1)) & 1));
 }
 // Index in P_C (C a subset of T) of entry s of P_T: the bits of s that
 // belong to columns of C, packed.

@@ -9,8 +9,8 @@
 // walk shape);
 // one persistent kernel per variant drains its group, the groups running
 // concurrently on several streams.  The FP64 pass of all matrices of the
-// class walk is one group whatever their orders (ryser_class.hip; an item is
-// a workgroup there, over the same subsets).  The whole launch sequence (counter reset,
+// class walk is one group per tree (class_tree.hpp) whatever their orders
+// (ryser_class.hip; an item is a workgroup there, over the same subsets).  The whole launch sequence (counter reset,
 // variant kernels, per-matrix reduction, result copy) is captured once in a
 // hipGraph at the second run and replayed from then on (the first run after a
 // build launches directly: a batch computed once pays no capture).
@@ -40,7 +40,8 @@ using perm::BatchMatrix;
 using perm::Partial;
 
 constexpr int kMaxStreams = 8;
-constexpr int kClassGroup = -2;
+constexpr int kClassGroup = -2, kThinGroup = -3;
+constexpr bool is_class_group(int vid) { return vid == kClassGroup || vid == kThinGroup; }
 
 struct Entry {
   int n = 0, variant = -1, walk_bits = 0, high_bits = 0;
@@ -53,6 +54,7 @@ struct Entry {
   // data buffer, its lane columns and walk offsets in the expanded tables
   bool classed = false;
   uint32_t live = 0;
+  bool thin = false;
   size_t rec_off = 0, ccol_off = 0, split_off = 0;
   int cost = 0;  // FP64 instructions per 32 subsets
   uint32_t first_item = 0, item_count = 0;
@@ -70,10 +72,10 @@ struct perm_batch {
   std::vector<Entry> ents;
   std::vector<BatchItem> items;
   struct Group {
-    int vid;      // batch variant, or kClassGroup
+    int vid;      // batch variant, or kClassGroup / kThinGroup
     uint32_t begin, end;
     double work;
-    int max_n;  // kClassGroup: largest order
+    int max_n;  // class groups: largest order
   };
   std::vector<Group> groups;
   // device
@@ -142,6 +144,7 @@ int fill_entry(perm_batch* B, Entry& e, int n, perm::Prepared& p) {
   e.classed = p.classed;
   if (p.classed) {
     e.live = p.plan.live;
+    e.thin = p.plan.thin;
     e.cost = p.plan.cost;
     while (B->data.size() % 8) B->data.push_back(0.0);  // records are 64 bytes
     e.rec_off = B->data.size();
@@ -177,10 +180,10 @@ size_t align256(size_t v) { return (v + 255) / 256 * 256; }
 hipError_t launch_group(perm_batch* B, size_t gi, hipStream_t stream) {
   const perm_batch::Group& G = B->groups[gi];
   const uint32_t items = G.end - G.begin;
-  if (G.vid == kClassGroup)
-    return perm::launch_class_batch(B->d_cls, B->d_items, G.begin, G.end, B->d_counters + gi,
-                                    B->d_partials, G.max_n, std::min(items, B->max_grid_u()),
-                                    stream);
+  if (is_class_group(G.vid))
+    return perm::launch_class_batch(G.vid == kThinGroup, B->d_cls, B->d_items, G.begin, G.end,
+                                    B->d_counters + gi, B->d_partials, G.max_n,
+                                    std::min(items, B->max_grid_u()), stream);
   const uint32_t grid = std::max(1u, std::min<uint32_t>((items + 3) / 4, B->max_grid_u()));
   return perm::launch_batch_variant(G.vid, B->d_mats, B->d_items, G.begin, G.end,
                                     B->d_counters + gi, B->d_partials, grid, stream);
@@ -245,8 +248,8 @@ bool class_split_ok(int walk_bits) {
 bool runs_classed(const Entry& e) { return e.classed && class_split_ok(e.walk_bits); }
 
 // Append the items of entries `idx` to B->items, grouped by variant (the
-// class walk's entries as one group, decreasing n), the groups in decreasing
-// work, each group a contiguous item range.
+// class walk's entries as one group per tree, longest items first), the
+// groups in decreasing work, each group a contiguous item range.
 void plan_items(perm_batch* B, const std::vector<uint32_t>& idx) {
   std::vector<std::vector<uint32_t>> by_var;
   std::vector<int> var_ids;
@@ -256,7 +259,7 @@ void plan_items(perm_batch* B, const std::vector<uint32_t>& idx) {
     e.first_item = 0;
     e.item_count = 0;
     if (e.zero) continue;  // no walk: its result is exactly 0
-    const int vid = runs_classed(e) ? kClassGroup : e.variant;
+    const int vid = !runs_classed(e) ? e.variant : e.thin ? kThinGroup : kClassGroup;
     auto it = std::find(var_ids.begin(), var_ids.end(), vid);
     if (it == var_ids.end()) {
       var_ids.push_back(vid);
@@ -271,12 +274,12 @@ void plan_items(perm_batch* B, const std::vector<uint32_t>& idx) {
     order[v] = v;
     for (uint32_t m : by_var[v]) {
       const Entry& e = B->ents[m];
-      work[v] += var_ids[v] == kClassGroup
+      work[v] += is_class_group(var_ids[v])
                      ? std::ldexp((double)e.cost, e.n - 1 - perm::kClassBits)
                      : std::ldexp((double)perm::nest_cost(e.n, e.shape), e.n - 4);
     }
     // the longest items first: the last ones drain quickly
-    if (var_ids[v] == kClassGroup)
+    if (is_class_group(var_ids[v]))
       std::stable_sort(by_var[v].begin(), by_var[v].end(), [&](uint32_t a, uint32_t b) {
         const Entry &x = B->ents[a], &y = B->ents[b];
         return std::ldexp(x.cost, x.walk_bits) > std::ldexp(y.cost, y.walk_bits);
@@ -312,8 +315,9 @@ size_t place_split(Entry& e, size_t at) {
 perm::ClassMatrix class_entry(const perm_batch* B, const Entry& e) {
   if (!runs_classed(e)) return {};
   const double* lane = B->d_split + e.split_off;
-  return perm::class_matrix(e.n, e.live, e.walk_bits - perm::kClassBits, B->d_data + e.rec_off,
-                            B->d_data + e.ccol_off, lane, lane + 8 * (size_t)e.n);
+  return perm::class_matrix(e.n, e.live, e.thin, e.walk_bits - perm::kClassBits,
+                            B->d_data + e.rec_off, B->d_data + e.ccol_off, lane,
+                            lane + 8 * (size_t)e.n);
 }
 
 // Device memory for `data` doubles, `split` doubles of expanded tables, nm

@@ -235,8 +235,9 @@ void bind_plan_memory(perm_plan* P, const Prepared& prep, void* base, bool recor
   if (prep.classed) {
     const perm::ClassTables& t = prep.tables;
     const double* d = (const double*)(b + l.col + l.x);
-    P->cls = perm::class_matrix(P->n, prep.plan.live, perm::class_walk_bits(P->n), d, d + t.cols,
-                                d + t.lane, d + t.walk);
+    P->cls = perm::class_matrix(P->n, prep.plan.live, prep.plan.thin,
+                                perm::class_walk_bits(P->n), d, d + t.cols, d + t.lane,
+                                d + t.walk);
   }
   if (records) {
     P->L.partials = (perm::Partial*)(b + l.fixed());

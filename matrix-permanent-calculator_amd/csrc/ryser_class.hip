@@ -5,9 +5,17 @@
 
 namespace perm {
 
+// Waves per SIMD: the arrays of one path through the tree are 63 doubles per
+// lane (150 registers), 47 in the thin tree (120).  The fourth wave is worth
+// 8-9 % to a batch (512 matrices of n = 24, density 0.2..0.4: one kernel for
+// both trees, at three waves, 2.21 ms; a kernel for each 2.03 ms).
+template <bool THIN>
+constexpr int kClassWaves = THIN ? 4 : 3;
+
 // Workgroup b of the launch walks block block_begin + b.
+template <bool THIN>
 __global__ __launch_bounds__(256)
-__attribute__((amdgpu_waves_per_eu(3)))
+__attribute__((amdgpu_waves_per_eu(kClassWaves<THIN>)))
 void ryser_class_kernel(ClassMatrix m, Partial* __restrict__ partials, uint64_t block_begin,
                         uint64_t* __restrict__ begin_tick) {
   extern __shared__ double lds[];
@@ -18,7 +26,7 @@ void ryser_class_kernel(ClassMatrix m, Partial* __restrict__ partials, uint64_t 
   if (begin_tick && blockIdx.x == 0 && threadIdx.x == 0) *begin_tick = r0;
   DD s;
   Moments mo;
-  class_walk(m, block_begin + blockIdx.x, lds, s, mo);
+  class_walk<THIN>(m, block_begin + blockIdx.x, lds, s, mo);
   const uint64_t c1 = __builtin_amdgcn_s_memtime();
   const uint64_t r1 = __builtin_amdgcn_s_memrealtime();
   const double ratio = r1 > r0 ? (double)(c1 - c0) / (double)(r1 - r0) : 0.0;
@@ -33,7 +41,8 @@ hipError_t launch_class(const ClassLaunch& L, hipStream_t stream) {
       L.block_end - L.block_begin > 0xffffffffull)
     return hipErrorInvalidValue;
   const size_t lds = (size_t)(m.n + 2) * kWave * sizeof(double);
-  ryser_class_kernel<<<dim3((unsigned)(L.block_end - L.block_begin)), dim3(256), lds, stream>>>(
+  const auto kernel = m.thin ? ryser_class_kernel<true> : ryser_class_kernel<false>;
+  kernel<<<dim3((unsigned)(L.block_end - L.block_begin)), dim3(256), lds, stream>>>(
       m, L.partials, L.block_begin, L.begin_tick);
   return hipGetLastError();
 }
@@ -76,8 +85,9 @@ hipError_t launch_class_expand(const ClassMatrix* mats, uint32_t count, hipStrea
 
 // Persistent: every workgroup takes items from the counter until they are
 // drained.
+template <bool THIN>
 __global__ __launch_bounds__(256)
-__attribute__((amdgpu_waves_per_eu(3)))
+__attribute__((amdgpu_waves_per_eu(kClassWaves<THIN>)))
 void ryser_class_batch_kernel(const ClassMatrix* __restrict__ mats,
                               const BatchItem* __restrict__ items, uint32_t begin, uint32_t end,
                               uint32_t* __restrict__ counter, Partial* __restrict__ partials) {
@@ -93,18 +103,19 @@ void ryser_class_batch_kernel(const ClassMatrix* __restrict__ mats,
     const ClassMatrix m = mats[d.matrix];
     DD s;
     Moments mo;
-    class_walk(m, d.lane_base / kItemLanes, lds, s, mo);
+    class_walk<THIN>(m, d.lane_base / kItemLanes, lds, s, mo);
     block_reduce_store(s, mo, scratch, partials + it);
     __syncthreads();  // (the tables, the records and the ticket are reused)
   }
 }
 
-hipError_t launch_class_batch(const ClassMatrix* mats, const BatchItem* items, uint32_t begin,
-                              uint32_t end, uint32_t* counter, Partial* partials, int max_n,
-                              uint32_t grid, hipStream_t stream) {
+hipError_t launch_class_batch(bool thin, const ClassMatrix* mats, const BatchItem* items,
+                              uint32_t begin, uint32_t end, uint32_t* counter,
+                              Partial* partials, int max_n, uint32_t grid, hipStream_t stream) {
   if (end <= begin || max_n < 1 || max_n > 64 || grid == 0) return hipErrorInvalidValue;
   const size_t lds = (size_t)(max_n + 2) * kWave * sizeof(double);
-  ryser_class_batch_kernel<<<grid, 256, lds, stream>>>(mats, items, begin, end, counter, partials);
+  const auto kernel = thin ? ryser_class_batch_kernel<true> : ryser_class_batch_kernel<false>;
+  kernel<<<grid, 256, lds, stream>>>(mats, items, begin, end, counter, partials);
   return hipGetLastError();
 }
 

@@ -20,15 +20,17 @@ struct ClassMatrix {
   int32_t n;
   int32_t walk_bits;        // 2^walk_bits groups per lane
   int32_t block_bits;
+  int32_t thin;             // which tree: the kernel that walks it
 };
 
 // The descriptor of a matrix of order n split into 2^walk_bits groups per
 // lane, from where its parts are on the device (ClassTables).
-inline ClassMatrix class_matrix(int n, uint32_t live, int walk_bits, const double* records,
-                                const double* cols, const double* lane, const double* walk) {
+inline ClassMatrix class_matrix(int n, uint32_t live, bool thin, int walk_bits,
+                                const double* records, const double* cols, const double* lane,
+                                const double* walk) {
   const int before = walk_bits + kClassLaneBits;  // columns after the class ones
-  return {records, lane,      cols + (size_t)before * n, walk,
-          live,    (int32_t)n, walk_bits,                n - 1 - kClassBits - before};
+  return {records,   lane,      cols + (size_t)before * n,     walk, live,
+          (int32_t)n, walk_bits, n - 1 - kClassBits - before, thin};
 }
 
 // Workgroups [block_begin, block_end) of the walk (block b fixes the block
@@ -47,8 +49,9 @@ struct BatchItem;
 hipError_t launch_class_expand(const ClassMatrix* mats, uint32_t count, hipStream_t stream);
 // Persistent kernel over items [begin, end), each one workgroup's walk of
 // one block (lane_base / 64) of its matrix; `counter` must be zero; the
-// record of item i goes to partials[i].  max_n: largest order among them.
-hipError_t launch_class_batch(const ClassMatrix* mats, const BatchItem* items, uint32_t begin,
+// record of item i goes to partials[i].  max_n: largest order among them;
+// thin: the tree of all of them.
+hipError_t launch_class_batch(bool thin, const ClassMatrix* mats, const BatchItem* items, uint32_t begin,
                               uint32_t end, uint32_t* counter, Partial* partials, int max_n,
                               uint32_t grid, hipStream_t stream);
 

@@ -33,7 +33,9 @@
 // Bound: VALU issue (86 % of the cycles at n = 36, density 0.5; the rest is
 // waiting for the visit's scalar loads, which three waves per SIMD -- 150
 // VGPRs: the arrays of one path through the tree are 63 doubles -- do not
-// quite cover).  Tried and dropped: K = 4 (86 VGPRs, five waves, 94 % busy)
+// quite cover; the thin tree's 120 allow four).  Thin against full tree, one
+// pass: n = 27, density 0.2 35 against 43 us; n = 33, 0.3 1.44 against 1.98 ms;
+// n = 36, 0.2 10.7 against 14.7 ms; n = 34, 0.4 3.6 against 4.4 ms.  Tried and dropped: K = 4 (86 VGPRs, five waves, 94 % busy)
 // is 12 % slower, its 21.8 instructions per subset at n = 36 outweighing the
 // waves; visits of four rows of the small classes cost more scalar work than
 // they hide; a second pair of chains in the final accumulation changes
@@ -183,41 +185,45 @@ if constexpr (M <= 2) {
 }
 
 // P_T: the product of the rows of class T and of its live children's arrays.
-template <int K, int T>
+template <int K, bool THIN, int T>
 __device__ __forceinline__ void class_eval(double (&P)[1 << class_popcount(T)], RowFeed& f,
                                            uint32_t live);
 
-template <int K, int T, int C>
+template <int K, bool THIN, int T, int C>
 __device__ __forceinline__ void class_child(double (&P)[1 << class_popcount(T)], RowFeed& f,
                                             uint32_t live) {
-  constexpr bool kChild = C < T && class_parent(C) == T && !(T == (1 << K) - 1 && C == T >> 1);
+  // (the classes without the last column meet it in the final sum only)
+  constexpr bool kChild = C < T && class_allowed(K, THIN, C) &&
+                          class_parent(K, THIN, C) == T &&
+                          !(T == class_root(K, THIN) && C == (1 << (K - 1)) - 1);
   if constexpr (kChild) {
     if ((live >> C) & 1u) {
       double Q[1 << class_popcount(C)];
-      class_eval<K, C>(Q, f, live);
+      class_eval<K, THIN, C>(Q, f, live);
 #pragma unroll
       for (int s = 0; s < (1 << class_popcount(T)); ++s) P[s] *= Q[class_drop(T, C, s)];
     }
   }
 }
 
-template <int K, int T, int... C>
+template <int K, bool THIN, int T, int... C>
 __device__ __forceinline__ void class_children(double (&P)[1 << class_popcount(T)], RowFeed& f,
                                                uint32_t live, std::integer_sequence<int, C...>) {
-  (class_child<K, T, C>(P, f, live), ...);
+  (class_child<K, THIN, T, C>(P, f, live), ...);
 }
 
-template <int K, int T>
+template <int K, bool THIN, int T>
 __device__ __forceinline__ void class_eval(double (&P)[1 << class_popcount(T)], RowFeed& f,
                                            uint32_t live) {
   class_rows<class_popcount(T)>(P, f);
-  class_children<K, T>(P, f, live, std::make_integer_sequence<int, T>{});
+  class_children<K, THIN, T>(P, f, live, std::make_integer_sequence<int, T>{});
 }
 
 // The walk of this workgroup's block `block` of one matrix: the calling
 // wave's share of the groups, summed over its lanes' subsets (signs of the
 // block and lane columns applied).  `lds` holds (n + 2) * 64 doubles (two
 // rows are read ahead); every thread of the workgroup calls it.
+template <bool THIN>
 __device__ __forceinline__ void class_walk(const ClassMatrix& m, uint64_t block, double* lds,
                                            DD& s, Moments& mo) {
   constexpr int K = kClassBits;
@@ -263,22 +269,37 @@ __device__ __forceinline__ void class_walk(const ClassMatrix& m, uint64_t block,
     f.record_off = f.row_off = 0;
     f.lane_lds = (uint32_t)(uintptr_t)((LdsPtr)lds + lane);
     f.fetch();
-    constexpr int kRoot = (1 << K) - 1, kHalf = kRoot / 2;
-    double P[1 << K];
-    class_eval<K, kRoot>(P, f, live);
+    constexpr int kAll = (1 << K) - 1, kHalf = kAll / 2, kRoot = class_root(K, THIN);
+    double P[1 << class_popcount(kRoot)];
+    class_eval<K, THIN, kRoot>(P, f, live);
     double Q[1 << (K - 1)];
     if ((live >> kHalf) & 1u) {
-      class_eval<K, kHalf>(Q, f, live);
+      class_eval<K, THIN, kHalf>(Q, f, live);
     } else {
 #pragma unroll
       for (int i = 0; i <= kHalf; ++i) Q[i] = 1.0;
     }
     double pg = 0.0;
+    if constexpr (THIN) {
+      // P over columns 1 .. K-1, Q over 0 .. K-2: the sums over the last and
+      // over the first column are one factor each (6 instead of 8
+      // instructions per four subsets)
+      constexpr int kShared = 1 << (K - 2);
 #pragma unroll
-    for (int i = 0; i <= kRoot; ++i) {
-      const double q = Q[i & kHalf];
-      pg = __builtin_fma(class_popcount(i) & 1 ? -P[i] : P[i], q, pg);
-      mo.a = __builtin_fma(__builtin_fabs(P[i]), __builtin_fabs(q), mo.a);
+      for (int i = 0; i < kShared; ++i) {
+        const double p0 = P[i], p1 = P[i + kShared], q0 = Q[2 * i], q1 = Q[2 * i + 1];
+        const double dp = p0 - p1;
+        pg = __builtin_fma(class_popcount(i) & 1 ? -dp : dp, q0 - q1, pg);
+        mo.a = __builtin_fma(__builtin_fabs(p0) + __builtin_fabs(p1),
+                             __builtin_fabs(q0) + __builtin_fabs(q1), mo.a);
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i <= kAll; ++i) {
+        const double q = Q[i & kHalf];
+        pg = __builtin_fma(class_popcount(i) & 1 ? -P[i] : P[i], q, pg);
+        mo.a = __builtin_fma(__builtin_fabs(P[i]), __builtin_fabs(q), mo.a);
+      }
     }
     p = __builtin_fma(__builtin_popcount(t) & 1 ? -1.0 : 1.0, pg, p);
     if ((g & (kRun - 1)) == kRun - 1 || g + 1 == share) {  // fold into double-double

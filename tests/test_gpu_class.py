@@ -138,3 +138,26 @@ def test_rows_of_far_apart_magnitudes(n, exponent):
     r = P.dense(b)
     assert np.isfinite(r.value), (n, exponent, r)
     assert abs(r.value - base.value) <= r.stated + base.stated, (n, exponent, r, base)
+
+
+@pytest.mark.parametrize("n", [12, 17, 23, 26])
+def test_batch_of_both_trees(n):
+    """One batch whose matrices take the thin tree (two class columns without
+    a common row), the full one, or neither, against the double-double
+    oracle (the single runs from 24 rows on)."""
+    mats = [P.synthetic_matrix(n, d, 40 * n + i, full_support=True)
+            for i, d in enumerate((0.12, 0.2, 0.3, 0.45, 0.6, 0.9, 1.0, 0.15))]
+    b = P.Batch()
+    for m in mats:
+        b.add(m)
+    out, _ = b.run()
+    b.close()
+    for d, (m, r) in enumerate(zip(mats, out)):
+        if r.zero_pattern:  # no perfect matching: exactly 0, no walk
+            assert r.value == 0.0
+        elif n < 24:
+            hi, lo = O.ryser_dd(m)
+            assert abs(r.value - (hi + lo)) <= r.stated, (n, d, r)
+        else:
+            s = P.dense(m)
+            assert abs(r.value - s.value) <= r.stated + s.stated, (n, d, r, s)
