@@ -25,6 +25,7 @@
 #include <vector>
 
 #include "../../include/perman_hip.h"
+#include "perman_cached.hpp"
 #include "perman_internal.hpp"
 #include "ryser_class.hpp"
 #include "ryser_host.hpp"
@@ -530,10 +531,9 @@ int plan_run_impl(perm_plan* P, int mode, perm_result* out) {
   return ok();
 }
 
-// Bind a borrowed plan to the per-device cache and upload a prepared
-// matrix (caller holds C.mu).  direct: a walk of one workgroup may bring the
-// matrix in itself (the next launch is a run_pass).
-int bind_oneshot(int n, const Prepared& prep, DeviceCache& C, perm_plan& P, bool direct) {
+// The cache's stream and `bytes` of its memory, with no earlier call's work
+// left on them (caller holds C.mu).
+int reserve_cache(DeviceCache& C, size_t bytes) {
   if (!C.stream) {
     HIP_TRY(hipStreamCreateWithFlags(&C.stream, hipStreamNonBlocking));
     HIP_TRY(hipEventCreate(&C.ev0));
@@ -542,27 +542,18 @@ int bind_oneshot(int n, const Prepared& prep, DeviceCache& C, perm_plan& P, bool
   }
   if (C.busy) HIP_TRY(hipStreamSynchronize(C.stream));  // an earlier call failed midway
   C.busy = true;
-  P.device = perm::current_device();
-  P.borrowed = true;
-  P.rec = C.rec;
-  P.stream = C.stream;
-  P.ev0 = C.ev0;
-  P.ev1 = C.ev1;
-  P.integral = prep.integral;
-  set_shape(&P, n, prep);
-  const size_t need = layout_plan(&P, n, prep);
-  if (need > C.bytes) {
+  if (bytes > C.bytes) {
     if (C.base) HIP_TRY(hipFree(C.base));
     C.base = nullptr;
     C.bytes = 0;
-    HIP_TRY(hipMalloc(&C.base, need));
-    C.bytes = need;
+    HIP_TRY(hipMalloc(&C.base, bytes));
+    C.bytes = bytes;
   }
-  bind_plan_memory(&P, prep, C.base);
-  // one asynchronous copy from pinned staging in the device layout; the
-  // stream orders the kernels after it, and the staging is reused only by
-  // the next call under C.mu, after this call's last kernel has reported
-  const size_t up = packed_bytes(&P, prep);
+  return PERM_OK;
+}
+
+// `up` bytes of its pinned upload staging (after reserve_cache).
+int reserve_stage(DeviceCache& C, size_t up) {
   if (up > C.stage_bytes) {
     if (C.stage) HIP_TRY(hipHostFree(C.stage));
     C.stage = nullptr;
@@ -570,6 +561,29 @@ int bind_oneshot(int n, const Prepared& prep, DeviceCache& C, perm_plan& P, bool
     HIP_TRY(hipHostMalloc((void**)&C.stage, up, hipHostMallocDefault));
     C.stage_bytes = up;
   }
+  return PERM_OK;
+}
+
+// Bind a borrowed plan to the per-device cache and upload a prepared
+// matrix (caller holds C.mu).  direct: a walk of one workgroup may bring the
+// matrix in itself (the next launch is a run_pass).
+int bind_oneshot(int n, const Prepared& prep, DeviceCache& C, perm_plan& P, bool direct) {
+  set_shape(&P, n, prep);
+  const size_t need = layout_plan(&P, n, prep);
+  if (int s = reserve_cache(C, need)) return s;
+  P.device = perm::current_device();
+  P.borrowed = true;
+  P.rec = C.rec;
+  P.stream = C.stream;
+  P.ev0 = C.ev0;
+  P.ev1 = C.ev1;
+  P.integral = prep.integral;
+  bind_plan_memory(&P, prep, C.base);
+  // one asynchronous copy from pinned staging in the device layout; the
+  // stream orders the kernels after it, and the staging is reused only by
+  // the next call under C.mu, after this call's last kernel has reported
+  const size_t up = packed_bytes(&P, prep);
+  if (int s = reserve_stage(C, up)) return s;
   pack_matrix(&P, prep, C.stage);
   if (direct && n <= perm::kMaxDirectN && !prep.classed) {
     P.L.direct = (const double*)C.stage;
@@ -595,6 +609,34 @@ int run_oneshot(int n, const Prepared& prep, int mode, perm_result* out) {
   C.busy = st != PERM_OK;
   return st;
 }
+
+}  // namespace
+
+namespace perm {
+
+int run_cached(const void* up, size_t up_bytes, size_t bytes,
+               const std::function<hipError_t(char*, hipStream_t, const RunReport&)>& launch,
+               CachedRun& out) {
+  DeviceCache& C = device_cache(current_device());
+  std::lock_guard<std::mutex> guard(C.mu);
+  const size_t tick = align_up(bytes, 256);
+  if (int s = reserve_cache(C, tick + 256)) return s;
+  if (int s = reserve_stage(C, up_bytes)) return s;
+  std::memcpy(C.stage, up, up_bytes);
+  char* base = static_cast<char*>(C.base);
+  HIP_TRY(hipMemcpyAsync(base, C.stage, up_bytes, hipMemcpyHostToDevice, C.stream));
+  const RunReport report{(uint64_t*)(base + tick), C.rec, next_seq()};
+  HIP_TRY(launch(base, C.stream, report));
+  if (int s = wait_record(C.stream, C.rec, report.seq)) return s;
+  out.sum = C.rec->sum;
+  out.ms = (float)(1e-5 * (double)(C.rec->end - C.rec->begin));
+  C.busy = false;
+  return PERM_OK;
+}
+
+}  // namespace perm
+
+namespace {
 
 // The reference's chunked GPU+CPU scheduler (multigpucpu_chunks,
 // gpu_exact_dense.cu:777-911) on one GPU.  The FP64 walk is cut into

@@ -1,6 +1,8 @@
 // perman_skip.cpp -- the sparse skipper (reference sparse ID 7,
 // gpu_perman64_xshared_coalescing_mshared_skipper, gpu_exact_sparse.cu:1123-1190)
-// on the zero-run skipping kernel (ryser_skip_impl.hpp).
+// by a search of the subsets without a zero row (ryser_skip_tree.hip), or,
+// where that would cut too little, on the zero-run skipping walk
+// (ryser_skip_impl.hpp).
 //
 // Inputs follow the reference's skipper: the dense matrix for x0 and the
 // CCS (entries > 0) for the column updates; its CRS (rptrs/cols) is accepted
@@ -13,21 +15,26 @@
 // the fewest rows not yet touched; ties by fewer nonzeros, then index) so the
 // low columns touch few rows; rows ordered by the first walk column that
 // touches them (lev, ascending; rows untouched by the walked part get lev =
-// walk_bits).  Both orders leave the permanent unchanged.
+// walk_bits).  Both orders leave the permanent unchanged.  The search decides
+// the columns in the opposite order: the high ones complete rows early.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
 #include <cmath>
+#include <cstdlib>
 #include <cstring>
+#include <map>
 #include <mutex>
 #include <numeric>
 #include <string>
 #include <vector>
 
 #include "../../include/perman_hip.h"
+#include "perman_cached.hpp"
 #include "perman_internal.hpp"
 #include "ryser_host.hpp"
 #include "ryser_kernels.hpp"
+#include "skip_tree.hpp"
 
 namespace {
 
@@ -43,6 +50,7 @@ size_t align256(size_t v) { return (v + 255) / 256 * 256; }
 struct SkipPrepared {
   std::vector<double> x0, cs;
   std::vector<int> lev;
+  std::vector<int> order;  // original index of the i-th walked column
   int walk_bits = 0, high_bits = 0;
   double product_bits = 1e9;  // integer_product_bits of the matrix
 };
@@ -51,33 +59,33 @@ struct SkipPrepared {
 void prepare_order(int n, const std::vector<double>& x0, const std::vector<double>& cols,
                    int walk_bits, SkipPrepared& sp) {
   const int B = n - 1;
-  std::vector<int> order;
-  std::vector<char> used(B, 0), touched(n, 0);
+  std::vector<int>& order = sp.order;
+  uint64_t sup[64], touched = 0, used = 0;
+  for (int k = 0; k < B; ++k) {
+    sup[k] = 0;
+    for (int j = 0; j < n; ++j)
+      if (cols[(size_t)k * n + j] != 0.0) sup[k] |= 1ull << j;
+  }
   for (int step = 0; step < B; ++step) {
     int best = -1, best_new = 0, best_nnz = 0;
     for (int k = 0; k < B; ++k) {
-      if (used[k]) continue;
-      int nw = 0, nz = 0;
-      for (int j = 0; j < n; ++j)
-        if (cols[(size_t)k * n + j] != 0.0) {
-          ++nz;
-          nw += touched[j] ? 0 : 1;
-        }
+      if (used >> k & 1) continue;
+      const int nz = __builtin_popcountll(sup[k]);
+      const int nw = __builtin_popcountll(sup[k] & ~touched);
       if (best < 0 || nw < best_new || (nw == best_new && nz < best_nnz)) {
         best = k;
         best_new = nw;
         best_nnz = nz;
       }
     }
-    used[best] = 1;
+    used |= 1ull << best;
     order.push_back(best);
-    for (int j = 0; j < n; ++j)
-      if (cols[(size_t)best * n + j] != 0.0) touched[j] = 1;
+    touched |= sup[best];
   }
   std::vector<int> lev(n, walk_bits);
   for (int j = 0; j < n; ++j)
     for (int c = 0; c < walk_bits; ++c)
-      if (cols[(size_t)order[c] * n + j] != 0.0) {
+      if (sup[order[c]] >> j & 1) {
         lev[j] = c;
         break;
       }
@@ -255,6 +263,150 @@ int run_skip(int n, const SkipPrepared& sp, int mode, int check_bits, perm::Part
   return PERM_OK;
 }
 
+// The search's plan and its expected cost.
+struct TreePlan {
+  std::vector<perm::SkipLevel> levels;
+  std::vector<perm::SkipRecord> records;
+  int top_bits = 0;
+  uint32_t waves = 0;
+  double cost = 0.0;  // records met by all prefixes, and 2 per prefix
+};
+
+// The search is expected to meet `cost` records, each some ten instructions
+// for one prefix; the walk skips what 64 neighbouring lanes can.  Where the
+// rows cut little (many columns per row, or odd sums, which are never zero)
+// the walk's 2n instructions per subset are fewer.  Kernel times, 0/1
+// matrices, search / walk: cost 0.24 2^(n-1) (n = 30, density 0.25) 0.87 /
+// 3.17 ms; 0.43 (n = 33, 0.35) 5.6 / 8.0; 0.53 (n = 30, 0.4) 0.82 / 0.86;
+// 1.6 (n = 28, 0.4) 0.46 / 0.31; 3.4 (n = 30, 0.5) 3.3 / 1.2.  Up to some
+// 2^24 records the search is the shorter one anyway (n = 25, 0.5: cost 1.5,
+// 0.080 / 0.174; n = 18, a 4x9 grid: 6.1, 0.013 / 0.076).
+constexpr double kTreeShare = 0.5, kTreeSmall = 1 << 24;
+
+// Lanes' prefixes in the first level: enough to hold the chip's waves and to
+// spread the surviving ones over them (8x10 grid: 2^18 1.1, 2^20 0.81, 2^22
+// 0.65-0.74, 2^24 0.83 ms; 8x9: 0.179, 0.184, 0.20, 0.38), and the columns
+// of the others (8x10: one 1.01, two 0.74, three 0.74 ms).
+int tree_top_bits(int b) { return std::min(b, std::max(18, std::min(24, b - 17))); }
+uint32_t tree_waves(int top_bits) { return top_bits >= 22 ? 8192u : 1u << std::min(12, top_bits - 6); }
+int tree_level_bits(int left) { return left <= 20 ? 2 : 3; }
+
+// Share of the subsets of the columns of values v at which start + sum is 0.
+double zero_share(double start, const std::vector<double>& v) {
+  constexpr size_t kMost = 256;  // (a row of many different sums: hardly ever)
+  std::map<double, double> at{{start, 1.0}};
+  for (double a : v) {
+    std::map<double, double> next;
+    for (const auto& e : at) {
+      next[e.first] += 0.5 * e.second;
+      next[e.first + a] += 0.5 * e.second;
+    }
+    at.swap(next);
+    if (at.size() > kMost) return 0.0;
+  }
+  const auto z = at.find(0.0);
+  return z == at.end() ? 0.0 : z->second;
+}
+
+// A walk's split or limits are set: the walk runs.
+bool walk_asked() {
+  for (const char* v : {"PERMAN_WALK_BITS", "PERMAN_SKIP_CHECK_BITS", "PERMAN_SKIP_BUDGET",
+                        "PERMAN_SKIP_SPLIT_BITS", "PERMAN_SKIP_LANE_REVERSE"})
+    if (std::getenv(v)) return true;
+  return false;
+}
+
+// x0 and cols as gathered (rows in the matrix's order).
+void plan_tree(int n, const std::vector<double>& x0, const std::vector<double>& cols,
+               const std::vector<int>& order, TreePlan& tp) {
+  const int B = n - 1;
+  struct Row {
+    int low = 0;  // lowest column with an entry: x is known from there on
+    double zero = 0.0;
+    std::vector<perm::SkipRecord> rec;
+  };
+  std::vector<Row> rows(n);
+  for (int j = 0; j < n; ++j) {
+    Row& r = rows[j];
+    r.low = B;
+    std::vector<double> v;
+    for (int c = B - 1; c >= 0; --c) {
+      const double a = cols[(size_t)order[c] * n + j];
+      if (a == 0.0) continue;
+      r.low = c;
+      v.push_back(a);
+      auto it = std::find_if(r.rec.begin(), r.rec.end(),
+                             [&](const perm::SkipRecord& e) { return e.value == a; });
+      if (it == r.rec.end()) it = r.rec.insert(r.rec.end(), {0, a, 0.0, 0});
+      it->mask |= 1ull << c;
+    }
+    if (r.rec.empty()) r.rec.push_back({0, 0.0, 0.0, 0});
+    r.rec.front().start = x0[j];
+    r.rec.back().last = 1;
+    r.zero = zero_share(x0[j], v);
+  }
+  std::stable_sort(rows.begin(), rows.end(),
+                   [](const Row& a, const Row& b) { return a.low > b.low; });
+  tp.top_bits = tree_top_bits(B);
+  tp.waves = tree_waves(tp.top_bits);
+  const int left = B - tp.top_bits, per = tree_level_bits(left);
+  std::vector<int> bits{tp.top_bits};
+  for (int d = left; d > 0;) {
+    const int b = d % per ? d % per : per;
+    bits.push_back(b);
+    d -= b;
+  }
+  int base = B;
+  size_t at = 0;
+  double prefixes = 1.0;
+  for (int b : bits) {
+    base -= b;
+    perm::SkipLevel lv{b, base, (uint32_t)tp.records.size(), 0};
+    prefixes *= std::ldexp(1.0, b);
+    tp.cost += 2.0 * prefixes;
+    for (; at < rows.size() && rows[at].low >= base; ++at) {
+      tp.cost += prefixes * (double)rows[at].rec.size();
+      prefixes *= 1.0 - rows[at].zero;
+      tp.records.insert(tp.records.end(), rows[at].rec.begin(), rows[at].rec.end());
+    }
+    lv.end = (uint32_t)tp.records.size();
+    tp.levels.push_back(lv);
+  }
+}
+
+int run_tree(int n, const TreePlan& tp, int mode, perm::Partial& r, double& walked_frac,
+             float& ms) {
+  const size_t lev_b = align256(tp.levels.size() * sizeof(perm::SkipLevel));
+  const size_t rec_b = align256(tp.records.size() * sizeof(perm::SkipRecord));
+  const size_t part_b = align256(tp.waves * sizeof(perm::Partial));
+  std::vector<char> up(lev_b + rec_b);
+  std::memcpy(up.data(), tp.levels.data(), tp.levels.size() * sizeof(perm::SkipLevel));
+  std::memcpy(up.data() + lev_b, tp.records.data(), tp.records.size() * sizeof(perm::SkipRecord));
+  perm::CachedRun run;
+  const int st = perm::run_cached(
+      up.data(), up.size(), up.size() + part_b + 256,
+      [&](char* d, hipStream_t stream, const perm::RunReport& report) {
+        perm::SkipTreeLaunch L{};
+        L.levels = (const perm::SkipLevel*)d;
+        L.records = (const perm::SkipRecord*)(d + lev_b);
+        L.partials = (perm::Partial*)(d + lev_b + rec_b);
+        L.result = (perm::Partial*)(d + lev_b + rec_b + part_b);
+        L.n_levels = (int)tp.levels.size();
+        L.top_bits = tp.top_bits;
+        L.mode = mode;
+        L.waves = tp.waves;
+        L.begin_tick = report.begin;
+        return perm::launch_skip_tree(L, stream, report);
+      },
+      run);
+  if (st != PERM_OK) return st;
+  r = run.sum;
+  walked_frac = r.sq_run / std::ldexp(1.0, n - 1);
+  r.sq_run = 0.0;
+  ms = run.ms;
+  return PERM_OK;
+}
+
 void fill(int n, const SkipPrepared& sp, const perm::Partial& r, int mode, perm_result* out) {
   std::memset(out, 0, sizeof(*out));
   const double scale = (double)(4 * (n & 1) - 2);
@@ -309,16 +461,26 @@ int perm_skip(int dtype, const void* mat, const int* rptrs, const int* cols, con
   // 8x9, 8x10, 6x12 against 2^4..2^6
   int check_bits = perm::env_int("PERMAN_SKIP_CHECK_BITS", 3);
   check_bits = std::max(R, std::min(check_bits, sp.walk_bits));
+  TreePlan tp;
+  bool tree = !walk_asked();
+  if (tree) {
+    plan_tree(nov, x0, cc, sp.order, tp);
+    tree = tp.cost <= std::max(kTreeSmall, kTreeShare * std::ldexp(1.0, nov - 1));
+  }
+  const auto run = [&](int mode, perm::Partial& r, double& walked, float& ms) {
+    return tree ? run_tree(nov, tp, mode, r, walked, ms)
+                : run_skip(nov, sp, mode, check_bits, r, walked, ms);
+  };
   perm::Partial r;
   double walked = 0.0;
   float ms = 0.f, ms2 = 0.f;
-  if (int s = run_skip(nov, sp, 0, check_bits, r, walked, ms)) return s;
+  if (int s = run(0, r, walked, ms)) return s;
   fill(nov, sp, r, 0, out);
   // integer matrix: X is exact, so the only escalation is double-double
   // products (exact rounding below 2^53, error ~2^-104 A above)
   if (perm::escalation_mode(*out) == 1) {
     double walked2 = 0.0;
-    if (int s = run_skip(nov, sp, 1, check_bits, r, walked2, ms2)) return s;
+    if (int s = run(1, r, walked2, ms2)) return s;
     fill(nov, sp, r, 1, out);
   }
   out->kernel_ms = (double)ms + (double)ms2;

@@ -1,0 +1,211 @@
+// ryser_skip_tree.hip -- Ryser's sum over the subsets without a zero row, by
+// a search from the last walked column down.
+//
+// For an integer matrix every x_j(S) is exact.  Deciding the columns from the
+// highest to the lowest, row j's x is known once its lowest column is: a
+// prefix of the subset at which some known x is zero contributes nothing,
+// whatever the columns below.  The prefixes are grown a level (a few columns)
+// at a time; what is left of 2^(n-1) subsets are those with a nonzero term
+// and a few times as many prefixes (grid graph 8x10, n = 40: 3.1e6 terms of
+// 5.5e11 subsets, 9e6 prefixes; the Gray walk with skips, whose waves skip
+// only what all their 64 lanes can, walks 2.6e8).
+//
+// One wave searches its share depth first.  Per level it holds a stack of
+// prefixes (subset, product of the rows known so far) in LDS; a step takes
+// 64 >> bits prefixes of one level, gives each lane one prefix and one
+// setting of the level's columns, completes the level's rows (x by the
+// popcount of the subset in the row's mask: scalar operands, no per-lane
+// table), and pushes the lanes without a zero onto the next level's stack,
+// or, at column 0, adds their terms to the lane's sum.  The deepest level
+// with a full step goes first, so a stack never holds more than a step's
+// worth and 64; when the first level is used up, levels from the top down are
+// emptied by part-filled steps.  The first level's prefixes are numbered:
+// wave w takes the tiles of 64 numbers w, w + waves, ...; the numbers are
+// scattered over the prefixes, since those that survive are alike in most of
+// their bits (unscattered, 750 of 8192 waves hold all of the 8x10 grid's
+// terms and the search takes 2.2 ms instead of 0.29).
+//
+// The order of all sums is fixed by the launch: the same result every time.
+//
+// Bound: the latency of a step (level, records and stack are read one after
+// the other), 40 to 100 of them per wave at 11 waves per compute unit (LDS);
+// the first level's 2^18..2^24 numbers are 10 to 40 us of it.  Kernel times,
+// walk -> search: grid 8x10 (4 % of the bonds missing, n = 40) 6.05 -> 0.67
+// ms, 8x10 2.95 -> 0.29, 8x9 1.48 -> 0.18, 8x8 0.29 -> 0.040; random 0/1
+// n = 30, density 0.15 0.57 -> 0.086, n = 33, 0.2 9.6 -> 2.1 ms (two passes).
+#include "ryser_device.hpp"
+#include "ryser_kernels.hpp"
+#include "skip_tree.hpp"
+
+namespace perm {
+
+typedef uint64_t Word4 __attribute__((ext_vector_type(4)));
+typedef const Word4 __attribute__((address_space(4)))* RecordPtr;
+typedef const SkipLevel __attribute__((address_space(4)))* LevelPtr;
+
+template <bool DDP>
+struct Prefix {
+  uint64_t set;
+  double prod, tail;  // (tail: double-double products only)
+};
+
+// A permutation of the numbers of `bits` bits without order: neighbours land
+// anywhere.
+__device__ __forceinline__ uint32_t scatter(uint32_t v, int bits) {
+  const uint32_t mask = (1u << bits) - 1u;
+  const int half = (bits + 1) / 2;
+  v ^= v >> half;
+  v = v * 0x9e3779b1u & mask;
+  v ^= v >> half;
+  v = v * 0x85ebca6bu & mask;
+  return v ^ v >> half;
+}
+
+// Multiply the rows of records [begin, end) into p; false: one of them is
+// zero.  Stops when that is so in every lane.
+template <bool DDP>
+__device__ __forceinline__ bool complete_rows(Prefix<DDP>& p, RecordPtr records, uint32_t begin,
+                                              uint32_t end, bool alive) {
+  double x = 0.0;
+  Word4 r = begin < end ? records[begin] : Word4{0, 0, 0, 0};
+  for (uint32_t i = begin; i < end; ++i) {
+    const Word4 next = records[i + 1 < end ? i + 1 : i];
+    x += __builtin_bit_cast(double, (uint64_t)r[2]);
+    x = __builtin_fma(__builtin_bit_cast(double, (uint64_t)r[1]),
+                      (double)__builtin_popcountll(p.set & r[0]), x);
+    if (r[3]) {
+      alive = alive && x != 0.0;
+      const double h = p.prod * x;
+      if constexpr (DDP) {
+        const double e = __builtin_fma(p.tail, x, __builtin_fma(p.prod, x, -h));
+        const DD n = quick_two_sum(h, e);
+        p.prod = n.hi;
+        p.tail = n.lo;
+      } else {
+        p.prod = h;
+      }
+      x = 0.0;
+      if (__builtin_amdgcn_ballot_w64(alive) == 0) return false;
+    }
+    r = next;
+  }
+  return alive;
+}
+
+template <bool DDP>
+__global__ __launch_bounds__(kWave)
+void ryser_skip_tree_kernel(const SkipRecord* __restrict__ records_arg,
+                            const SkipLevel* __restrict__ levels_arg, int n_levels, int top_bits,
+                            uint32_t waves, Partial* __restrict__ partials,
+                            uint64_t* __restrict__ begin_tick) {
+  extern __shared__ uint64_t lds[];
+  __shared__ Partial scratch[1];
+  if (begin_tick && blockIdx.x == 0 && threadIdx.x == 0)
+    *begin_tick = __builtin_amdgcn_s_memrealtime();
+  const RecordPtr records = (RecordPtr)records_arg;
+  const LevelPtr levels = (LevelPtr)levels_arg;
+  const uint32_t lane = threadIdx.x;
+  constexpr uint32_t kWords = DDP ? 3 : 2;
+  // stack of level l >= 1: sets, products(, tails), kSkipLevelRoom each
+  auto stack = [&](int l) { return lds + (uint32_t)(l - 1) * kWords * kSkipLevelRoom; };
+  uint32_t held = 0;  // lane l: prefixes on level l's stack
+  uint64_t tile = blockIdx.x;
+  const uint64_t tiles = 1ull << (top_bits - 6);
+  int empty = 0;  // levels [0, empty) are used up
+  int l = 0;
+  DD s = {0.0, 0.0};
+  Moments mo = {0.0, 0.0, 0.0};
+  double formed = 0.0;
+  const int last = n_levels - 1;
+  for (;;) {
+    const SkipLevel lv = {levels[l].bits, levels[l].base, levels[l].begin, levels[l].end};
+    Prefix<DDP> p;
+    bool alive;
+    if (l == 0) {
+      if (tile >= tiles) {  // used up: on with what is held
+        if (empty == 0) empty = 1;
+        if (last == 0) break;
+        l = 1;
+        continue;
+      }
+      p.set = (uint64_t)scatter((uint32_t)tile * kWave + lane, top_bits) << lv.base;
+      p.prod = 1.0;
+      p.tail = 0.0;
+      tile += waves;
+      alive = true;
+    } else {
+      const uint32_t have = (uint32_t)__builtin_amdgcn_readlane((int)held, l);
+      const uint32_t full = (uint32_t)kWave >> lv.bits;
+      if (have < full && (l > empty || have == 0)) {
+        // not a full step: back up, or, below used-up levels, down
+        if (l > empty) {
+          --l;
+        } else {
+          if (l == last) break;
+          empty = ++l;
+        }
+        continue;
+      }
+      const uint32_t take = have < full ? have : full;
+      const uint32_t at = have - take + (lane >> lv.bits);
+      alive = (lane >> lv.bits) < take;
+      const uint64_t* st = stack(l);
+      p.set = 0;
+      p.prod = 0.0;
+      p.tail = 0.0;
+      if (alive) {
+        p.set = st[at] | (uint64_t)(lane & ((1u << lv.bits) - 1u)) << lv.base;
+        p.prod = __builtin_bit_cast(double, st[kSkipLevelRoom + at]);
+        if constexpr (DDP) p.tail = __builtin_bit_cast(double, st[2 * kSkipLevelRoom + at]);
+      }
+      held = lane == (uint32_t)l ? have - take : held;
+    }
+    if (l == last) formed += alive ? 1.0 : 0.0;
+    alive = complete_rows<DDP>(p, records, lv.begin, lv.end, alive);
+    if (l == last) {
+      if (alive) {
+        const bool odd = __builtin_popcountll(p.set) & 1;
+        s = dd_add_d(s, odd ? -p.prod : p.prod);
+        if constexpr (DDP) s = dd_add_d(s, odd ? -p.tail : p.tail);
+        mo.a += __builtin_fabs(p.prod);
+        mo.q = __builtin_fma(p.prod, p.prod, mo.q);
+      }
+      continue;
+    }
+    const uint64_t mask = __builtin_amdgcn_ballot_w64(alive);
+    if (mask == 0) continue;
+    ++l;
+    const uint32_t have = (uint32_t)__builtin_amdgcn_readlane((int)held, l);
+    if (alive) {
+      const uint32_t at =
+          have + __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32),
+                                           __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
+      uint64_t* st = stack(l);
+      st[at] = p.set;
+      st[kSkipLevelRoom + at] = __builtin_bit_cast(uint64_t, p.prod);
+      if constexpr (DDP) st[2 * kSkipLevelRoom + at] = __builtin_bit_cast(uint64_t, p.tail);
+    }
+    // the pushes are read by other lanes of this wave
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    held = lane == (uint32_t)l ? have + (uint32_t)__builtin_popcountll(mask) : held;
+  }
+  // `formed` rides through the reduction as the (unused) drift statistic
+  mo.r = formed;
+  block_reduce_store(s, mo, scratch, partials + blockIdx.x);
+}
+
+hipError_t launch_skip_tree(const SkipTreeLaunch& L, hipStream_t stream, const RunReport& report) {
+  if (L.n_levels < 1 || L.n_levels > kSkipMaxLevels || L.top_bits < 6 ||
+      L.top_bits > kSkipMaxTopBits || L.waves < 1 || L.waves > 1u << (L.top_bits - 6) ||
+      (L.mode != 0 && L.mode != 1))
+    return hipErrorInvalidValue;
+  const size_t lds = (size_t)(L.n_levels - 1) * (L.mode ? 3 : 2) * kSkipLevelRoom * 8;
+  const auto kernel = L.mode ? ryser_skip_tree_kernel<true> : ryser_skip_tree_kernel<false>;
+  kernel<<<L.waves, kWave, lds, stream>>>(L.records, L.levels, L.n_levels, L.top_bits, L.waves,
+                                          L.partials, L.begin_tick);
+  if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
+  return launch_reduce(L.partials, L.waves, L.result, stream, report);
+}
+
+}  // namespace perm

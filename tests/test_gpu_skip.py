@@ -62,3 +62,52 @@ def test_fallbacks_follow_the_sparse_path():
 def test_dropin_skipper(dtype):
     G = O.grid_graph_matrix(6, 6).astype(dtype)
     assert P.dropin_skipper(G) == float(O.domino_tilings(6, 6))
+
+
+def _skip_cases():
+    """name, matrix: the search's levels from one to many, rows of one and of
+    many values, both precisions."""
+    def binary(n, d):
+        return P.synthetic_matrix(n, d, 70 + n, binary=True, full_support=True).astype(np.int32)
+
+    rng = np.random.default_rng(9)
+
+    def integer(n, d):
+        a = rng.integers(0, 4, size=(n, n)) * (rng.random((n, n)) < d)  # (CCS: entries > 0)
+        np.fill_diagonal(a, 1)
+        return a.astype(np.int32)
+
+    cases = [(f"binary{n}", binary(n, d)) for n, d in ((16, 0.3), (18, 0.9), (19, 0.3), (20, 0.2),
+                                                       (21, 0.5), (22, 0.25), (24, 0.3))]
+    cases += [(f"integer{n}", integer(n, d)) for n, d in ((16, 0.6), (20, 0.3), (23, 0.2))]
+    arrow = np.eye(20, dtype=np.int32)          # a row of the last column only
+    arrow[0, :] = arrow[:, 0] = 1
+    cases += [("identity", np.eye(24, dtype=np.int32)), ("arrow", arrow),
+              ("rotated arrow", np.ascontiguousarray(arrow[::-1, ::-1])),
+              ("dense", np.ones((17, 17), dtype=np.int32))]
+    return cases
+
+
+@pytest.mark.parametrize("name,a", _skip_cases(), ids=lambda v: v if isinstance(v, str) else "")
+def test_search_and_walk_vs_exact(monkeypatch, name, a):
+    ex = O.exact_permanent(a)
+    r = P.skip(a)
+    monkeypatch.setenv("PERMAN_SKIP_CHECK_BITS", "3")  # the walk
+    w = P.skip(a)
+    for q in (r, w):
+        assert abs(q.value - float(ex)) <= q.stated + 2.0 ** -53 * abs(float(ex)), (name, q, ex)
+    assert r.value == w.value or r.stated > 0 or w.stated > 0
+    again = [P.skip(a).value for _ in range(3)]
+    assert again == [again[0]] * 3
+
+
+@pytest.mark.parametrize("n,density", [(28, 0.15), (30, 0.3), (33, 0.15), (36, 0.1)])
+def test_search_vs_walk_at_larger_orders(monkeypatch, n, density):
+    a = P.synthetic_matrix(n, density, 5 * n, binary=True, full_support=True).astype(np.int32)
+    r = P.skip(a)
+    with monkeypatch.context() as m:
+        m.setenv("PERMAN_SKIP_CHECK_BITS", "3")
+        w = P.skip(a)
+    assert r.main_subsets <= w.main_subsets
+    assert r.value == w.value or abs(r.value - w.value) <= r.stated + w.stated
+    assert [P.skip(a).value for _ in range(3)] == [r.value] * 3
