@@ -71,6 +71,8 @@ struct perm_plan {
   bool classed = false;  // the FP64 pass is the class walk
   size_t table_doubles = 0;  // ClassTables::data
   perm::ClassMatrix cls{};
+  uint32_t tree_modes = 0;  // passes that are a search (bit m: mode m)
+  perm::SkipTreeLaunch tree{};
   int nu = 0;             // rows touched by Gray column 0 for the FP64 kernel (n: none)
   int nu1 = 0, nu2 = 0;   // rows touched by Gray columns 0-1 and 0-2 (n: not nested)
   bool integral = false;  // every entry an integer of magnitude < 2^31
@@ -239,6 +241,8 @@ void bind_plan_memory(perm_plan* P, const Prepared& prep, void* base, bool recor
     P->cls = perm::class_matrix(P->n, prep.plan.live, prep.plan.thin,
                                 perm::class_walk_bits(P->n), d, d + t.cols, d + t.lane,
                                 d + t.walk);
+    P->tree_modes = prep.tree_modes;
+    if (prep.tree_modes) P->tree = perm::tree_launch(prep.tree, d + prep.tree_off, 0);
   }
   if (records) {
     P->L.partials = (perm::Partial*)(b + l.fixed());
@@ -371,6 +375,21 @@ int make_plan(int n, const Prepared& prep, perm_plan** out) {
 // ms = device time of all its kernels, main_ms = of the main pass.
 int run_pass(perm_plan* P, int mode, perm::Partial& r, float& ms, float& main_ms) {
   configure_passes(P, mode);
+  if ((P->tree_modes >> mode) & 1u && P->tree.waves <= P->L.total_blocks) {
+    perm::SkipTreeLaunch T = P->tree;
+    T.mode = mode;
+    T.partials = P->L.partials;
+    T.result = P->L.result;
+    T.begin_tick = P->begin;
+    const perm::RunReport report{P->begin, P->rec, next_seq()};
+    HIP_TRY(perm::launch_skip_tree(T, P->stream, report));
+    if (int s = wait_record(P->stream, P->rec, report.seq)) return s;
+    r = P->rec->sum;
+    r.sq_run = 0.0;  // (the subsets formed)
+    ms = (float)(1e-5 * (double)(P->rec->end - P->rec->begin));
+    main_ms = (float)(1e-5 * (double)(P->rec->main_end - P->rec->begin));
+    return PERM_OK;
+  }
   // one workgroup: its record is the sum, the walk the only kernel
   const bool single = P->L.total_blocks <= 1;
   perm::RunReport& report = P->L.report;

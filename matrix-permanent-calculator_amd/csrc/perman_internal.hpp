@@ -7,6 +7,7 @@
 #include <vector>
 
 #include "class_plan.hpp"
+#include "skip_tree.hpp"
 #include "nest_shape.hpp"
 
 struct perm_result;
@@ -42,6 +43,12 @@ struct Prepared {
   bool classed = false;
   ClassPlan plan;
   ClassTables tables;
+  // Search of the subsets without a zero row (ryser_skip_tree.hip), for sparse
+  // integer matrices: its passes (bit m: mode m), its plan and where it is in
+  // `tables` (doubles, after the class walk's own).
+  uint32_t tree_modes = 0;
+  TreePlan tree;
+  size_t tree_off = 0;
   // no perfect matching in the matrix's nonzero pattern: every term of the
   // permanent vanishes, the result is exactly 0 and no walk is run
   bool zero = false;

@@ -23,7 +23,6 @@
 #include <cmath>
 #include <cstdlib>
 #include <cstring>
-#include <map>
 #include <mutex>
 #include <numeric>
 #include <string>
@@ -59,29 +58,15 @@ struct SkipPrepared {
 void prepare_order(int n, const std::vector<double>& x0, const std::vector<double>& cols,
                    int walk_bits, SkipPrepared& sp) {
   const int B = n - 1;
-  std::vector<int>& order = sp.order;
-  uint64_t sup[64], touched = 0, used = 0;
+  uint64_t sup[64];
   for (int k = 0; k < B; ++k) {
     sup[k] = 0;
     for (int j = 0; j < n; ++j)
       if (cols[(size_t)k * n + j] != 0.0) sup[k] |= 1ull << j;
   }
-  for (int step = 0; step < B; ++step) {
-    int best = -1, best_new = 0, best_nnz = 0;
-    for (int k = 0; k < B; ++k) {
-      if (used >> k & 1) continue;
-      const int nz = __builtin_popcountll(sup[k]);
-      const int nw = __builtin_popcountll(sup[k] & ~touched);
-      if (best < 0 || nw < best_new || (nw == best_new && nz < best_nnz)) {
-        best = k;
-        best_new = nw;
-        best_nnz = nz;
-      }
-    }
-    used |= 1ull << best;
-    order.push_back(best);
-    touched |= sup[best];
-  }
+  sp.order.resize(B);
+  perm::skip_order(B, sup, sp.order.data());
+  const std::vector<int>& order = sp.order;
   std::vector<int> lev(n, walk_bits);
   for (int j = 0; j < n; ++j)
     for (int c = 0; c < walk_bits; ++c)
@@ -263,15 +248,6 @@ int run_skip(int n, const SkipPrepared& sp, int mode, int check_bits, perm::Part
   return PERM_OK;
 }
 
-// The search's plan and its expected cost.
-struct TreePlan {
-  std::vector<perm::SkipLevel> levels;
-  std::vector<perm::SkipRecord> records;
-  int top_bits = 0;
-  uint32_t waves = 0;
-  double cost = 0.0;  // records met by all prefixes, and 2 per prefix
-};
-
 // The search is expected to meet `cost` records, each some ten instructions
 // for one prefix; the walk skips what 64 neighbouring lanes can.  Where the
 // rows cut little (many columns per row, or odd sums, which are never zero)
@@ -283,31 +259,6 @@ struct TreePlan {
 // 0.080 / 0.174; n = 18, a 4x9 grid: 6.1, 0.013 / 0.076).
 constexpr double kTreeShare = 0.5, kTreeSmall = 1 << 24;
 
-// Lanes' prefixes in the first level: enough to hold the chip's waves and to
-// spread the surviving ones over them (8x10 grid: 2^18 1.1, 2^20 0.81, 2^22
-// 0.65-0.74, 2^24 0.83 ms; 8x9: 0.179, 0.184, 0.20, 0.38), and the columns
-// of the others (8x10: one 1.01, two 0.74, three 0.74 ms).
-int tree_top_bits(int b) { return std::min(b, std::max(18, std::min(24, b - 17))); }
-uint32_t tree_waves(int top_bits) { return top_bits >= 22 ? 8192u : 1u << std::min(12, top_bits - 6); }
-int tree_level_bits(int left) { return left <= 20 ? 2 : 3; }
-
-// Share of the subsets of the columns of values v at which start + sum is 0.
-double zero_share(double start, const std::vector<double>& v) {
-  constexpr size_t kMost = 256;  // (a row of many different sums: hardly ever)
-  std::map<double, double> at{{start, 1.0}};
-  for (double a : v) {
-    std::map<double, double> next;
-    for (const auto& e : at) {
-      next[e.first] += 0.5 * e.second;
-      next[e.first + a] += 0.5 * e.second;
-    }
-    at.swap(next);
-    if (at.size() > kMost) return 0.0;
-  }
-  const auto z = at.find(0.0);
-  return z == at.end() ? 0.0 : z->second;
-}
-
 // A walk's split or limits are set: the walk runs.
 bool walk_asked() {
   for (const char* v : {"PERMAN_WALK_BITS", "PERMAN_SKIP_CHECK_BITS", "PERMAN_SKIP_BUDGET",
@@ -316,85 +267,18 @@ bool walk_asked() {
   return false;
 }
 
-// x0 and cols as gathered (rows in the matrix's order).
-void plan_tree(int n, const std::vector<double>& x0, const std::vector<double>& cols,
-               const std::vector<int>& order, TreePlan& tp) {
-  const int B = n - 1;
-  struct Row {
-    int low = 0;  // lowest column with an entry: x is known from there on
-    double zero = 0.0;
-    std::vector<perm::SkipRecord> rec;
-  };
-  std::vector<Row> rows(n);
-  for (int j = 0; j < n; ++j) {
-    Row& r = rows[j];
-    r.low = B;
-    std::vector<double> v;
-    for (int c = B - 1; c >= 0; --c) {
-      const double a = cols[(size_t)order[c] * n + j];
-      if (a == 0.0) continue;
-      r.low = c;
-      v.push_back(a);
-      auto it = std::find_if(r.rec.begin(), r.rec.end(),
-                             [&](const perm::SkipRecord& e) { return e.value == a; });
-      if (it == r.rec.end()) it = r.rec.insert(r.rec.end(), {0, a, 0.0, 0});
-      it->mask |= 1ull << c;
-    }
-    if (r.rec.empty()) r.rec.push_back({0, 0.0, 0.0, 0});
-    r.rec.front().start = x0[j];
-    r.rec.back().last = 1;
-    r.zero = zero_share(x0[j], v);
-  }
-  std::stable_sort(rows.begin(), rows.end(),
-                   [](const Row& a, const Row& b) { return a.low > b.low; });
-  tp.top_bits = tree_top_bits(B);
-  tp.waves = tree_waves(tp.top_bits);
-  const int left = B - tp.top_bits, per = tree_level_bits(left);
-  std::vector<int> bits{tp.top_bits};
-  for (int d = left; d > 0;) {
-    const int b = d % per ? d % per : per;
-    bits.push_back(b);
-    d -= b;
-  }
-  int base = B;
-  size_t at = 0;
-  double prefixes = 1.0;
-  for (int b : bits) {
-    base -= b;
-    perm::SkipLevel lv{b, base, (uint32_t)tp.records.size(), 0};
-    prefixes *= std::ldexp(1.0, b);
-    tp.cost += 2.0 * prefixes;
-    for (; at < rows.size() && rows[at].low >= base; ++at) {
-      tp.cost += prefixes * (double)rows[at].rec.size();
-      prefixes *= 1.0 - rows[at].zero;
-      tp.records.insert(tp.records.end(), rows[at].rec.begin(), rows[at].rec.end());
-    }
-    lv.end = (uint32_t)tp.records.size();
-    tp.levels.push_back(lv);
-  }
-}
-
-int run_tree(int n, const TreePlan& tp, int mode, perm::Partial& r, double& walked_frac,
+int run_tree(int n, const perm::TreePlan& tp, int mode, perm::Partial& r, double& walked_frac,
              float& ms) {
-  const size_t lev_b = align256(tp.levels.size() * sizeof(perm::SkipLevel));
-  const size_t rec_b = align256(tp.records.size() * sizeof(perm::SkipRecord));
+  const std::vector<uint64_t> up = perm::pack_tree(tp);
+  const size_t up_b = align256(up.size() * sizeof(uint64_t));
   const size_t part_b = align256(tp.waves * sizeof(perm::Partial));
-  std::vector<char> up(lev_b + rec_b);
-  std::memcpy(up.data(), tp.levels.data(), tp.levels.size() * sizeof(perm::SkipLevel));
-  std::memcpy(up.data() + lev_b, tp.records.data(), tp.records.size() * sizeof(perm::SkipRecord));
   perm::CachedRun run;
   const int st = perm::run_cached(
-      up.data(), up.size(), up.size() + part_b + 256,
+      up.data(), up.size() * sizeof(uint64_t), up_b + part_b + 256,
       [&](char* d, hipStream_t stream, const perm::RunReport& report) {
-        perm::SkipTreeLaunch L{};
-        L.levels = (const perm::SkipLevel*)d;
-        L.records = (const perm::SkipRecord*)(d + lev_b);
-        L.partials = (perm::Partial*)(d + lev_b + rec_b);
-        L.result = (perm::Partial*)(d + lev_b + rec_b + part_b);
-        L.n_levels = (int)tp.levels.size();
-        L.top_bits = tp.top_bits;
-        L.mode = mode;
-        L.waves = tp.waves;
+        perm::SkipTreeLaunch L = perm::tree_launch(tp, d, mode);
+        L.partials = (perm::Partial*)(d + up_b);
+        L.result = (perm::Partial*)(d + up_b + part_b);
         L.begin_tick = report.begin;
         return perm::launch_skip_tree(L, stream, report);
       },
@@ -461,11 +345,14 @@ int perm_skip(int dtype, const void* mat, const int* rptrs, const int* cols, con
   // 8x9, 8x10, 6x12 against 2^4..2^6
   int check_bits = perm::env_int("PERMAN_SKIP_CHECK_BITS", 3);
   check_bits = std::max(R, std::min(check_bits, sp.walk_bits));
-  TreePlan tp;
+  perm::TreePlan tp;
   bool tree = !walk_asked();
   if (tree) {
-    plan_tree(nov, x0, cc, sp.order, tp);
-    tree = tp.cost <= std::max(kTreeSmall, kTreeShare * std::ldexp(1.0, nov - 1));
+    const double limit = std::max(kTreeSmall, kTreeShare * std::ldexp(1.0, nov - 1));
+    double zero[64];
+    perm::nonzero_share(nov, x0.data(), cc.data(), zero);
+    perm::plan_tree(nov, x0.data(), cc.data(), sp.order.data(), zero, tp);
+    tree = tp.cost <= limit;
   }
   const auto run = [&](int mode, perm::Partial& r, double& walked, float& ms) {
     return tree ? run_tree(nov, tp, mode, r, walked, ms)

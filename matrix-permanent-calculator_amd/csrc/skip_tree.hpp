@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <vector>
+
 namespace perm {
 
 struct Partial;
@@ -31,7 +33,7 @@ constexpr int kSkipMaxTopBits = 26;
 constexpr int kSkipLevelRoom = 32 + 64;
 
 struct SkipTreeLaunch {
-  const SkipRecord* records;  // device
+  const SkipRecord* records;  // device, 32-byte aligned
   const SkipLevel* levels;    // device: n_levels, columns from the top down to 0
   Partial* partials;          // device: `waves` records
   Partial* result;            // device: 1 record
@@ -42,5 +44,32 @@ struct SkipTreeLaunch {
 // Enqueue the search and the grid reduction, which reports.  pad of the sum:
 // subsets of all columns formed (the rest was cut off).
 hipError_t launch_skip_tree(const SkipTreeLaunch& L, hipStream_t stream, const RunReport& report);
+
+// The search's plan (host; perman_skip_plan.cpp).
+struct TreePlan {
+  std::vector<SkipLevel> levels;
+  std::vector<SkipRecord> records;
+  int top_bits = 0;
+  uint32_t waves = 0;
+  double cost = 0.0;  // records expected to be met by all prefixes, and 2 per prefix
+};
+// Greedy order of b columns, the lowest first: next, the column adding the
+// fewest rows not yet touched (ties by fewer nonzeros, then index).  sup[k]:
+// rows with an entry in column k.
+void skip_order(int b, const uint64_t* sup, int* order);
+// x0: n start values; cols[k * n + j] = a[j][k], k < n - 1; an integer matrix.
+// zero[j]: share of the subsets at which row j is zero.  Returns the share of
+// the subsets at which no row is, the rows taken as independent.
+double nonzero_share(int n, const double* x0, const double* cols, double* zero);
+// order: of the walked columns (skip_order); n >= 7.
+void plan_tree(int n, const double* x0, const double* cols, const int* order, const double* zero,
+               TreePlan& tp);
+// Levels and records as the device reads them (32-byte aligned there).
+inline size_t tree_record_word(const TreePlan& tp) {
+  return (tp.levels.size() * sizeof(SkipLevel) + 31) / 32 * 4;
+}
+std::vector<uint64_t> pack_tree(const TreePlan& tp);
+// The launch's plan part; records, result and tick are the caller's.
+SkipTreeLaunch tree_launch(const TreePlan& tp, const void* packed, int mode);
 
 }  // namespace perm

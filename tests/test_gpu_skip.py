@@ -111,3 +111,24 @@ def test_search_vs_walk_at_larger_orders(monkeypatch, n, density):
     assert r.main_subsets <= w.main_subsets
     assert r.value == w.value or abs(r.value - w.value) <= r.stated + w.stated
     assert [P.skip(a).value for _ in range(3)] == [r.value] * 3
+
+
+@pytest.mark.parametrize("n,density", [(28, 0.15), (29, 0.12), (30, 0.2), (31, 0.3), (33, 0.12),
+                                       (34, 0.2)])
+def test_plain_calls_of_sparse_integer_matrices(monkeypatch, n, density):
+    """The dense, sparse and plan calls search where that is the faster pass
+    (in one mode, both or none of them); the Gray walk in the columns' own
+    order (PERMAN_PAIR=0) and the sum over block ranges never do."""
+    a = P.synthetic_matrix(n, density, 3 * n, binary=True, full_support=True).astype(np.int32)
+    calls = [P.dense(a), P.sparse(a)]
+    plan = P.Plan(a)
+    calls += [plan.run(), plan.run(mode=0), plan.run(mode=1), plan.run()]
+    plan.close()
+    with monkeypatch.context() as m:
+        m.setenv("PERMAN_PAIR", "0")
+        want = P.dense(a)
+    for r in calls:
+        assert abs(r.value - want.value) <= r.stated + want.stated, (n, density, r, want)
+        if r.zero_pattern == want.zero_pattern:  # (no walk, no sum of |terms|)
+            assert abs(r.abs_sum - want.abs_sum) <= 1e-12 * want.abs_sum
+    assert calls[2].value == calls[5].value == calls[0].value
