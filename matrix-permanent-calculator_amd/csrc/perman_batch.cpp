@@ -17,13 +17,16 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <chrono>
 #include <cstdio>
 #include <cmath>
 #include <cstring>
+#include <memory>
 #include <mutex>
 #include <string>
 #include <thread>
+#include <utility>
 #include <vector>
 
 #include "../../include/perman_hip.h"
@@ -60,15 +63,98 @@ struct Entry {
   uint32_t first_item = 0, item_count = 0;
 };
 
+// resize() leaves new elements as they are: the data buffer's pages are first
+// touched by the threads that fill them.
+template <class T>
+struct RawAllocator : std::allocator<T> {
+  template <class U>
+  struct rebind {
+    using other = RawAllocator<U>;
+  };
+  template <class U>
+  void construct(U*) {}
+  template <class U, class... A>
+  void construct(U* p, A&&... a) {
+    ::new ((void*)p) U(std::forward<A>(a)...);
+  }
+};
+
+// A batch's streams and events.
+struct BatchStreams {
+  hipStream_t s[kMaxStreams] = {};
+  hipEvent_t ev_fork = nullptr, ev_join[kMaxStreams] = {}, ev0 = nullptr, ev1 = nullptr;
+
+  hipError_t create() {
+    hipError_t e = hipSuccess;
+    for (int i = 0; i < kMaxStreams && e == hipSuccess; ++i)
+      e = hipStreamCreateWithFlags(&s[i], hipStreamNonBlocking);
+    if (e == hipSuccess) e = hipEventCreateWithFlags(&ev_fork, hipEventDisableTiming);
+    for (int i = 0; i < kMaxStreams && e == hipSuccess; ++i)
+      e = hipEventCreateWithFlags(&ev_join[i], hipEventDisableTiming);
+    if (e == hipSuccess) e = hipEventCreate(&ev0);
+    if (e == hipSuccess) e = hipEventCreate(&ev1);
+    return e;
+  }
+  // True if every stream ended its work without an error.
+  bool idle() {
+    bool ok = true;
+    for (hipStream_t q : s)
+      if (q) ok = hipStreamSynchronize(q) == hipSuccess && ok;
+    return ok;
+  }
+  void destroy() {
+    for (int i = 0; i < kMaxStreams; ++i) {
+      if (s[i]) (void)hipStreamDestroy(s[i]);
+      if (ev_join[i]) (void)hipEventDestroy(ev_join[i]);
+    }
+    if (ev_fork) (void)hipEventDestroy(ev_fork);
+    if (ev0) (void)hipEventDestroy(ev0);
+    if (ev1) (void)hipEventDestroy(ev1);
+    *this = BatchStreams{};
+  }
+};
+
+// Streams of destroyed batches for the next ones, at most kKeptStreams sets
+// per device (idle; kept until the process ends): creating and destroying a
+// set takes 0.35 ms, a tenth of a batch of 512 matrices of n = 12..27.
+constexpr size_t kKeptStreams = 4;
+struct StreamPool {
+  std::mutex mu;
+  std::vector<std::pair<int, BatchStreams>> kept;  // (device, set)
+
+  bool take(int device, BatchStreams& out) {
+    std::lock_guard<std::mutex> g(mu);
+    for (size_t i = 0; i < kept.size(); ++i)
+      if (kept[i].first == device) {
+        out = kept[i].second;
+        kept.erase(kept.begin() + (long)i);
+        return true;
+      }
+    return false;
+  }
+  bool give(int device, const BatchStreams& set) {
+    std::lock_guard<std::mutex> g(mu);
+    size_t have = 0;
+    for (const auto& k : kept) have += k.first == device;
+    if (have >= kKeptStreams) return false;
+    kept.emplace_back(device, set);
+    return true;
+  }
+};
+StreamPool& stream_pool() {
+  static StreamPool* pool = new StreamPool();  // (batches may outlive statics)
+  return *pool;
+}
+
 }  // namespace
 
-struct perm_batch {
+struct perm_batch : BatchStreams {
   int device = 0;
   int item_log2 = 17;   // subsets per item (64 lanes x 2^(item_log2-6) steps)
   int streams = 8;
   int max_grid = 1024;  // workgroups per variant kernel
   uint32_t max_grid_u() const { return (uint32_t)max_grid; }
-  std::vector<double> data;
+  std::vector<double, RawAllocator<double>> data;
   std::vector<Entry> ents;
   std::vector<BatchItem> items;
   struct Group {
@@ -90,8 +176,6 @@ struct perm_batch {
   Partial* d_results = nullptr;
   uint32_t* d_counters = nullptr;
   Partial* h_results = nullptr;  // pinned
-  hipStream_t s[kMaxStreams] = {};
-  hipEvent_t ev_fork = nullptr, ev_join[kMaxStreams] = {}, ev0 = nullptr, ev1 = nullptr;
   hipGraphExec_t graph = nullptr;
   bool built = false;
   bool ran = false;  // one direct run since the build: the next run captures the graph
@@ -120,9 +204,18 @@ void release_device(perm_batch* B) {
 }
 
 
-// Fill entry e from the prepared matrix and append its column store and
-// start vector to B->data.
-int fill_entry(perm_batch* B, Entry& e, int n, perm::Prepared& p) {
+// Room of an entry's column store, start vector and class tables in the data
+// buffer: whole 256-byte lines, so the next entry's are aligned.
+size_t entry_room(size_t store, size_t tables) {
+  return ((store + 7) / 8 * 8 + tables + 31) / 32 * 32;  // (records are 64 bytes)
+}
+size_t entry_room(const perm::Prepared& p) {
+  return entry_room(p.cs.size() + p.x0.size(), p.classed ? p.tables.data.size() : 0);
+}
+
+// Fill entry e from the prepared matrix and write its entry_room(p) doubles
+// at data + at.
+int fill_entry(Entry& e, int n, const perm::Prepared& p, double* data, size_t at) {
   if (n > perm::kMaxBatchN)
     return perm::fail(PERM_ERR_SIZE, "batch matrices are limited to n <= " +
                                          std::to_string(perm::kMaxBatchN));
@@ -137,27 +230,36 @@ int fill_entry(perm_batch* B, Entry& e, int n, perm::Prepared& p) {
                                   p.nu2 > 0 ? p.nu2 : n});
   e.variant = perm::batch_variant(n, e.shape);
   if (e.variant < 0) return perm::fail(PERM_ERR_ARG, "no batch kernel for this n");
-  e.col_off = B->data.size();
-  B->data.insert(B->data.end(), p.cs.begin(), p.cs.end());
-  e.x0_off = B->data.size();
-  B->data.insert(B->data.end(), p.x0.begin(), p.x0.end());
+  const size_t end = at + entry_room(p);
+  auto put = [&](const std::vector<double>& v) {
+    const size_t off = at;
+    std::copy(v.begin(), v.end(), data + at);
+    at += v.size();
+    return off;
+  };
+  e.col_off = put(p.cs);
+  e.x0_off = put(p.x0);
   e.classed = p.classed;
   if (p.classed) {
     e.live = p.plan.live;
     e.thin = p.plan.thin;
     e.cost = p.plan.cost;
-    while (B->data.size() % 8) B->data.push_back(0.0);  // records are 64 bytes
-    e.rec_off = B->data.size();
+    while (at % 8) data[at++] = 0.0;
+    e.rec_off = put(p.tables.data);
     e.ccol_off = e.rec_off + p.tables.cols;
-    B->data.insert(B->data.end(), p.tables.data.begin(), p.tables.data.end());
   }
-  while (B->data.size() % 32) B->data.push_back(0.0);  // 256-B alignment of the next store
+  std::fill(data + at, data + end, 0.0);
   return PERM_OK;
 }
 
 int add_prepared(perm_batch* B, int n, perm::Prepared& p, int* index) {
   Entry e;
-  if (int st = fill_entry(B, e, n, p)) return st;
+  const size_t at = B->data.size();
+  B->data.resize(at + entry_room(p));
+  if (int st = fill_entry(e, n, p, B->data.data(), at)) {
+    B->data.resize(at);
+    return st;
+  }
   // (after perm_batch_compute_dense the entries are in processing order;
   // a matrix added later keeps the caller's insertion index)
   if (!B->caller.empty()) B->caller.push_back((uint32_t)B->ents.size());
@@ -816,14 +918,8 @@ int perm_batch_create(perm_batch** out) {
   if (int s = perm::select_device()) return s;
   auto* B = new perm_batch();
   B->device = perm::current_device();
-  hipError_t e = hipSuccess;
-  for (int i = 0; i < kMaxStreams && e == hipSuccess; ++i)
-    e = hipStreamCreateWithFlags(&B->s[i], hipStreamNonBlocking);
-  if (e == hipSuccess) e = hipEventCreateWithFlags(&B->ev_fork, hipEventDisableTiming);
-  for (int i = 0; i < kMaxStreams && e == hipSuccess; ++i)
-    e = hipEventCreateWithFlags(&B->ev_join[i], hipEventDisableTiming);
-  if (e == hipSuccess) e = hipEventCreate(&B->ev0);
-  if (e == hipSuccess) e = hipEventCreate(&B->ev1);
+  const hipError_t e =
+      stream_pool().take(B->device, *B) ? hipSuccess : B->BatchStreams::create();
   if (e != hipSuccess) {
     perm_batch_destroy(B);
     return perm::fail(PERM_ERR_HIP, std::string("batch streams: ") + hipGetErrorString(e));
@@ -963,23 +1059,26 @@ int perm_batch_compute_dense(perm_batch* B, int count, const int* dtypes,
   }
   // device memory from the orders alone (upper bounds: column store, start
   // vector and padding per matrix; every matrix's items)
-  size_t data_ub = 0, items_ub = 0, split_ub = 0;
-  for (int i = 0; i < count; ++i) {
+  size_t items_ub = 0, split_ub = 0;
+  std::vector<size_t> place((size_t)count + 1, 0);  // of matrix order[k] in the data buffer
+  for (int k = 0; k < count; ++k) {
+    const uint32_t i = order[(size_t)k];
     const size_t n = (size_t)novs[i];
-    data_ub += (2 * n - 1) * n + 2 * n + 32;
+    size_t tables = 0;
     int w = 0, h = 0;
     perm::batch_split(novs[i], B->item_log2, w, h);
     items_ub += ((1ull << h) + perm::kItemLanes - 1) / perm::kItemLanes;
     if (novs[i] >= perm::kMinBatchClassN && class_split_ok(w)) {
-      data_ub += perm::class_tables_bound(novs[i]) + 8;
+      tables = perm::class_tables_bound(novs[i]);
       split_ub += perm::class_split_doubles(novs[i], w - perm::kClassBits) + 8;
     }
+    place[(size_t)k + 1] = place[(size_t)k] + entry_room((2 * n - 1) * n + 2 * n, tables);
   }
+  const size_t data_ub = place[(size_t)count];
   if (items_ub > 0xffffffffull) return perm::fail(PERM_ERR_SIZE, "too many items");
   B->ents.assign((size_t)count, Entry{});
   B->caller.assign(order.begin(), order.end());
-  B->data.clear();
-  B->data.reserve(data_ub);  // no reallocation: the phase uploads read from it
+  B->data.resize(data_ub);
   B->items.clear();
   B->items.reserve(items_ub);
   B->groups.clear();
@@ -1007,43 +1106,69 @@ int perm_batch_compute_dense(perm_batch* B, int count, const int* dtypes,
   std::vector<double> stream_work((size_t)ke, 0.0);
   HIP_TRYB(hipEventRecord(B->ev0, s0));
   HIP_TRYB(perm::launch_batch_reset(B->d_counters, (uint32_t)(3 * count), s0));
-  std::vector<perm::Prepared> prep((size_t)count);
   std::vector<int> status((size_t)count, PERM_OK);
   std::vector<std::string> msg((size_t)count);
   std::vector<BatchMatrix> dm((size_t)count);
   std::vector<perm::ClassMatrix> dc((size_t)count);
   size_t split = 0;
   const size_t phases[4] = {0, cut[0], std::max(cut[0], cut[1]), (size_t)count};
+  // `threads` host threads (this one among them) prepare the matrices in
+  // processing order, each straight into its place in the data buffer; a
+  // phase is planned, uploaded and launched here as soon as its last matrix
+  // is ready, while the others go on with the next phase.  (512 matrices,
+  // n = 12..27, 16 threads: threads started per phase and entries copied by
+  // this thread, the last launch was out at 2.1-2.4 ms and the device, 2.4 ms
+  // of work, waited 0.5 ms for it.)
+  std::atomic<size_t> next{0}, ready[3] = {{0}, {0}, {0}};
+  std::atomic<bool> stop{false};
+  auto prepare_one = [&](size_t k) {
+    perm::Prepared p;
+    const uint32_t i = order[k];
+    int st = perm::prepare_dense(dtypes[i], mats[i], novs[i], p, perm::kMenuBatch);
+    if (st == PERM_OK && entry_room(p) > place[k + 1] - place[k])
+      st = perm::fail(PERM_ERR_SIZE, "batch data bound");
+    if (st == PERM_OK) st = fill_entry(B->ents[k], novs[i], p, B->data.data(), place[k]);
+    status[k] = st;
+    if (st != PERM_OK) msg[k] = perm::last_error();
+    ready[k < phases[1] ? 0 : k < phases[2] ? 1 : 2].fetch_add(1, std::memory_order_release);
+  };
+  struct Workers {
+    std::vector<std::thread> pool;
+    std::atomic<bool>& stop;
+    ~Workers() {
+      stop = true;
+      for (auto& th : pool) th.join();
+    }
+  } workers{{}, stop};
+  for (int t = 1; t < threads; ++t)
+    workers.pool.emplace_back([&] {
+      while (!stop) {
+        const size_t k = next.fetch_add(1);
+        if (k >= (size_t)count) break;
+        prepare_one(k);
+      }
+    });
   for (int ph = 0; ph < 3; ++ph) {
     const size_t p0 = phases[ph], p1 = phases[ph + 1];
     if (p0 == p1) continue;
-    // prepare the phase's matrices on `threads` host threads (the first
-    // phase's kernels run meanwhile)
-    {
-      const int t_n = std::max(1, std::min<int>(threads, (int)(p1 - p0)));
-      std::vector<std::thread> pool;
-      for (int t = 0; t < t_n; ++t)
-        pool.emplace_back([&, t] {
-          for (size_t k = p0 + (size_t)t; k < p1; k += (size_t)t_n) {
-            const uint32_t i = order[k];
-            status[k] = perm::prepare_dense(dtypes[i], mats[i], novs[i], prep[k], perm::kMenuBatch);
-            if (status[k] != PERM_OK) msg[k] = perm::last_error();
-          }
-        });
-      for (auto& th : pool) th.join();
+    while (ready[ph].load(std::memory_order_acquire) < p1 - p0) {
+      size_t k = next.load();
+      if (k >= p1)
+        std::this_thread::yield();  // the others have the rest of the phase
+      else if (next.compare_exchange_strong(k, k + 1))
+        prepare_one(k);
     }
     mark(ph == 0 ? "phase 0 prepared" : ph == 1 ? "phase 1 prepared" : "phase 2 prepared");
     for (size_t k = p0; k < p1; ++k)
-      if (status[k] != PERM_OK)
+      if (status[k] != PERM_OK) {
+        stop = true;
+        for (auto& th : workers.pool) th.join();
+        workers.pool.clear();
         return undo(perm::fail(status[k], "matrix " + std::to_string(order[k]) + ": " + msg[k]));
-    const size_t d0 = B->data.size(), i0 = B->items.size(), g0 = B->groups.size();
+      }
+    const size_t d0 = place[p0], d1 = place[p1], i0 = B->items.size(), g0 = B->groups.size();
     std::vector<uint32_t> idx;
-    for (size_t k = p0; k < p1; ++k) {
-      if (int st = fill_entry(B, B->ents[k], novs[order[k]], prep[k])) return undo(st);
-      prep[k] = perm::Prepared();
-      idx.push_back((uint32_t)k);
-    }
-    if (B->data.size() > data_ub) return undo(perm::fail(PERM_ERR_SIZE, "batch data bound"));
+    for (size_t k = p0; k < p1; ++k) idx.push_back((uint32_t)k);
     plan_items(B, idx);
     for (size_t k = p0; k < p1; ++k) {
       split = place_split(B->ents[k], split);
@@ -1053,7 +1178,7 @@ int perm_batch_compute_dense(perm_batch* B, int count, const int* dtypes,
     mark("planned");
     // this phase's data, matrices and items, then its variant kernels
     HIP_TRYB(hipMemcpyAsync(B->d_data + d0, B->data.data() + d0,
-                            (B->data.size() - d0) * sizeof(double), hipMemcpyHostToDevice, s0));
+                            (d1 - d0) * sizeof(double), hipMemcpyHostToDevice, s0));
     HIP_TRYB(hipMemcpyAsync(B->d_mats + p0, dm.data() + p0, (p1 - p0) * sizeof(BatchMatrix),
                             hipMemcpyHostToDevice, s0));
     if (B->items.size() > i0)
@@ -1174,16 +1299,9 @@ int perm_batch_get(const perm_batch* B, perm_batch_tuning* out) {
 void perm_batch_destroy(perm_batch* B) {
   if (!B) return;
   (void)hipSetDevice(B->device);
-  for (int i = 0; i < kMaxStreams; ++i)
-    if (B->s[i]) (void)hipStreamSynchronize(B->s[i]);
+  const bool idle = B->idle();
   release_device(B);
-  for (int i = 0; i < kMaxStreams; ++i) {
-    if (B->s[i]) (void)hipStreamDestroy(B->s[i]);
-    if (B->ev_join[i]) (void)hipEventDestroy(B->ev_join[i]);
-  }
-  if (B->ev_fork) (void)hipEventDestroy(B->ev_fork);
-  if (B->ev0) (void)hipEventDestroy(B->ev0);
-  if (B->ev1) (void)hipEventDestroy(B->ev1);
+  if (!idle || !B->ev1 || !stream_pool().give(B->device, *B)) B->BatchStreams::destroy();
   delete B;
 }
 
