@@ -432,16 +432,16 @@ static bool class_range(int n, const std::vector<double>& x0, const std::vector<
 
 // The search of the subsets without a zero row takes the passes of a sparse
 // integer matrix where it is expected to be the faster one: a record it meets
-// costs as much as some 95 FP64 instructions of the class walk (3.2e-12 against
+// costs as much as some 60 FP64 instructions of the class walk (2e-12 against
 // 3.4e-14 s) or rows of a subset with double-double products in the Gray walk
-// (3.8e-12 against 3.9e-14 s), half as much again left for the estimate's
+// (2.4e-12 against 3.9e-14 s), half as much again left for the estimate's
 // error (the rows' zeros are taken as independent).  Whole calls, 0/1
-// matrices, without / with it: n = 30, density 0.1 0.31 / 0.15 ms; n = 33,
-// 0.1 1.27 / 0.17; 0.18 (both passes) 7.0 / 0.58; n = 36, 0.1 9.6 / 0.35;
-// 0.14 (both) 55 / 5.8.  At n = 27 the walk's kernel takes 0.05 ms: nothing
+// matrices, without / with it: n = 30, density 0.1 0.31 / 0.14 ms; n = 33,
+// 0.1 1.27 / 0.20; 0.18 (both passes) 7.0 / 0.48; n = 36, 0.1 9.6 / 0.32;
+// 0.14 (both) 55 / 2.8.  At n = 27 the walk's kernel takes 0.05 ms: nothing
 // to gain over the plan's own time.
 constexpr int kMinTreeN = 29;
-constexpr double kTreeRecord = 145.0;
+constexpr double kTreeRecord = 95.0;
 
 static void prepare_tree(int n, const uint64_t* sup, const std::vector<double>& cols,
                          Prepared& p) {
@@ -458,7 +458,7 @@ static void prepare_tree(int n, const uint64_t* sup, const std::vector<double>& 
   p.tree_modes = (p.tree.cost <= walk ? 1u : 0u) | (p.tree.cost <= dd ? 2u : 0u);
   if (!p.tree_modes) return;
   std::vector<double>& t = p.tables.data;
-  while (t.size() % 4) t.push_back(0.0);
+  while (t.size() % 8) t.push_back(0.0);
   p.tree_off = t.size();
   const std::vector<uint64_t> packed = pack_tree(p.tree);
   t.resize(p.tree_off + packed.size());

@@ -248,16 +248,15 @@ int run_skip(int n, const SkipPrepared& sp, int mode, int check_bits, perm::Part
   return PERM_OK;
 }
 
-// The search is expected to meet `cost` records, each some ten instructions
+// The search is expected to meet `cost` records, each some eight instructions
 // for one prefix; the walk skips what 64 neighbouring lanes can.  Where the
 // rows cut little (many columns per row, or odd sums, which are never zero)
-// the walk's 2n instructions per subset are fewer.  Kernel times, 0/1
-// matrices, search / walk: cost 0.24 2^(n-1) (n = 30, density 0.25) 0.87 /
-// 3.17 ms; 0.43 (n = 33, 0.35) 5.6 / 8.0; 0.53 (n = 30, 0.4) 0.82 / 0.86;
-// 1.6 (n = 28, 0.4) 0.46 / 0.31; 3.4 (n = 30, 0.5) 3.3 / 1.2.  Up to some
-// 2^24 records the search is the shorter one anyway (n = 25, 0.5: cost 1.5,
-// 0.080 / 0.174; n = 18, a 4x9 grid: 6.1, 0.013 / 0.076).
-constexpr double kTreeShare = 0.5, kTreeSmall = 1 << 24;
+// the walk's 2n instructions per subset are fewer.  Kernel ms, 0/1 matrices,
+// search / walk: cost 0.53 2^(n-1) (n = 30, density 0.4) 0.45 / 0.86; 0.82
+// (28, 0.35) 0.15 / 0.32; 1.6 (28, 0.4) 0.24 / 0.31; 2.5 (28, 0.5) 0.36 /
+// 0.31; 3.4 (30, 0.5) 1.49 / 1.17.  Up to some 2^24 records the search is the
+// shorter one anyway (n = 18, a 4x9 grid: cost 6.1, 0.011 / 0.076).
+constexpr double kTreeShare = 1.5, kTreeSmall = 1 << 24;
 
 // A walk's split or limits are set: the walk runs.
 bool walk_asked() {

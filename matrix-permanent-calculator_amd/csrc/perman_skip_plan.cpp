@@ -30,12 +30,15 @@ void skip_order(int b, const uint64_t* sup, int* order) {
 
 namespace {
 
-// Lanes' prefixes in the first level: enough to hold the chip's waves and to
-// spread the surviving ones over them (8x10 grid: 2^18 1.1, 2^20 0.81, 2^22
-// 0.65-0.74, 2^24 0.83 ms; 8x9: 0.179, 0.184, 0.20, 0.38), and the columns
-// of the others (8x10: one 1.01, two 0.74, three 0.74 ms).
-int tree_top_bits(int b) { return std::min(b, std::max(18, std::min(24, b - 17))); }
-uint32_t tree_waves(int top_bits) { return top_bits >= 22 ? 8192u : 1u << std::min(12, top_bits - 6); }
+// Columns of the first level: enough of its prefixes survive to hold the
+// chip's waves and to spread evenly over them, and the numbers themselves stay
+// cheap; and the waves.  Kernel ms at 18, 20, 22, 23 columns with 8192 waves:
+// grid 7x10 (n = 35) 0.177, 0.111, 0.109, 0.138; 8x9 0.132, 0.123, 0.123,
+// 0.139; 8x10 0.76, 0.55, 0.48, 0.41; 8x8 with 4096 waves 0.033, 0.032, 0.046,
+// 0.067.  The other levels: one column each 1.01, two 0.74, three 0.74 ms
+// (8x10, an earlier form of the kernel).
+int tree_top_bits(int b) { return std::min(b, std::max(18, std::min(23, b - 14))); }
+uint32_t tree_waves(int top_bits) { return top_bits >= 20 ? 8192u : 1u << std::min(12, top_bits - 6); }
 int tree_level_bits(int left) { return left <= 20 ? 2 : 3; }
 
 // Share of the subsets of the columns of values v[0, d) at which start + sum
@@ -100,6 +103,7 @@ void plan_tree(int n, const double* x0, const double* cols, const int* order, co
   tp.levels.clear();
   tp.records.clear();
   tp.cost = 0.0;
+  tp.single = true;
   double prefixes = 1.0;
   int at = 0;
   for (int base = B; base > 0;) {
@@ -122,9 +126,11 @@ void plan_tree(int n, const double* x0, const double* cols, const int* order, co
       if (tp.records.size() == first) tp.records.push_back({0, 0.0, 0.0, 0});
       tp.records[first].start = x0[j];
       tp.records.back().last = 1;
+      tp.single = tp.single && tp.records.size() == first + 1;
       tp.cost += prefixes * (double)(tp.records.size() - first);
       prefixes *= 1.0 - rows[at].zero;
     }
+    while (tp.records.size() % kSkipRecordStep) tp.records.push_back({0, 0.0, 1.0, 1});
     lv.end = (uint32_t)tp.records.size();
     tp.levels.push_back(lv);
   }
@@ -146,6 +152,7 @@ SkipTreeLaunch tree_launch(const TreePlan& tp, const void* packed, int mode) {
   L.top_bits = tp.top_bits;
   L.mode = mode;
   L.waves = tp.waves;
+  L.single = tp.single;
   return L;
 }
 

@@ -27,21 +27,24 @@
 //
 // The order of all sums is fixed by the launch: the same result every time.
 //
-// Bound: the latency of a step (level, records and stack are read one after
-// the other), 40 to 100 of them per wave at 11 waves per compute unit (LDS);
-// the first level's 2^18..2^24 numbers are 10 to 40 us of it.  Kernel times,
-// walk -> search: grid 8x10 (4 % of the bonds missing, n = 40) 6.05 -> 0.67
-// ms, 8x10 2.95 -> 0.29, 8x9 1.48 -> 0.18, 8x8 0.29 -> 0.040; random 0/1
-// n = 30, density 0.15 0.57 -> 0.086, n = 33, 0.2 9.6 -> 2.1 ms (two passes).
+// Bound: the latency of a step (stack, then four records at a time as scalar
+// loads) at eleven waves per compute unit (their stacks fill the LDS), 40 to
+// 100 steps per wave; the first level's 2^18..2^23 numbers are 5 to 30 us of
+// it.  Records one by one, with the level's description loaded in each step
+// and a test of every row, took 1.4 times as long.  Kernel times, walk ->
+// search: grid 8x10 (4 % of the bonds missing, n = 40) 6.05 -> 0.41 ms, 8x10
+// 2.95 -> 0.20, 8x9 1.48 -> 0.12, 8x8 0.29 -> 0.032, 8x12 (n = 48, two passes)
+// 233 -> 6.2; random 0/1 n = 30, density 0.1 0.28 -> 0.031, n = 33, 0.18 (two
+// passes) 9.6 -> 0.33 ms.
 #include "ryser_device.hpp"
 #include "ryser_kernels.hpp"
 #include "skip_tree.hpp"
 
 namespace perm {
 
-typedef uint64_t Word4 __attribute__((ext_vector_type(4)));
-typedef const Word4 __attribute__((address_space(4)))* RecordPtr;
-typedef const SkipLevel __attribute__((address_space(4)))* LevelPtr;
+// Four records as two scalar loads.
+typedef uint64_t Word8 __attribute__((ext_vector_type(8)));
+typedef const Word8 __attribute__((address_space(4)))* RecordPtr;
 
 template <bool DDP>
 struct Prefix {
@@ -61,38 +64,47 @@ __device__ __forceinline__ uint32_t scatter(uint32_t v, int bits) {
   return v ^ v >> half;
 }
 
-// Multiply the rows of records [begin, end) into p; false: one of them is
-// zero.  Stops when that is so in every lane.
-template <bool DDP>
+// Multiply the rows of records [begin, end) (a multiple of four) into p; false:
+// one of them is zero (the product is: no x is below 1/2 otherwise, so 63 of
+// them do not underflow).  Stops when that is so in every lane.  SINGLE: every
+// row is one record.
+template <bool DDP, bool SINGLE>
 __device__ __forceinline__ bool complete_rows(Prefix<DDP>& p, RecordPtr records, uint32_t begin,
-                                              uint32_t end, bool alive) {
+                                              uint32_t end) {
+  static_assert(kSkipRecordStep == 4);
   double x = 0.0;
-  Word4 r = begin < end ? records[begin] : Word4{0, 0, 0, 0};
-  for (uint32_t i = begin; i < end; ++i) {
-    const Word4 next = records[i + 1 < end ? i + 1 : i];
-    x += __builtin_bit_cast(double, (uint64_t)r[2]);
-    x = __builtin_fma(__builtin_bit_cast(double, (uint64_t)r[1]),
-                      (double)__builtin_popcountll(p.set & r[0]), x);
-    if (r[3]) {
-      alive = alive && x != 0.0;
-      const double h = p.prod * x;
-      if constexpr (DDP) {
-        const double e = __builtin_fma(p.tail, x, __builtin_fma(p.prod, x, -h));
-        const DD n = quick_two_sum(h, e);
-        p.prod = n.hi;
-        p.tail = n.lo;
-      } else {
-        p.prod = h;
+  for (uint32_t i = begin; i < end; i += 4) {
+    const Word8 r[2] = {records[i / 2], records[i / 2 + 1]};
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const uint64_t mask = r[k / 2][4 * (k % 2)];
+      const double value = __builtin_bit_cast(double, (uint64_t)r[k / 2][4 * (k % 2) + 1]);
+      const double start = __builtin_bit_cast(double, (uint64_t)r[k / 2][4 * (k % 2) + 2]);
+      const uint64_t set = p.set & mask;
+      const int count = __builtin_popcount((uint32_t)set) + __builtin_popcount((uint32_t)(set >> 32));
+      if constexpr (SINGLE)
+        x = __builtin_fma(value, (double)count, start);
+      else
+        x = __builtin_fma(value, (double)count, x + start);
+      if (SINGLE || r[k / 2][4 * (k % 2) + 3]) {
+        const double h = p.prod * x;
+        if constexpr (DDP) {
+          const double e = __builtin_fma(p.tail, x, __builtin_fma(p.prod, x, -h));
+          const DD n = quick_two_sum(h, e);
+          p.prod = n.hi;
+          p.tail = n.lo;
+        } else {
+          p.prod = h;
+        }
+        x = 0.0;
       }
-      x = 0.0;
-      if (__builtin_amdgcn_ballot_w64(alive) == 0) return false;
     }
-    r = next;
+    if (__builtin_amdgcn_ballot_w64(p.prod != 0.0) == 0) return false;
   }
-  return alive;
+  return p.prod != 0.0;
 }
 
-template <bool DDP>
+template <bool DDP, bool SINGLE>
 __global__ __launch_bounds__(kWave)
 void ryser_skip_tree_kernel(const SkipRecord* __restrict__ records_arg,
                             const SkipLevel* __restrict__ levels_arg, int n_levels, int top_bits,
@@ -103,8 +115,10 @@ void ryser_skip_tree_kernel(const SkipRecord* __restrict__ records_arg,
   if (begin_tick && blockIdx.x == 0 && threadIdx.x == 0)
     *begin_tick = __builtin_amdgcn_s_memrealtime();
   const RecordPtr records = (RecordPtr)records_arg;
-  const LevelPtr levels = (LevelPtr)levels_arg;
   const uint32_t lane = threadIdx.x;
+  // lane l holds level l
+  const SkipLevel mine = levels_arg[lane < (uint32_t)n_levels ? lane : 0u];
+  auto of_level = [](int v, int l) { return __builtin_amdgcn_readlane(v, l); };
   constexpr uint32_t kWords = DDP ? 3 : 2;
   // stack of level l >= 1: sets, products(, tails), kSkipLevelRoom each
   auto stack = [&](int l) { return lds + (uint32_t)(l - 1) * kWords * kSkipLevelRoom; };
@@ -118,9 +132,10 @@ void ryser_skip_tree_kernel(const SkipRecord* __restrict__ records_arg,
   double formed = 0.0;
   const int last = n_levels - 1;
   for (;;) {
-    const SkipLevel lv = {levels[l].bits, levels[l].base, levels[l].begin, levels[l].end};
+    const SkipLevel lv = {of_level(mine.bits, l), of_level(mine.base, l),
+                          (uint32_t)of_level((int)mine.begin, l),
+                          (uint32_t)of_level((int)mine.end, l)};
     Prefix<DDP> p;
-    bool alive;
     if (l == 0) {
       if (tile >= tiles) {  // used up: on with what is held
         if (empty == 0) empty = 1;
@@ -132,7 +147,7 @@ void ryser_skip_tree_kernel(const SkipRecord* __restrict__ records_arg,
       p.prod = 1.0;
       p.tail = 0.0;
       tile += waves;
-      alive = true;
+      if (last == 0) formed += 1.0;
     } else {
       const uint32_t have = (uint32_t)__builtin_amdgcn_readlane((int)held, l);
       const uint32_t full = (uint32_t)kWave >> lv.bits;
@@ -148,20 +163,19 @@ void ryser_skip_tree_kernel(const SkipRecord* __restrict__ records_arg,
       }
       const uint32_t take = have < full ? have : full;
       const uint32_t at = have - take + (lane >> lv.bits);
-      alive = (lane >> lv.bits) < take;
       const uint64_t* st = stack(l);
       p.set = 0;
       p.prod = 0.0;
       p.tail = 0.0;
-      if (alive) {
+      if ((lane >> lv.bits) < take) {
+        if (l == last) formed += 1.0;
         p.set = st[at] | (uint64_t)(lane & ((1u << lv.bits) - 1u)) << lv.base;
         p.prod = __builtin_bit_cast(double, st[kSkipLevelRoom + at]);
         if constexpr (DDP) p.tail = __builtin_bit_cast(double, st[2 * kSkipLevelRoom + at]);
       }
       held = lane == (uint32_t)l ? have - take : held;
     }
-    if (l == last) formed += alive ? 1.0 : 0.0;
-    alive = complete_rows<DDP>(p, records, lv.begin, lv.end, alive);
+    const bool alive = complete_rows<DDP, SINGLE>(p, records, lv.begin, lv.end);
     if (l == last) {
       if (alive) {
         const bool odd = __builtin_popcountll(p.set) & 1;
@@ -201,7 +215,9 @@ hipError_t launch_skip_tree(const SkipTreeLaunch& L, hipStream_t stream, const R
       (L.mode != 0 && L.mode != 1))
     return hipErrorInvalidValue;
   const size_t lds = (size_t)(L.n_levels - 1) * (L.mode ? 3 : 2) * kSkipLevelRoom * 8;
-  const auto kernel = L.mode ? ryser_skip_tree_kernel<true> : ryser_skip_tree_kernel<false>;
+  const auto kernel =
+      L.mode ? L.single ? ryser_skip_tree_kernel<true, true> : ryser_skip_tree_kernel<true, false>
+             : L.single ? ryser_skip_tree_kernel<false, true> : ryser_skip_tree_kernel<false, false>;
   kernel<<<L.waves, kWave, lds, stream>>>(L.records, L.levels, L.n_levels, L.top_bits, L.waves,
                                           L.partials, L.begin_tick);
   if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;

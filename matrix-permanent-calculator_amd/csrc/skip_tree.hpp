@@ -29,17 +29,20 @@ struct SkipLevel {
 constexpr int kSkipMaxLevels = 20;
 constexpr int kSkipMaxLevelBits = 4;
 constexpr int kSkipMaxTopBits = 26;
+// Records per level: a multiple of this (rows of x = 1 fill up).
+constexpr uint32_t kSkipRecordStep = 4;
 // Stored prefixes per level: less than one full step, and one step's.
 constexpr int kSkipLevelRoom = 32 + 64;
 
 struct SkipTreeLaunch {
-  const SkipRecord* records;  // device, 32-byte aligned
+  const SkipRecord* records;  // device, 64-byte aligned
   const SkipLevel* levels;    // device: n_levels, columns from the top down to 0
   Partial* partials;          // device: `waves` records
   Partial* result;            // device: 1 record
   uint64_t* begin_tick;       // device
   int n_levels, top_bits, mode;  // mode 0 FP64, 1 double-double products
   uint32_t waves;
+  bool single;  // every row is one record
 };
 // Enqueue the search and the grid reduction, which reports.  pad of the sum:
 // subsets of all columns formed (the rest was cut off).
@@ -51,6 +54,7 @@ struct TreePlan {
   std::vector<SkipRecord> records;
   int top_bits = 0;
   uint32_t waves = 0;
+  bool single = true;
   double cost = 0.0;  // records expected to be met by all prefixes, and 2 per prefix
 };
 // Greedy order of b columns, the lowest first: next, the column adding the
@@ -64,9 +68,9 @@ double nonzero_share(int n, const double* x0, const double* cols, double* zero);
 // order: of the walked columns (skip_order); n >= 7.
 void plan_tree(int n, const double* x0, const double* cols, const int* order, const double* zero,
                TreePlan& tp);
-// Levels and records as the device reads them (32-byte aligned there).
+// Levels and records as the device reads them (64-byte aligned there).
 inline size_t tree_record_word(const TreePlan& tp) {
-  return (tp.levels.size() * sizeof(SkipLevel) + 31) / 32 * 4;
+  return (tp.levels.size() * sizeof(SkipLevel) + 63) / 64 * 8;
 }
 std::vector<uint64_t> pack_tree(const TreePlan& tp);
 // The launch's plan part; records, result and tick are the caller's.
