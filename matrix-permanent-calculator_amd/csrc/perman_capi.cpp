@@ -609,7 +609,7 @@ int bind_oneshot(int n, const Prepared& prep, DeviceCache& C, perm_plan& P, bool
     P.L.direct_doubles = (uint32_t)(up / sizeof(double));
     return PERM_OK;
   }
-  HIP_TRY(hipMemcpyAsync((void*)P.L.colpm, C.stage, up, hipMemcpyHostToDevice, P.stream));
+  HIP_TRY(perm::launch_fetch(C.stage, (void*)P.L.colpm, up, P.stream));
   return PERM_OK;
 }
 
@@ -643,7 +643,7 @@ int run_cached(const void* up, size_t up_bytes, size_t bytes,
   if (int s = reserve_stage(C, up_bytes)) return s;
   std::memcpy(C.stage, up, up_bytes);
   char* base = static_cast<char*>(C.base);
-  HIP_TRY(hipMemcpyAsync(base, C.stage, up_bytes, hipMemcpyHostToDevice, C.stream));
+  HIP_TRY(launch_fetch(C.stage, base, up_bytes, C.stream));
   const RunReport report{(uint64_t*)(base + tick), C.rec, next_seq()};
   HIP_TRY(launch(base, C.stream, report));
   if (int s = wait_record(C.stream, C.rec, report.seq)) return s;

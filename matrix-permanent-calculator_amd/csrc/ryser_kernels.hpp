@@ -86,6 +86,9 @@ hipError_t launch_skip(const SkipLaunch& L, hipStream_t stream);
 // Only the walk of L (its block range), no reduction (the caller sums the
 // partial records).
 hipError_t launch_dense_pass_only(const DenseLaunch& L, hipStream_t stream);
+// Copies `bytes` (a multiple of 8) of pinned host memory to the device with a
+// kernel.
+hipError_t launch_fetch(const void* host, void* out, size_t bytes, hipStream_t stream);
 // The grid reduction: the DD sum of in[0, count) into *out, in a fixed order.
 hipError_t launch_reduce(const Partial* in, uint64_t count, Partial* out, hipStream_t stream,
                          const RunReport& report = {});
