@@ -33,7 +33,6 @@
 #include "perman_internal.hpp"
 #include "ryser_host.hpp"
 #include "ryser_kernels.hpp"
-#include "skip_tree.hpp"
 
 namespace {
 

@@ -5,6 +5,7 @@
 
 #include "nest_shape.hpp"
 #include "ryser_device.hpp"
+#include "skip_tree.hpp"
 
 namespace perm {
 
@@ -56,6 +57,7 @@ struct DenseLaunch {
 // Largest order whose walk is one workgroup (2^8 lanes).
 constexpr int kMaxDirectN = 12;
 
+
 // One skipping walk (integer matrices; see ryser_skip_impl.hpp).
 struct SkipLaunch {
   const double* colpm;        // device: column store in walk order
@@ -82,6 +84,11 @@ struct SkipLaunch {
 constexpr int kMinSkipN = 16;
 // Enqueue the skipping kernel and the grid reduction on `stream`.
 hipError_t launch_skip(const SkipLaunch& L, hipStream_t stream);
+
+// Enqueue the search of the subsets without a zero row and the grid reduction,
+// which reports.  sq_run of the sum: subsets of all columns formed (the rest
+// was cut off).
+hipError_t launch_skip_tree(const SkipTreeLaunch& L, hipStream_t stream, const RunReport& report);
 
 // Only the walk of L (its block range), no reduction (the caller sums the
 // partial records).

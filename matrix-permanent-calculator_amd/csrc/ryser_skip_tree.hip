@@ -38,7 +38,6 @@
 // passes) 9.6 -> 0.33 ms.
 #include "ryser_device.hpp"
 #include "ryser_kernels.hpp"
-#include "skip_tree.hpp"
 
 namespace perm {
 

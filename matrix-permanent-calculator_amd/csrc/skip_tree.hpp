@@ -1,7 +1,6 @@
 // skip_tree.hpp -- the skipping walk as a tree search (ryser_skip_tree.hip):
-// what its host plan and its kernel share.  No device code.
+// what its host plan and its kernel share (no HIP headers).
 #pragma once
-#include <hip/hip_runtime.h>
 #include <stdint.h>
 
 #include <vector>
@@ -9,7 +8,6 @@
 namespace perm {
 
 struct Partial;
-struct RunReport;
 
 // Columns of one value in one row.  A row is the records up to the one with
 // `last`; x = start + sum over its records of value * popcount(S & mask).
@@ -44,10 +42,6 @@ struct SkipTreeLaunch {
   uint32_t waves;
   bool single;  // every row is one record
 };
-// Enqueue the search and the grid reduction, which reports.  pad of the sum:
-// subsets of all columns formed (the rest was cut off).
-hipError_t launch_skip_tree(const SkipTreeLaunch& L, hipStream_t stream, const RunReport& report);
-
 // The search's plan (host; perman_skip_plan.cpp).
 struct TreePlan {
   std::vector<SkipLevel> levels;
