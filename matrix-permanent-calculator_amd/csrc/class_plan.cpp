@@ -91,7 +91,7 @@ bool settle(uint64_t (&rows)[kClasses], bool thin) {
 }
 
 int plan_cost(const uint64_t (&rows)[kClasses], bool thin) {
-  int cost = 2 * kClasses;
+  int cost = thin ? 3 * kClasses / 2 : 2 * kClasses;  // the final sum
   for (int t = 0; t < kClasses; ++t) {
     if (!rows[t]) continue;
     cost += (2 * __builtin_popcountll(rows[t]) - 1) << class_popcount(t);
