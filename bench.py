@@ -30,9 +30,10 @@ os.environ.setdefault("OMP_PROC_BIND", "close")
 FULL_CPU_SET = os.sched_getaffinity(0)
 
 # HBM bytes per launch of the n=40 kernel on this workload: rocprofv3 FETCH_SIZE
-# + WRITE_SIZE (profiles/ryser_class.md): 856 KiB read + 65536 KiB written
-# (2^20 workgroup records of 48 B, each one 64-B line write).
-TRAFFIC_BYTES_N40 = (856.1 + 65536.0) * 1024
+# + WRITE_SIZE (profiles/ryser_class.md, another n = 40 matrix of density 0.5):
+# 1708 KiB read + 65536 KiB written (2^20 workgroup records of 48 B, each one
+# 64-B line write).
+TRAFFIC_BYTES_N40 = (1707.6 + 65536.0) * 1024
 FP64_PEAK_TFLOPS = 78.6
 # FP64 lane-instructions the chip issues per second (an FMA is one: half the
 # flop rate), in T/s
