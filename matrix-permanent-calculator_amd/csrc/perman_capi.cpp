@@ -88,6 +88,9 @@ struct perm_plan {
   uint64_t rec_cap = 0;
   double* zdev = nullptr;   // device: one variance weight per workgroup record
   perm::HostRecord* rec = nullptr;  // pinned: where a run's last kernel reports
+  // non-null: the kernels report into this record in device memory instead,
+  // and its copy lands in `rec` (any host memory)
+  perm::HostRecord* dev_rec = nullptr;
   uint64_t* begin = nullptr;        // device: begin tick of the run
   perm::Partial* vrec = nullptr;  // device: 2 kVerifyUnits records (FP64, then mode 2)
   std::vector<double> zhost;      // host copy of zdev (kept between runs)
@@ -174,6 +177,18 @@ int wait_record(hipStream_t stream, const perm::HostRecord* rec, uint64_t seq) {
   HIP_TRY(hipStreamSynchronize(stream));
   if (!arrived()) return fail(PERM_ERR_HIP, "a run ended without its record");
   return PERM_OK;
+}
+
+// Where P's kernels report run `seq`, and the wait for it.
+perm::RunReport next_report(const perm_plan* P) {
+  return {P->begin, P->dev_rec ? P->dev_rec : P->rec, next_seq()};
+}
+int wait_run(perm_plan* P, uint64_t seq) {
+  if (P->dev_rec) {
+    HIP_TRY(hipMemcpyAsync(P->rec, P->dev_rec, sizeof(*P->rec), hipMemcpyDeviceToHost, P->stream));
+    HIP_TRY(hipStreamSynchronize(P->stream));
+  }
+  return wait_record(P->stream, P->rec, seq);
 }
 
 // Device layout of a plan: column store, x0, the class walk's tables (these
@@ -381,9 +396,9 @@ int run_pass(perm_plan* P, int mode, perm::Partial& r, float& ms, float& main_ms
     T.partials = P->L.partials;
     T.result = P->L.result;
     T.begin_tick = P->begin;
-    const perm::RunReport report{P->begin, P->rec, next_seq()};
+    const perm::RunReport report = next_report(P);
     HIP_TRY(perm::launch_skip_tree(T, P->stream, report));
-    if (int s = wait_record(P->stream, P->rec, report.seq)) return s;
+    if (int s = wait_run(P, report.seq)) return s;
     r = P->rec->sum;
     r.sq_run = 0.0;  // (the subsets formed)
     ms = (float)(1e-5 * (double)(P->rec->end - P->rec->begin));
@@ -393,14 +408,14 @@ int run_pass(perm_plan* P, int mode, perm::Partial& r, float& ms, float& main_ms
   // one workgroup: its record is the sum, the walk the only kernel
   const bool single = P->L.total_blocks <= 1;
   perm::RunReport& report = P->L.report;
-  report = {P->begin, P->rec, next_seq()};
+  report = next_report(P);
   HIP_TRY(launch_walk(P, 0, P->L.total_blocks, 0));
   P->L.direct = nullptr;  // (the matrix is in place now)
   if (!single)
     HIP_TRY(perm::launch_reduce(P->L.partials, P->L.total_blocks, P->L.result, P->stream, report));
   const uint64_t seq = report.seq;
   report = {};
-  if (int s = wait_record(P->stream, P->rec, seq)) return s;
+  if (int s = wait_run(P, seq)) return s;
   r = P->rec->sum;
   ms = (float)(1e-5 * (double)(P->rec->end - P->rec->begin));  // 10 ns ticks
   main_ms = (float)(1e-5 * (double)(P->rec->main_end - P->rec->begin));
@@ -792,6 +807,8 @@ int run_prepared(int n, const Prepared& p, int mode, perm_result* out) {
 // records of 48 bytes); larger n are rejected with PERM_ERR_SIZE.
 constexpr size_t kScratchBytes = (size_t)4 << 20;
 static __device__ __align__(256) char scratch[kScratchBytes];
+// The record its runs report into: pinned host memory would be an allocation.
+static __device__ __align__(256) char scratch_record[sizeof(perm::HostRecord)];
 
 namespace {
 
@@ -804,7 +821,8 @@ struct NoallocDevice {
   std::mutex mu;
   bool ready = false;
   char* ptr = nullptr;
-  perm::HostRecord* rec = nullptr;
+  perm::HostRecord* dev_rec = nullptr;  // scratch_record
+  perm::HostRecord rec;                 // its copy
   hipStream_t stream = nullptr;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
 };
@@ -817,7 +835,10 @@ int noalloc_setup(NoallocDevice& D) {
   HIP_TRY(hipStreamCreateWithFlags(&D.stream, hipStreamNonBlocking));
   HIP_TRY(hipEventCreate(&D.ev0));
   HIP_TRY(hipEventCreate(&D.ev1));
-  if (int s = take_record(&D.rec)) return s;
+  void* r = nullptr;
+  HIP_TRY(hipGetSymbolAddress(&r, HIP_SYMBOL(scratch_record)));
+  if (!r) return fail(PERM_ERR_HIP, "hipGetSymbolAddress(scratch_record) returned a null address");
+  D.dev_rec = (perm::HostRecord*)r;
   D.ptr = (char*)p;
   D.ready = true;
   return PERM_OK;
@@ -935,7 +956,8 @@ int perm_dense_noalloc(int dtype, const void* mat, int nov, int algo_id, perm_re
   P.device = dev;
   P.borrowed = true;
   P.stream = D.stream;
-  P.rec = D.rec;
+  P.rec = &D.rec;
+  P.dev_rec = D.dev_rec;
   P.ev0 = D.ev0;
   P.ev1 = D.ev1;
   P.integral = p.integral;
