@@ -1068,9 +1068,12 @@ int perm_batch_compute_dense(perm_batch* B, int count, const int* dtypes,
     int w = 0, h = 0;
     perm::batch_split(novs[i], B->item_log2, w, h);
     items_ub += ((1ull << h) + perm::kItemLanes - 1) / perm::kItemLanes;
-    if (novs[i] >= perm::kMinBatchClassN && class_split_ok(w)) {
+    if (novs[i] >= perm::kMinBatchClassN) {
+      // (prepared whatever the split: the class plan also sets the column
+      // order, and the split may be changed before a later run)
       tables = perm::class_tables_bound(novs[i]);
-      split_ub += perm::class_split_doubles(novs[i], w - perm::kClassBits) + 8;
+      if (class_split_ok(w))
+        split_ub += perm::class_split_doubles(novs[i], w - perm::kClassBits) + 8;
     }
     place[(size_t)k + 1] = place[(size_t)k] + entry_room((2 * n - 1) * n + 2 * n, tables);
   }
