@@ -568,11 +568,25 @@ int plan_run_impl(perm_plan* P, int mode, perm_result* out) {
 // The cache's stream and `bytes` of its memory, with no earlier call's work
 // left on them (caller holds C.mu).
 int reserve_cache(DeviceCache& C, size_t bytes) {
-  if (!C.stream) {
-    HIP_TRY(hipStreamCreateWithFlags(&C.stream, hipStreamNonBlocking));
-    HIP_TRY(hipEventCreate(&C.ev0));
-    HIP_TRY(hipEventCreate(&C.ev1));
-    if (int s = take_record(&C.rec)) return s;
+  if (!C.stream) {  // all of them, or none: a call that fails leaves the cache as it was
+    hipStream_t stream = nullptr;
+    hipEvent_t ev0 = nullptr, ev1 = nullptr;
+    hipError_t e = hipStreamCreateWithFlags(&stream, hipStreamNonBlocking);
+    if (e == hipSuccess) e = hipEventCreate(&ev0);
+    if (e == hipSuccess) e = hipEventCreate(&ev1);
+    int s = PERM_OK;
+    if (e != hipSuccess)
+      s = fail(PERM_ERR_HIP, std::string("stream and events: ") + hipGetErrorString(e));
+    if (s == PERM_OK) s = take_record(&C.rec);
+    if (s != PERM_OK) {
+      if (ev1) (void)hipEventDestroy(ev1);
+      if (ev0) (void)hipEventDestroy(ev0);
+      if (stream) (void)hipStreamDestroy(stream);
+      return s;
+    }
+    C.stream = stream;
+    C.ev0 = ev0;
+    C.ev1 = ev1;
   }
   if (C.busy) HIP_TRY(hipStreamSynchronize(C.stream));  // an earlier call failed midway
   C.busy = true;
