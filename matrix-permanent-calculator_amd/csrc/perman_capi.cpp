@@ -784,6 +784,7 @@ int run_chunked(int n, const Prepared& prep, bool use_cpu, int threads, perm_res
     }
     out->kernel_ms += chunk_ms;
   }
+  C.busy = false;
   return ok();
 }
 

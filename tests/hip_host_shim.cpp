@@ -85,6 +85,14 @@ hipError_t hipMemcpyAsync(void* dst, const void* src, size_t bytes, hipMemcpyKin
   std::memcpy(dst, src, bytes);
   return called("hipMemcpyAsync");
 }
+// (around every <<<>>>: the stub between them passes the values on)
+hipError_t __hipPushCallConfiguration(dim3, dim3, size_t, hipStream_t) { return hipSuccess; }
+hipError_t __hipPopCallConfiguration(dim3* grid, dim3* block, size_t* lds, hipStream_t* stream) {
+  *grid = *block = dim3(1, 1, 1);
+  *lds = 0;
+  *stream = nullptr;
+  return hipSuccess;
+}
 hipError_t hipLaunchKernel(const void*, dim3, dim3, void**, size_t, hipStream_t) {
   return called("hipLaunchKernel");
 }

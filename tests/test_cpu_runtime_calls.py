@@ -74,3 +74,23 @@ events = made.count("hipEventCreate") - made.count("hipEventDestroy")
 failed = {{"hipStreamCreateWithFlags": (1, 0), "hipEventCreate": (0, 1)}}.get("{name}", (0, 0))
 assert (live, events) == (1 + failed[0], 2 + failed[1]), (made, live, events)
 """)
+
+
+@needs_hip
+def test_call_after_a_chunked_one_does_not_wait(shim):
+    """A chunked run waits for its last kernel: the call after it finds the
+    stream idle and starts without another wait; after one that failed midway
+    it waits first."""
+    run(shim, """
+P.chunked(real)
+calls()
+error(lambda: P.dense(real))
+log = calls()
+assert log.index("hipLaunchKernel") < log.index("hipStreamSynchronize"), log
+shim.shim_fail(b"hipEventRecord", 1)
+assert error(lambda: P.chunked(real))
+calls()
+error(lambda: P.dense(real))
+log = calls()
+assert log.index("hipStreamSynchronize") < log.index("hipLaunchKernel"), log
+""")
