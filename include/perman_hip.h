@@ -299,8 +299,9 @@ double perm_xshared_coalescing_mshared_skipper_f64(const double* mat, const int*
  * shared counter to the GPU and, with cpu != 0, to a CPU worker using
  * `threads` OpenMP threads; the partial sums are combined by the same grid
  * reduction as the one-launch path.
- * Without the CPU worker the value equals the one-launch value bitwise; with
- * it, the chunks the CPU took differ in rounding only.  ID 8 runs the skipper
+ * Without the CPU worker the value equals the one-launch value bitwise (a
+ * sparse integer matrix that perm_dense and perm_sparse compute by a search
+ * is searched in one piece); with it, sums differ in rounding only.  ID 8 runs the skipper
  * on the GPU alone.  perm_chunked is the full-result form (cptrs NULL:
  * dense); *cpu_chunks receives the number of chunks the CPU computed. */
 int perm_chunked(int dtype, const void* mat, const int* cptrs, const int* rows,

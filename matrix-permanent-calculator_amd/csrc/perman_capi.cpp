@@ -313,6 +313,12 @@ void configure_passes(perm_plan* P, int mode) {
   L.total_blocks = L.main.blocks;
 }
 
+// A run's pass in `mode` is the search (after configure_passes: its records
+// have the room of the walk's).
+bool searched(const perm_plan& P, int mode) {
+  return (P.tree_modes >> mode) & 1u && P.tree.waves <= P.L.total_blocks;
+}
+
 // Bytes of the column store, start vector and class tables as they lie on the
 // device, from colpm on; packed: written there (one copy uploads them).
 size_t packed_bytes(const perm_plan* P, const Prepared& prep) {
@@ -390,7 +396,7 @@ int make_plan(int n, const Prepared& prep, perm_plan** out) {
 // ms = device time of all its kernels, main_ms = of the main pass.
 int run_pass(perm_plan* P, int mode, perm::Partial& r, float& ms, float& main_ms) {
   configure_passes(P, mode);
-  if ((P->tree_modes >> mode) & 1u && P->tree.waves <= P->L.total_blocks) {
+  if (searched(*P, mode)) {
     perm::SkipTreeLaunch T = P->tree;
     T.mode = mode;
     T.partials = P->L.partials;
@@ -696,7 +702,8 @@ namespace {
 // `threads` OpenMP threads.  When the counter is exhausted the CPU chunks'
 // sums are written over their blocks' partial records and the device grid
 // reduction sums all records, in the one-launch order.
-// Without the CPU worker the result equals the one-launch result bitwise;
+// Without the CPU worker the result equals the one-launch result bitwise
+// (where that is a search, it is run in one piece here too);
 // with it, chunks the CPU took differ in rounding only.
 int run_chunked(int n, const Prepared& prep, bool use_cpu, int threads, perm_result* out,
                 int* cpu_chunks_out) {
@@ -712,6 +719,11 @@ int run_chunked(int n, const Prepared& prep, bool use_cpu, int threads, perm_res
   if (int s = bind_oneshot(n, prep, C, P, false)) return s;
   configure_passes(&P, 0);
   perm::DenseLaunch& L = P.L;
+  if (!use_cpu && searched(P, 0)) {  // no workgroups to hand out
+    if (int s = plan_run_impl(&P, -1, out)) return s;
+    C.busy = false;
+    return ok();
+  }
   const uint64_t mb = L.main.blocks;
   const int shift = std::max(0, n - (use_cpu ? 28 : 29));
   const uint64_t chunks =
