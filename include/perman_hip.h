@@ -80,14 +80,15 @@ typedef struct perm_result {
   int integral;         /* 1 if every entry is an integer (X is then exact) */
   double err_est;       /* statistical error estimate (independent roundings) */
   int nu;               /* FP64 kernel: rows touched by Gray column 0 (pair/nested variant), or n */
-  double main_ms;       /* single-matrix path: device time of the main walk kernel */
-  double main_subsets;  /* subsets that kernel evaluated */
+  double main_ms;       /* single-matrix path: device time of the first pass's walk or search */
+  double main_subsets;  /* subsets that kernel evaluated (a search forms a part of them) */
   int nu1;              /* FP64 kernel: rows touched by Gray columns 0-1 (nested variant), or n */
   int nu2;              /* FP64 kernel: rows touched by Gray columns 0-2 (nested variant), or n */
   int certified;        /* 1: exact, or err_est <= 1e-10 |value| */
   int zero_pattern;     /* 1: no perfect matching in the nonzero pattern; value is exactly 0 */
   double clock_ghz;     /* single-matrix path: mean shader clock of the first pass's walk,
-                           from its workgroups' cycle and 100 MHz real-time counters (0: none) */
+                           from its workgroups' cycle and 100 MHz real-time counters (0: not
+                           measured, as by a search) */
   int verified_units;   /* single-matrix path: workgroups of the FP64 walk recomputed in mode 2
                            to measure its error (err_est then comes from them); 0: none */
 } perm_result;

@@ -392,9 +392,20 @@ int make_plan(int n, const Prepared& prep, perm_plan** out) {
   return ok();
 }
 
-// Launch one run (FP64 or double-double products) and read the result;
-// ms = device time of all its kernels, main_ms = of the main pass.
-int run_pass(perm_plan* P, int mode, perm::Partial& r, float& ms, float& main_ms) {
+// One run (FP64, double-double products or double-double X) as read back.
+struct PassRun {
+  perm::Partial sum;
+  float ms = 0.f, main_ms = 0.f;  // device time of all its kernels, of the walk or search
+  double subsets = 0.0;           // that one evaluated
+  double clock_ghz = 0.0;         // its mean shader clock (0: not measured)
+};
+// Launch one run and read the result.
+int run_pass(perm_plan* P, int mode, PassRun& out) {
+  const auto read_record = [&] {
+    out.sum = P->rec->sum;
+    out.ms = (float)(1e-5 * (double)(P->rec->end - P->rec->begin));  // 10 ns ticks
+    out.main_ms = (float)(1e-5 * (double)(P->rec->main_end - P->rec->begin));
+  };
   configure_passes(P, mode);
   if (searched(*P, mode)) {
     perm::SkipTreeLaunch T = P->tree;
@@ -405,10 +416,10 @@ int run_pass(perm_plan* P, int mode, perm::Partial& r, float& ms, float& main_ms
     const perm::RunReport report = next_report(P);
     HIP_TRY(perm::launch_skip_tree(T, P->stream, report));
     if (int s = wait_run(P, report.seq)) return s;
-    r = P->rec->sum;
-    r.sq_run = 0.0;  // (the subsets formed)
-    ms = (float)(1e-5 * (double)(P->rec->end - P->rec->begin));
-    main_ms = (float)(1e-5 * (double)(P->rec->main_end - P->rec->begin));
+    read_record();
+    out.subsets = out.sum.sq_run;  // (the subsets formed)
+    out.sum.sq_run = 0.0;
+    out.clock_ghz = 0.0;
     return PERM_OK;
   }
   // one workgroup: its record is the sum, the walk the only kernel
@@ -422,9 +433,9 @@ int run_pass(perm_plan* P, int mode, perm::Partial& r, float& ms, float& main_ms
   const uint64_t seq = report.seq;
   report = {};
   if (int s = wait_run(P, seq)) return s;
-  r = P->rec->sum;
-  ms = (float)(1e-5 * (double)(P->rec->end - P->rec->begin));  // 10 ns ticks
-  main_ms = (float)(1e-5 * (double)(P->rec->main_end - P->rec->begin));
+  read_record();
+  out.subsets = (double)P->L.main.lanes * std::ldexp(1.0, P->L.main.walk_bits);
+  out.clock_ghz = 0.1 * out.sum.pad / (double)std::max<uint64_t>(1, P->L.total_blocks);
   return PERM_OK;
 }
 
@@ -537,14 +548,11 @@ int plan_run_impl(perm_plan* P, int mode, perm_result* out) {
   }
   HIP_TRY(hipSetDevice(P->device));
   if (int s = ensure_records(P, blocks_of(1ull << P->high_bits))) return s;
-  perm::Partial r;
-  float ms = 0.f, main_ms = 0.f, first_main_ms = 0.f;
+  PassRun run;
   const int first = mode < 0 ? 0 : mode;
-  if (int s = run_pass(P, first, r, ms, first_main_ms)) return s;
-  fill_result(P, r, first, out);
-  const double clock_ghz = 0.1 * r.pad / (double)std::max<uint64_t>(1, P->L.total_blocks);
-  double total_ms = ms;
-  const double first_subsets = (double)P->L.main.lanes * std::ldexp(1.0, P->L.main.walk_bits);
+  if (int s = run_pass(P, first, run)) return s;
+  fill_result(P, run.sum, first, out);
+  double total_ms = run.ms;
   uint32_t verified = 0;
   if (mode < 0) {
     // a non-integer result over many workgroups: measure its error on a
@@ -558,16 +566,17 @@ int plan_run_impl(perm_plan* P, int mode, perm_result* out) {
     }
     // at most two more passes: the mode strictly increases
     for (int next = perm::escalation_mode(*out); next >= 0; next = perm::escalation_mode(*out)) {
-      if (int s = run_pass(P, next, r, ms, main_ms)) return s;
-      fill_result(P, r, next, out);
-      total_ms += ms;
+      PassRun more;
+      if (int s = run_pass(P, next, more)) return s;
+      fill_result(P, more.sum, next, out);
+      total_ms += more.ms;
     }
   }
   out->verified_units = (int)verified;
   out->kernel_ms = total_ms;
-  out->main_ms = first_main_ms;
-  out->main_subsets = first_subsets;
-  out->clock_ghz = clock_ghz;
+  out->main_ms = run.main_ms;
+  out->main_subsets = run.subsets;
+  out->clock_ghz = run.clock_ghz;
   return ok();
 }
 

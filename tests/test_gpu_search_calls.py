@@ -28,3 +28,22 @@ def test_chunked_without_the_cpu_has_the_bits_of_one_launch(n, density):
             one.value, one.sum_hi, one.sum_lo, one.abs_sum, one.err_est, one.mode, one.certified)
     h, _ = P.chunked(a, use_cpu=True, threads=4)
     assert abs(h.value - one.value) <= h.stated + one.stated
+
+
+@pytest.mark.parametrize("n,density", [(29, 0.1), (30, 0.12), (33, 0.12)])
+def test_main_subsets_are_those_the_search_formed(n, density):
+    """main_subsets: subsets the first pass evaluated, which the search and
+    the skipper (the same search) agree on; other passes evaluate all."""
+    a = threes(n, density) // 3
+    plan = P.Plan(a)
+    runs = [P.dense(a), P.sparse(a), P.chunked(a)[0], plan.run(), plan.run(mode=0)]
+    part = plan.run_blocks(0, 1)
+    plan.close()
+    want = P.skip(a).main_subsets
+    assert 0 < want < 0.1 * 2.0 ** (n - 1)
+    for r in runs:
+        assert r.main_subsets == want and r.subsets == 2.0 ** (n - 1), r
+        assert r.clock_ghz == 0.0  # (the search measures none)
+    assert part.main_subsets < part.subsets
+    full = P.synthetic_matrix(n, 0.5, n)
+    assert P.dense(full).main_subsets == 2.0 ** (n - 1)
