@@ -398,6 +398,7 @@ struct PassRun {
   float ms = 0.f, main_ms = 0.f;  // device time of all its kernels, of the walk or search
   double subsets = 0.0;           // that one evaluated
   double clock_ghz = 0.0;         // its mean shader clock (0: not measured)
+  bool searched = false;
 };
 // Launch one run and read the result.
 int run_pass(perm_plan* P, int mode, PassRun& out) {
@@ -420,6 +421,7 @@ int run_pass(perm_plan* P, int mode, PassRun& out) {
     out.subsets = out.sum.sq_run;  // (the subsets formed)
     out.sum.sq_run = 0.0;
     out.clock_ghz = 0.0;
+    out.searched = true;
     return PERM_OK;
   }
   // one workgroup: its record is the sum, the walk the only kernel
@@ -439,7 +441,9 @@ int run_pass(perm_plan* P, int mode, PassRun& out) {
   return PERM_OK;
 }
 
-void fill_result(const perm_plan* P, const perm::Partial& r, int mode, perm_result* out) {
+// r: the sum of a run in `mode`, by a search or a walk.
+void fill_result(const perm_plan* P, const perm::Partial& r, int mode, perm_result* out,
+                 bool by_search = false) {
   const int n = P->n;
   const double scale = (double)(4 * (n & 1) - 2);
   out->n = n;
@@ -447,8 +451,11 @@ void fill_result(const perm_plan* P, const perm::Partial& r, int mode, perm_resu
   out->sum_lo = r.lo;
   out->value = scale * (r.hi + r.lo);
   out->abs_sum = std::fabs(scale) * r.abs_sum;
-  out->err_bound = perm::error_statement(out->abs_sum, out->value, n, P->walk_bits,
-                                         P->unroll_bits, P->integral, mode);
+  out->err_bound =
+      by_search && mode == 1
+          ? perm::search_error_statement(out->abs_sum, std::fabs(scale) * r.pad, n)
+          : perm::error_statement(out->abs_sum, out->value, n, P->walk_bits, P->unroll_bits,
+                                  P->integral, mode);
   out->subsets = std::ldexp(1.0, n - 1);
   out->err_est = perm::error_estimate(scale * scale * r.sq_sum, scale * scale * r.sq_run,
                                       out->value, n, mode == 0 ? P->est_walk_bits : P->walk_bits,
@@ -551,7 +558,7 @@ int plan_run_impl(perm_plan* P, int mode, perm_result* out) {
   PassRun run;
   const int first = mode < 0 ? 0 : mode;
   if (int s = run_pass(P, first, run)) return s;
-  fill_result(P, run.sum, first, out);
+  fill_result(P, run.sum, first, out, run.searched);
   double total_ms = run.ms;
   uint32_t verified = 0;
   if (mode < 0) {
@@ -568,7 +575,7 @@ int plan_run_impl(perm_plan* P, int mode, perm_result* out) {
     for (int next = perm::escalation_mode(*out); next >= 0; next = perm::escalation_mode(*out)) {
       PassRun more;
       if (int s = run_pass(P, next, more)) return s;
-      fill_result(P, more.sum, next, out);
+      fill_result(P, more.sum, next, out, more.searched);
       total_ms += more.ms;
     }
   }

@@ -289,7 +289,9 @@ int run_tree(int n, const perm::TreePlan& tp, int mode, perm::Partial& r, double
   return PERM_OK;
 }
 
-void fill(int n, const SkipPrepared& sp, const perm::Partial& r, int mode, perm_result* out) {
+// r: the sum of a run in `mode`, by the search or the walk.
+void fill(int n, const SkipPrepared& sp, const perm::Partial& r, int mode, bool by_search,
+          perm_result* out) {
   std::memset(out, 0, sizeof(*out));
   const double scale = (double)(4 * (n & 1) - 2);
   out->n = n;
@@ -297,8 +299,11 @@ void fill(int n, const SkipPrepared& sp, const perm::Partial& r, int mode, perm_
   out->sum_lo = r.lo;
   out->value = scale * (r.hi + r.lo);
   out->abs_sum = std::fabs(scale) * r.abs_sum;
-  out->err_bound = perm::error_statement(out->abs_sum, out->value, n, sp.walk_bits,
-                                         perm::dense_unroll_bits(n), true, mode);
+  out->err_bound =
+      by_search && mode == 1
+          ? perm::search_error_statement(out->abs_sum, std::fabs(scale) * r.pad, n)
+          : perm::error_statement(out->abs_sum, out->value, n, sp.walk_bits,
+                                  perm::dense_unroll_bits(n), true, mode);
   out->err_est = perm::error_estimate(scale * scale * r.sq_sum, 0.0, out->value, n, sp.walk_bits,
                                       sp.high_bits, mode, true);
   out->subsets = std::ldexp(1.0, n - 1);
@@ -360,13 +365,13 @@ int perm_skip(int dtype, const void* mat, const int* rptrs, const int* cols, con
   double walked = 0.0;
   float ms = 0.f, ms2 = 0.f;
   if (int s = run(0, r, walked, ms)) return s;
-  fill(nov, sp, r, 0, out);
+  fill(nov, sp, r, 0, tree, out);
   // integer matrix: X is exact, so the only escalation is double-double
   // products (exact rounding below 2^53, error ~2^-104 A above)
   if (perm::escalation_mode(*out) == 1) {
     double walked2 = 0.0;
     if (int s = run(1, r, walked2, ms2)) return s;
-    fill(nov, sp, r, 1, out);
+    fill(nov, sp, r, 1, tree, out);
   }
   out->kernel_ms = (double)ms + (double)ms2;
   out->main_ms = ms;

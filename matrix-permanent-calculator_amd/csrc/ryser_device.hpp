@@ -22,7 +22,8 @@ constexpr int kWave = 64;
 // (signed sum of the run)^2 (the X drift: it moves a run's terms together,
 // so its effect follows the run's cancelled sum).  pad: the dense walk kernel
 // stores its workgroup's shader cycles per 10 ns real-time tick (summed by
-// the grid reduction: mean clock = 0.1 GHz * sum / workgroups).  48 bytes.
+// the grid reduction: mean clock = 0.1 GHz * sum / workgroups), the search of
+// double-double products its running sums' magnitudes.  48 bytes.
 struct Partial {
   double hi, lo, abs_sum, sq_sum, sq_run, pad;
 };
@@ -115,6 +116,16 @@ __device__ __forceinline__ void wave_reduce(DD& s, Moments& m) {
   m.a += mu.a;
   m.q += mu.q;
   m.r += mu.r;
+}
+
+// Wave-wide sum of v, valid in lane 0.
+__device__ __forceinline__ double wave_sum(double v) {
+  v += swizzle_xor<1>(v);
+  v += swizzle_xor<2>(v);
+  v += swizzle_xor<4>(v);
+  v += swizzle_xor<8>(v);
+  v += swizzle_xor<16>(v);
+  return v + readlane_d(v, 32);
 }
 
 __device__ __forceinline__ Partial make_partial(DD s, const Moments& m) {

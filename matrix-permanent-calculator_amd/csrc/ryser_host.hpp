@@ -156,6 +156,16 @@ inline double error_statement(double abs_sum_scaled, double value, int n, int wa
   return abs_sum_scaled * u * ((double)n + 1.0 + fold) + start;
 }
 
+// err_bound of the search with double-double products (integer matrices): its
+// lanes add up as many terms as they meet, not 2^w, so the additions are
+// bounded by what they did.  Each leaves at most 2^-105 of the running sum
+// (dd_add_d; two per term), `running` = |scale| * the sum of those magnitudes;
+// the reductions over lanes and waves, 6 + 32 + 10 additions deep, and a
+// term's n multiplications leave (n + 48) 2^-104 A more.
+inline double search_error_statement(double abs_sum_scaled, double running, int n) {
+  return std::ldexp(abs_sum_scaled * ((double)n + 48.0) + running, -104);
+}
+
 // Expected error (err_est, three standard deviations) when roundings behave
 // as independent random errors, from the moments the kernels measure:
 // Q = sum over runs of 2^(R+5) consecutive terms of (sum of |T| in the run)^2

@@ -87,7 +87,8 @@ hipError_t launch_skip(const SkipLaunch& L, hipStream_t stream);
 
 // Enqueue the search of the subsets without a zero row and the grid reduction,
 // which reports.  sq_run of the sum: subsets of all columns formed (the rest
-// was cut off).
+// was cut off); pad (mode 1): sum of the magnitudes of the lanes' running sums
+// after each of their additions (search_error_statement).
 hipError_t launch_skip_tree(const SkipTreeLaunch& L, hipStream_t stream, const RunReport& report);
 
 // Only the walk of L (its block range), no reduction (the caller sums the

@@ -129,6 +129,7 @@ void ryser_skip_tree_kernel(const SkipRecord* __restrict__ records_arg,
   DD s = {0.0, 0.0};
   Moments mo = {0.0, 0.0, 0.0};
   double formed = 0.0;
+  double running = 0.0;  // sum of the |running sum| after each addition (double-double products)
   const int last = n_levels - 1;
   for (;;) {
     const SkipLevel lv = {of_level(mine.bits, l), of_level(mine.base, l),
@@ -179,7 +180,11 @@ void ryser_skip_tree_kernel(const SkipRecord* __restrict__ records_arg,
       if (alive) {
         const bool odd = __builtin_popcountll(p.set) & 1;
         s = dd_add_d(s, odd ? -p.prod : p.prod);
-        if constexpr (DDP) s = dd_add_d(s, odd ? -p.tail : p.tail);
+        if constexpr (DDP) {
+          running += __builtin_fabs(s.hi);
+          s = dd_add_d(s, odd ? -p.tail : p.tail);
+          running += __builtin_fabs(s.hi);
+        }
         mo.a += __builtin_fabs(p.prod);
         mo.q = __builtin_fma(p.prod, p.prod, mo.q);
       }
@@ -205,7 +210,8 @@ void ryser_skip_tree_kernel(const SkipRecord* __restrict__ records_arg,
   }
   // `formed` rides through the reduction as the (unused) drift statistic
   mo.r = formed;
-  block_reduce_store(s, mo, scratch, partials + blockIdx.x);
+  if constexpr (DDP) running = wave_sum(running);
+  block_reduce_store(s, mo, scratch, partials + blockIdx.x, running);
 }
 
 hipError_t launch_skip_tree(const SkipTreeLaunch& L, hipStream_t stream, const RunReport& report) {

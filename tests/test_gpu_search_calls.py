@@ -47,3 +47,24 @@ def test_main_subsets_are_those_the_search_formed(n, density):
     assert part.main_subsets < part.subsets
     full = P.synthetic_matrix(n, 0.5, n)
     assert P.dense(full).main_subsets == 2.0 ** (n - 1)
+
+
+@pytest.mark.parametrize("n,density", [(29, 0.12), (33, 0.12), (33, 0.18)])
+def test_bound_of_a_search_counts_its_own_additions(monkeypatch, n, density):
+    """err_bound with double-double products covers the additions a lane made
+    (tens here), not those of a walk's lane of 2^9 subsets and more (2^10
+    additions of 2^-104 each), and the exact difference to the Gray walk's
+    sum stays within both bounds."""
+    a = threes(n, density)
+    plan = P.Plan(a)
+    r = plan.run(mode=1)
+    plan.close()
+    assert r.clock_ghz == 0.0 and r.main_subsets < r.subsets, "not the search"
+    assert (n + 48) * r.abs_sum * 2.0 ** -104 <= r.err_bound <= 512 * r.abs_sum * 2.0 ** -104, r
+    with monkeypatch.context() as m:
+        m.setenv("PERMAN_PAIR", "0")
+        plan = P.Plan(a)
+        w = plan.run(mode=1)
+        plan.close()
+    diff = abs((r.sum_hi - w.sum_hi) + (r.sum_lo - w.sum_lo))
+    assert 2.0 * diff <= r.err_bound + w.err_bound, (r, w)
