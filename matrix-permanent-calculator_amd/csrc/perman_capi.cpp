@@ -65,9 +65,12 @@ struct perm_plan {
   DeviceBuffers mem;
   perm::DenseLaunch L{};
   int unroll_bits = 0;
-  int walk_bits = 0, high_bits = 0;  // split of the n-1 Gray columns
-  // split the FP64 error estimate is stated for (error_estimate)
-  int est_walk_bits = 0, est_high_bits = 0;
+  int walk_bits = 0, high_bits = 0;  // split of the n-1 Gray columns: perm_plan_geometry
+  // the Gray walk's own split, the one the FP64 error estimate is stated for
+  // (error_estimate); where its walks are the longer ones, its whole passes
+  // run it too (n = 27: 2^8 steps against the class walk's 2^7, whose starts
+  // cost a pass in double-double X 3.5 %: 605 -> 626 us)
+  int gray_walk_bits = 0, gray_high_bits = 0;
   bool classed = false;  // the FP64 pass is the class walk
   size_t table_doubles = 0;  // ClassTables::data
   perm::ClassMatrix cls{};
@@ -203,6 +206,8 @@ struct PlanLayout {
 using perm::kVerifyUnits;
 
 uint64_t blocks_of(uint64_t lanes) { return (lanes + 255) / 256; }
+// Workgroup records of a whole pass, at most.
+uint64_t most_blocks(const perm_plan* P) { return blocks_of(1ull << P->high_bits); }
 
 PlanLayout plan_layout(const perm_plan* P) {
   PlanLayout l;
@@ -210,10 +215,10 @@ PlanLayout plan_layout(const perm_plan* P) {
   l.cls = align_up(P->table_doubles * sizeof(double), 256);
   l.col = align_up(col_doubles * sizeof(double), 256);
   l.x = align_up(2 * (size_t)P->n * sizeof(double), 256);  // start vector and its low parts
-  l.part = align_up(blocks_of(1ull << P->high_bits) * sizeof(perm::Partial), 256);
+  l.part = align_up(most_blocks(P) * sizeof(perm::Partial), 256);
   l.res = align_up(sizeof(perm::Partial) + sizeof(uint64_t), 256);  // and the begin tick
   l.ids = align_up(kVerifyUnits * sizeof(uint32_t), 256);
-  l.z = align_up(blocks_of(1ull << P->high_bits) * sizeof(double), 256);
+  l.z = align_up(most_blocks(P) * sizeof(double), 256);
   l.vrec = align_up(2 * kVerifyUnits * sizeof(perm::Partial), 256);
   return l;
 }
@@ -226,8 +231,8 @@ size_t layout_plan(perm_plan* P, int n, const Prepared& prep) {
   P->table_doubles = prep.classed ? prep.tables.data.size() : 0;
   P->unroll_bits = perm::dense_unroll_bits(n);
   const perm::Split sp = perm::choose_split(n, P->unroll_bits, env_int("PERMAN_WALK_BITS", 0));
-  P->walk_bits = P->est_walk_bits = sp.walk_bits;
-  P->high_bits = P->est_high_bits = sp.high_bits;
+  P->walk_bits = P->gray_walk_bits = sp.walk_bits;
+  P->high_bits = P->gray_high_bits = sp.high_bits;
   if (P->classed) {
     // a class walk workgroup covers the subsets of 256 Gray lanes; the
     // estimate keeps the Gray split's drift (the class walk has less)
@@ -239,7 +244,7 @@ size_t layout_plan(perm_plan* P, int n, const Prepared& prep) {
 }
 
 // Bind the fixed regions at `base`; with `records`, also the workgroup
-// records of all 2^h lanes and their weights right after them.
+// records of a whole pass and their weights right after them.
 void bind_plan_memory(perm_plan* P, const Prepared& prep, void* base, bool records = true) {
   const PlanLayout l = plan_layout(P);
   char* b = (char*)base;
@@ -294,8 +299,11 @@ void set_shape(perm_plan* P, int n, const Prepared& prep) {
   P->nu2 = prep.nu2 > 0 ? prep.nu2 : n;
 }
 
-// The walk of one run in `mode`: all 2^h lanes.
-void configure_passes(perm_plan* P, int mode) {
+// The walk of one run in `mode`: all lanes, of the plan's split or, for a
+// whole pass of the Gray walk in double-double, of its own where that is the
+// coarser one.
+void configure_passes(perm_plan* P, int mode, bool whole = false) {
+  const bool gray = whole && mode > 0 && P->gray_walk_bits > P->walk_bits;
   perm::DenseLaunch& L = P->L;
   L.mode = mode;
   // FP64 and double-double products run the prepared walk shape; the
@@ -303,20 +311,19 @@ void configure_passes(perm_plan* P, int mode) {
   L.nu = mode <= 1 ? P->nu : P->n;
   L.nu1 = mode <= 1 ? P->nu1 : P->n;
   L.nu2 = mode <= 1 ? P->nu2 : P->n;
-  L.main.lanes = 1ull << P->high_bits;
+  L.main.walk_bits = gray ? P->gray_walk_bits : P->walk_bits;
+  L.main.high_bits = gray ? P->gray_high_bits : P->high_bits;
+  L.main.lanes = 1ull << L.main.high_bits;
   L.main.blocks = blocks_of(L.main.lanes);
-  L.main.walk_bits = P->walk_bits;
-  L.main.high_bits = P->high_bits;
   L.main.partials = L.partials;
   L.main.block_begin = 0;
   L.main.block_end = 0;
   L.total_blocks = L.main.blocks;
 }
 
-// A run's pass in `mode` is the search (after configure_passes: its records
-// have the room of the walk's).
+// A run's pass in `mode` is the search (its records have the room of a walk's).
 bool searched(const perm_plan& P, int mode) {
-  return (P.tree_modes >> mode) & 1u && P.tree.waves <= P.L.total_blocks;
+  return (P.tree_modes >> mode) & 1u && P.tree.waves <= most_blocks(&P);
 }
 
 // Bytes of the column store, start vector and class tables as they lie on the
@@ -407,7 +414,7 @@ int run_pass(perm_plan* P, int mode, PassRun& out) {
     out.ms = (float)(1e-5 * (double)(P->rec->end - P->rec->begin));  // 10 ns ticks
     out.main_ms = (float)(1e-5 * (double)(P->rec->main_end - P->rec->begin));
   };
-  configure_passes(P, mode);
+  configure_passes(P, mode, true);
   if (searched(*P, mode)) {
     perm::SkipTreeLaunch T = P->tree;
     T.mode = mode;
@@ -454,12 +461,13 @@ void fill_result(const perm_plan* P, const perm::Partial& r, int mode, perm_resu
   out->err_bound =
       by_search && mode == 1
           ? perm::search_error_statement(out->abs_sum, std::fabs(scale) * r.pad, n)
-          : perm::error_statement(out->abs_sum, out->value, n, P->walk_bits, P->unroll_bits,
-                                  P->integral, mode);
+          : perm::error_statement(out->abs_sum, out->value, n, P->L.main.walk_bits,
+                                  P->unroll_bits, P->integral, mode);
   out->subsets = std::ldexp(1.0, n - 1);
   out->err_est = perm::error_estimate(scale * scale * r.sq_sum, scale * scale * r.sq_run,
-                                      out->value, n, mode == 0 ? P->est_walk_bits : P->walk_bits,
-                                      mode == 0 ? P->est_high_bits : P->high_bits, mode,
+                                      out->value, n,
+                                      mode == 0 ? P->gray_walk_bits : P->L.main.walk_bits,
+                                      mode == 0 ? P->gray_high_bits : P->L.main.high_bits, mode,
                                       P->integral);
   if (perm::integer_sum_exact(P->integral, P->product_bits, out->abs_sum, scale, n))
     out->err_bound = out->err_est = 0.0;  // exact arithmetic throughout
@@ -496,7 +504,7 @@ int verify_sampled(perm_plan* P, perm_result* out, uint32_t& units_out, float& m
   const uint64_t blocks = P->L.total_blocks;
   // variance weights of the FP64 pass's workgroup records, formed on the
   // device (8 bytes per record come back instead of the record)
-  const double run_weight = std::ldexp(1.0, P->est_walk_bits - 1) + (double)P->est_high_bits;
+  const double run_weight = std::ldexp(1.0, P->gray_walk_bits - 1) + (double)P->gray_high_bits;
   HIP_TRY(perm::launch_unit_weights(P->L.partials, blocks, run_weight, P->zdev, P->stream));
   P->zhost.resize(blocks);
   HIP_TRY(hipMemcpyAsync(P->zhost.data(), P->zdev, blocks * sizeof(double),
@@ -554,7 +562,7 @@ int plan_run_impl(perm_plan* P, int mode, perm_result* out) {
     return ok();
   }
   HIP_TRY(hipSetDevice(P->device));
-  if (int s = ensure_records(P, blocks_of(1ull << P->high_bits))) return s;
+  if (int s = ensure_records(P, most_blocks(P))) return s;
   PassRun run;
   const int first = mode < 0 ? 0 : mode;
   if (int s = run_pass(P, first, run)) return s;

@@ -107,19 +107,18 @@ int select_device() {
 // rows [0, K_l).  Row and column permutations leave the permanent unchanged.
 // `menu`: the shapes the kernels that will run the matrix provide.
 // PERMAN_PAIR=0 keeps the natural order; PERMAN_NEST=0 only pair shapes.
-// sup[k]: rows with a nonzero in walked column k.  cp: a column order on
-// entry, whose first `pool` columns are the candidates; the order chosen
-// (the candidates taken first, the others in the order given) on return.
-// rp: the row order chosen.
-void nest_order(int n, perm::NestMenu menu, const uint64_t* sup, int pool, int* cp, int* rp,
-                int& nu, int& nu1, int& nu2) {
+// sup[k]: rows with a nonzero in walked column k.  cand: the `pool`
+// candidates.  bc: the columns chosen (-1: none), the walk's first ones; rp:
+// the row order.
+void nest_order(int n, perm::NestMenu menu, const uint64_t* sup, const int* cand, int pool,
+                int (&bc)[3], int* rp, int& nu, int& nu1, int& nu2) {
   nu = nu1 = nu2 = n;
+  bc[0] = bc[1] = bc[2] = -1;
   for (int k = 0; k < n; ++k) rp[k] = k;
   if (n < perm::kMinPairN || n > perm::kMaxNestN || env_int("PERMAN_PAIR", 1) == 0) return;
   if (env_int("PERMAN_NEST", 1) == 0) menu.mask &= 1u;
   const bool nested = (menu.mask & ~1u) != 0 && n >= perm::kMinNestN;
-  const int B = n - 1;
-  std::vector<int> by_count(cp, cp + pool);
+  std::vector<int> by_count(cand, cand + pool);
   std::stable_sort(by_count.begin(), by_count.end(), [&](int a, int b) {
     return __builtin_popcountll(sup[a]) < __builtin_popcountll(sup[b]);
   });
@@ -128,7 +127,6 @@ void nest_order(int n, perm::NestMenu menu, const uint64_t* sup, int pool, int* 
   const int n0 = std::min(pool, nested ? 8 : 1), n12 = nested ? std::min(pool, 12) : 0;
   int best_cost = perm::nest_cost(n, {n, n, n});
   perm::NestShape best{n, n, n};
-  int bc[3] = {-1, -1, -1};
   // cheapest compiled shape covering supports of sizes (c0, c01, c012)
   auto cover = [&](int c0, int c01, int c012, perm::NestShape& out) {
     int cost = -1;
@@ -201,12 +199,6 @@ void nest_order(int n, perm::NestMenu menu, const uint64_t* sup, int pool, int* 
   }
   for (int j = 0; j < n; ++j)
     if (!((taken >> j) & 1)) rp[nr++] = j;
-  int nc = 0, old[64];
-  std::copy(cp, cp + B, old);
-  for (int l = 0; l < 3; ++l)
-    if (bc[l] >= 0) cp[nc++] = bc[l];
-  for (int k = 0; k < B; ++k)
-    if (old[k] != bc[0] && old[k] != bc[1] && old[k] != bc[2]) cp[nc++] = old[k];
   nu = best.k0;
   nu1 = best.k1;
   nu2 = best.k2;
@@ -443,8 +435,8 @@ static bool class_range(int n, const std::vector<double>& x0, const std::vector<
 constexpr int kMinTreeN = 29;
 constexpr double kTreeRecord = 95.0;
 
-static void prepare_tree(int n, const uint64_t* sup, const std::vector<double>& cols,
-                         Prepared& p) {
+static void plan_search(int n, const uint64_t* sup, const std::vector<double>& cols,
+                        Prepared& p) {
   const double subsets = std::ldexp(1.0, n - 1);
   const double walk = subsets / kTreeRecord * p.plan.cost / (1 << kClassBits);
   const double dd = subsets / kTreeRecord * n;
@@ -456,7 +448,10 @@ static void prepare_tree(int n, const uint64_t* sup, const std::vector<double>& 
   skip_order(n - 1, sup, order);
   plan_tree(n, p.x0.data(), cols.data(), order, zero, p.tree);
   p.tree_modes = (p.tree.cost <= walk ? 1u : 0u) | (p.tree.cost <= dd ? 2u : 0u);
-  if (!p.tree_modes) return;
+}
+
+// The search's plan after the class walk's tables.
+static void append_search(Prepared& p) {
   std::vector<double>& t = p.tables.data;
   while (t.size() % 8) t.push_back(0.0);
   p.tree_off = t.size();
@@ -464,6 +459,15 @@ static void prepare_tree(int n, const uint64_t* sup, const std::vector<double>& 
   t.resize(p.tree_off + packed.size());
   std::memcpy(t.data() + p.tree_off, packed.data(), packed.size() * sizeof(uint64_t));
 }
+
+// Smallest orders at which the Gray walk of a class-walked matrix looks for its
+// first columns among all of them (6 us of host time): its passes in
+// double-double products (of integer matrices; of others only where a caller
+// asks for them) take a millisecond and more there, and the class columns,
+// chosen to overlap little, cost them up to 8 % (density 0.5, n = 32 4.65 ->
+// 4.83 ms, n = 33 8.64 -> 9.26 ms).  Below, and where that pass is a search,
+// the class columns are the candidates.
+constexpr int kMinFreeNestIntegral = 30, kMinFreeNestN = 32;
 
 void finish_prepare(int n, const NestMenu& menu, std::vector<double>& cols, Prepared& p) {
   uint64_t sup[64];
@@ -473,26 +477,36 @@ void finish_prepare(int n, const NestMenu& menu, std::vector<double>& cols, Prep
       if (cols[(size_t)k * n + j] != 0.0) sup[k] |= 1ull << j;
   }
   if (p.integral) p.product_bits = perm::integer_product_bits(p.x0.data(), cols.data(), n);
-  int cp[64], rp[64];
+  const int B = n - 1;
+  int natural[64], rp[64], first[3];
+  for (int k = 0; k < B; ++k) natural[k] = k;
   p.classed = class_order(n, menu) && class_range(n, p.x0, cols);
   if (p.classed) {
     plan_classes(n, sup, p.plan);
     p.classed = p.plan.cost < kClassGain * (1 << kClassBits) * (2 * n + 2);
   }
+  const bool single = menu.mask == kMenuSingle.mask;
+  if (p.classed && single && p.integral && n >= kMinTreeN) plan_search(n, sup, cols, p);
+  const bool free_nest = !p.classed || (!(p.tree_modes & 2u) &&
+                                        n >= (p.integral ? kMinFreeNestIntegral : kMinFreeNestN));
+  nest_order(n, menu, sup, free_nest ? natural : p.plan.cols, free_nest ? B : kClassBits, first,
+             rp, p.nu, p.nu1, p.nu2);
+  const auto chosen = [&](int k) { return k == first[0] || k == first[1] || k == first[2]; };
   if (p.classed) {
+    // the Gray walk's first columns follow the class columns: both are among
+    // the first eight then, which a workgroup of either walk covers
+    std::stable_partition(p.plan.cols + kClassBits, p.plan.cols + B, chosen);
     // (a batch chooses its split later, and its tables are expanded on the
     // device)
-    const bool single = menu.mask == kMenuSingle.mask;
     build_class_tables(p.plan, p.x0.data(), cols.data(), single ? class_walk_bits(n) : -1,
                        p.tables);
-    if (single && p.integral && n >= kMinTreeN) prepare_tree(n, sup, cols, p);
-    std::copy(p.plan.cols, p.plan.cols + n - 1, cp);
-  } else {
-    for (int k = 0; k < n - 1; ++k) cp[k] = k;
+    if (p.tree_modes) append_search(p);
   }
-  // the Gray walk takes its first columns among the class columns, so that
-  // its workgroups cover the class walk's subsets
-  nest_order(n, menu, sup, p.classed ? kClassBits : n - 1, cp, rp, p.nu, p.nu1, p.nu2);
+  int cp[64], nc = 0;
+  for (int l = 0; l < 3; ++l)
+    if (first[l] >= 0) cp[nc++] = first[l];
+  for (const int *k = p.classed ? p.plan.cols : natural, *end = k + B; k < end; ++k)
+    if (!chosen(*k)) cp[nc++] = *k;
   std::vector<double> x0(2 * (size_t)n);
   for (int j = 0; j < n; ++j) {
     x0[j] = p.x0[rp[j]];
