@@ -819,6 +819,9 @@ int run_chunked(int n, const Prepared& prep, bool use_cpu, int threads, perm_res
       out->kernel_ms += prev;
     }
     out->kernel_ms += chunk_ms;
+    // (the next chunked run records events on the stream: behind commands the
+    // runtime has not retired yet they cost it 12 us more than this wait)
+    HIP_TRY(hipStreamSynchronize(P.stream));
   }
   C.busy = false;
   return ok();
