@@ -1,6 +1,7 @@
 // skip_tree.hpp -- the skipping walk as a tree search (ryser_skip_tree.hip):
 // what its host plan and its kernel share (no HIP headers).
 #pragma once
+#include <stddef.h>
 #include <stdint.h>
 
 #include <vector>
