@@ -50,7 +50,8 @@ extern "C" {
  * zero, so no useful worst-case bound exists); err_est covers it.
  * err_est: three standard deviations of the error when roundings behave as
  * independent random errors, from moments the kernel measures (sums over
- * runs of consecutive terms of the squared absolute and signed run sums);
+ * runs of consecutive terms of the squared absolute and signed run sums; a
+ * search, which adds up every term in double-double, sums squared terms);
  * calibrated against the double-double and exact oracles.
  * mode: 0 = FP64 products (the fast kernel), 1 = double-double products
  * (integer-valued matrices: exact X, so the result rounds to the exact
@@ -72,18 +73,22 @@ typedef struct perm_result {
   double sum_lo;
   double abs_sum;
   double err_bound;
-  double kernel_ms;     /* device time of the Ryser kernel(s), HIP events */
+  double kernel_ms;     /* device time of the Ryser kernel(s): single-matrix path, from the
+                           walk's (or search's) begin to the end of the reduction by the
+                           kernels' 100 MHz counter, summed over the passes; else HIP events */
   double subsets;       /* Gray-code subsets evaluated (2^(n-1)) */
   int n;
   int status;
   int mode;
   int integral;         /* 1 if every entry is an integer (X is then exact) */
   double err_est;       /* statistical error estimate (independent roundings) */
-  int nu;               /* FP64 kernel: rows touched by Gray column 0 (pair/nested variant), or n */
+  int nu;               /* the Gray walk prepared for the matrix: rows touched by its column 0
+                           (pair/nested variant), or n.  Passes that are the class walk or the
+                           search do not use it; mode 2 has n. */
   double main_ms;       /* single-matrix path: device time of the first pass's walk or search */
   double main_subsets;  /* subsets that kernel evaluated (a search forms a part of them) */
-  int nu1;              /* FP64 kernel: rows touched by Gray columns 0-1 (nested variant), or n */
-  int nu2;              /* FP64 kernel: rows touched by Gray columns 0-2 (nested variant), or n */
+  int nu1;              /* the same for its columns 0-1 (nested variant), or n */
+  int nu2;              /* the same for its columns 0-2 (nested variant), or n */
   int certified;        /* 1: exact, or err_est <= 1e-10 |value| */
   int zero_pattern;     /* 1: no perfect matching in the nonzero pattern; value is exactly 0 */
   double clock_ghz;     /* single-matrix path: mean shader clock of the first pass's walk,
@@ -266,13 +271,15 @@ int perm_batch_get(const perm_batch* batch, perm_batch_tuning* out);
 
 /* ---- sparse skipper, ID 7: gpu_perman64_xshared_coalescing_mshared_skipper(
  * T* mat, int* rptrs, int* cols, int* cptrs, int* rows, T* cvals, int nov,
- * int grid_dim, int block_dim), gpu_exact_sparse.cu:1124.  Skips, per wave,
- * aligned runs of Gray steps whose terms are all zero (a row of x that is
- * zero and untouched by the run's columns); needs exact zeros, so it runs
- * for integer matrices and n >= 16 -- other inputs take the sparse path
- * (same sum).  x0 from the dense matrix, column updates from the CCS;
- * the CRS (rptrs/cols) is accepted and not needed.  perm_skip's result:
- * main_subsets = subsets actually walked (the rest were skipped). */
+ * int grid_dim, int block_dim), gpu_exact_sparse.cu:1124.  Searches the
+ * subsets without a zero row from the last column down or, where the rows cut
+ * too little, walks and skips, per wave, aligned runs of Gray steps whose
+ * terms are all zero (a row of x that is zero and untouched by the run's
+ * columns); both need exact zeros, so they run for integer matrices and n >=
+ * 16 -- other inputs take the sparse path (same sum).  x0 from the dense
+ * matrix, column updates from the CCS; the CRS (rptrs/cols) is accepted and
+ * not needed.  perm_skip's result: main_subsets = subsets formed by the search
+ * or actually walked (the rest were cut off or skipped). */
 int perm_skip(int dtype, const void* mat, const int* rptrs, const int* cols, const int* cptrs,
               const int* rows, const void* cvals, int nov, perm_result* out);
 double perm_xshared_coalescing_mshared_skipper_i32(const int* mat, const int* rptrs,

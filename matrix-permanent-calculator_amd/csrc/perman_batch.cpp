@@ -10,8 +10,9 @@
 // one persistent kernel per variant drains its group, the groups running
 // concurrently on several streams.  The FP64 pass of all matrices of the
 // class walk is one group per tree (class_tree.hpp) whatever their orders
-// (ryser_class.hip; an item is a workgroup there, over the same subsets).  The whole launch sequence (counter reset,
-// variant kernels, per-matrix reduction, result copy) is captured once in a
+// (ryser_class.hip; an item is a workgroup there, over the same subsets).
+// The whole launch sequence (counter reset, variant kernels, per-matrix
+// reduction, result copy) is captured once in a
 // hipGraph at the second run and replayed from then on (the first run after a
 // build launches directly: a batch computed once pays no capture).
 #include <hip/hip_runtime.h>
@@ -423,9 +424,10 @@ perm::ClassMatrix class_entry(const perm_batch* B, const Entry& e) {
 }
 
 // Device memory for `data` doubles, `split` doubles of expanded tables, nm
-// matrices, `items` items and `groups` variant groups: data, tables, matrices, items, item records, results, counters
-// (one per group, then one per matrix for double-double passes), and the
-// pinned result copy.
+// matrices, `items` items and `groups` variant groups: data, matrices, items,
+// item records, results, counters (one per group, then one per matrix for
+// double-double passes), tables, class descriptors, and the pinned result
+// copy.
 int alloc_device(perm_batch* B, size_t data, size_t split, size_t nm, size_t items,
                  size_t groups) {
   const size_t data_b = align256(data * sizeof(double));

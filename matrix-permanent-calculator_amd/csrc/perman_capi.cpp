@@ -4,10 +4,10 @@
 //
 // Host flow of one permanent (reference wrapper gpu_exact_dense.cu:640-699):
 // x-init + column store on the host, upload, Ryser kernel, grid reduction,
-// one record written by the last kernel into host memory, scale by 4(n&1)-2.  Unlike the reference,
-// device buffers come from a per-device cache (no cudaMalloc/cudaFree per
-// call), the launch geometry is chosen here, and every HIP status is
-// checked.
+// one record written by the last kernel into host memory, scale by
+// 4(n&1)-2.  Unlike the reference, device buffers come from a per-device
+// cache (no cudaMalloc/cudaFree per call), the launch geometry is chosen here,
+// and every HIP status is checked.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -195,8 +195,9 @@ int wait_run(perm_plan* P, uint64_t seq) {
 }
 
 // Device layout of a plan: column store, x0, the class walk's tables (these
-// three uploaded as one), result record, sample ids and records, then the workgroup records and their
-// weights (the last two are a separate arena in owning plans).
+// three uploaded as one), result record, sample ids and records, then the
+// workgroup records and their weights (the last two are a separate arena in
+// owning plans).
 struct PlanLayout {
   size_t col, x, cls, res, ids, vrec, part, z;
   size_t fixed() const { return col + x + cls + res + ids + vrec; }
@@ -487,7 +488,12 @@ void fill_result(const perm_plan* P, const perm::Partial& r, int mode, perm_resu
 // error is measured instead of modelled.  The FP64 pass left one record
 // per workgroup; the error of the sum is the sum of the workgroups' errors,
 // independent from one workgroup to the next (each has its own roundings;
-// the shared x0 rounding is stated separately).  kVerifyUnits workgroups
+// the shared x0 rounding is stated separately).  In the class walk they share
+// the rounded offsets of the class and walk columns, 2^5 + 2^w values per row
+// that move the sum through its derivatives, of either sign from one
+// workgroup to the next: over 32 matrices of n = 24 to 26, densities 0.2 to
+// 0.7, (sum of errors)^2 / sum of squared errors is 0.94 on the mean (1: no
+// correlation).  kVerifyUnits workgroups
 // are chosen with probability proportional to their modelled variance
 // z_i = Q_i + (2^(w-1) + h) Qr_i (systematic sampling; a workgroup whose
 // share exceeds one sampling interval is taken with certainty) and walked

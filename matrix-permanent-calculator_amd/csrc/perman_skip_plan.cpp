@@ -38,7 +38,9 @@ namespace {
 // 0.067.  The other levels: one column each 1.01, two 0.74, three 0.74 ms
 // (8x10, an earlier form of the kernel).
 int tree_top_bits(int b) { return std::min(b, std::max(18, std::min(23, b - 14))); }
-uint32_t tree_waves(int top_bits) { return top_bits >= 20 ? 8192u : 1u << std::min(12, top_bits - 6); }
+uint32_t tree_waves(int top_bits) {
+  return top_bits >= 20 ? 8192u : 1u << std::min(12, top_bits - 6);
+}
 int tree_level_bits(int left) { return left <= 20 ? 2 : 3; }
 
 // Share of the subsets of the columns of values v[0, d) at which start + sum

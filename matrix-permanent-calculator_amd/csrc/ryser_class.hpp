@@ -51,8 +51,8 @@ hipError_t launch_class_expand(const ClassMatrix* mats, uint32_t count, hipStrea
 // one block (lane_base / 64) of its matrix; `counter` must be zero; the
 // record of item i goes to partials[i].  max_n: largest order among them;
 // thin: the tree of all of them.
-hipError_t launch_class_batch(bool thin, const ClassMatrix* mats, const BatchItem* items, uint32_t begin,
-                              uint32_t end, uint32_t* counter, Partial* partials, int max_n,
-                              uint32_t grid, hipStream_t stream);
+hipError_t launch_class_batch(bool thin, const ClassMatrix* mats, const BatchItem* items,
+                              uint32_t begin, uint32_t end, uint32_t* counter,
+                              Partial* partials, int max_n, uint32_t grid, hipStream_t stream);
 
 }  // namespace perm

@@ -7,9 +7,9 @@
 // and the product of a class's rows is formed once per subset of T:
 // sum_T r_T 2^|T| additions and multiplications per 32 subsets instead of
 // 32 n each, plus the multiplications that join the classes' arrays
-// (class_tree.hpp).  At n = 40 and density 0.5 that is 18.6 FP64
-// instructions per subset against 47.5 of the nested walk it replaces (80 of
-// the plain one); a full matrix puts every row into the class of all five
+// (class_tree.hpp).  At n = 40 and density 0.5 that is 17.4 to 22.0 FP64
+// instructions per subset (thirteen matrices) against 47.5 of the nested walk
+// it replaces (80 of the plain one); a full matrix puts every row into the class of all five
 // columns and costs what the plain walk does.
 //
 // One lane's 32 subsets are a group: x_j = L_j + U_j + O_j(s & T), where
@@ -23,21 +23,24 @@
 //  * O_j(s) are the class columns' offsets, constant over the groups: scalar
 //    loads from a stream of 64-byte records in the order the rows are met.
 // Every x_j is thus at most nine roundings from exact (six lane columns),
-// whatever the length of the walk; the nested walk's X drifts by one rounding per step.
+// whatever the length of the walk; the nested walk's X drifts by one rounding
+// per step.
 //
 // The matrix's class sizes are loop counts, not template parameters: one
 // kernel serves every matrix of every order.  The loads of the next visit (a
 // record, two U entries, two LDS rows) are issued between the additions and
 // the multiplications of the current one.
 //
-// Bound: VALU issue (86 % of the cycles at n = 36, density 0.5; the rest is
-// waiting for the visit's scalar loads, which three waves per SIMD -- 150
+// Bound: VALU issue (density 0.5: 84 to 87 % of the cycles at n = 40, 81 % at
+// n = 36, 79 % at n = 32, and 61 % at n = 27, where a lane has four groups;
+// thin tree 78 %).  FP64 instructions are nine tenths of it; the rest of the
+// cycles wait for the visit's scalar loads, which three waves per SIMD -- 150
 // VGPRs: the arrays of one path through the tree are 63 doubles -- do not
-// quite cover; the thin tree's 120 allow four).  Thin against full tree, one
+// quite cover; the thin tree's 120 allow four.  Thin against full tree, one
 // pass: n = 27, density 0.2 35 against 43 us; n = 33, 0.3 1.44 against 1.98 ms;
-// n = 36, 0.2 10.7 against 14.7 ms; n = 34, 0.4 3.6 against 4.4 ms.  Tried and dropped: K = 4 (86 VGPRs, five waves, 94 % busy)
-// is 12 % slower, its 21.8 instructions per subset at n = 36 outweighing the
-// waves; visits of four rows of the small classes cost more scalar work than
+// n = 36, 0.2 10.7 against 14.7 ms; n = 34, 0.4 3.6 against 4.4 ms.  Tried and
+// dropped: K = 4 (86 VGPRs, five waves, 94 % busy) is 12 % slower, its 21.8
+// instructions per subset at n = 36 outweighing the waves; visits of four rows of the small classes cost more scalar work than
 // they hide; a second pair of chains in the final accumulation changes
 // nothing.
 #pragma once
@@ -167,7 +170,7 @@ __device__ __forceinline__ void class_rows(double (&P)[1 << M], RowFeed& f) {
   f.take();
   const uint32_t ctl = f.control();
   uint32_t more = ctl & 0xffu;
-if constexpr (M <= 2) {
+  if constexpr (M <= 2) {
     visit_pair<M, true>(P, f, ctl & 0x100u);
 #pragma clang loop unroll(disable)
     for (; more > 0; --more) {

@@ -168,8 +168,8 @@ inline double search_error_statement(double abs_sum_scaled, double running, int 
 
 // Expected error (err_est, three standard deviations) when roundings behave
 // as independent random errors, from the moments the kernels measure:
-// Q = sum over runs of 2^(R+5) consecutive terms of (sum of |T| in the run)^2
-// (>= sum T^2) and Qr = sum over runs of (signed run sum)^2, both scaled by
+// Q = sum over runs of 2^(R+5) consecutive terms (in the search: of one term)
+// of (sum of |T| in the run)^2 (>= sum T^2) and Qr = sum over runs of (signed run sum)^2, both scaled by
 // scale^2 (sq_scaled, run_scaled).
 //  * Product and accumulation roundings: about n roundings of relative size
 //    u/sqrt(12) per term, independent across terms: variance (n/12) u^2 Q.

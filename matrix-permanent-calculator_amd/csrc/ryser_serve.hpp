@@ -19,8 +19,9 @@
 // which the host reads in order.  A launch ends when the host sets `stop`,
 // or when every pass of its kind has completed and none of its waves has
 // claimed an item or seen a new pass for `idle` ticks: its waves leave
-// together, never one by one while work may still come.  The host launches it again (one captured graph) when it
-// publishes work and no launch of that kind is live.
+// together, never one by one while work may still come.  The host launches it
+// again (one captured graph) when it publishes work and no launch of that
+// kind is live.
 //
 // Orders are served by kernels of padded orders: a request of order n runs
 // the kernel of N = serve_padded_n(n) >= n, its start vector padded with

@@ -27,6 +27,14 @@
 //
 // The order of all sums is fixed by the launch: the same result every time.
 //
+// Error: x is exact, a term is a product of n rounded factors and joins the
+// lane's double-double sum at once, so its sq_sum is the sum of the squared
+// terms, runs of one term each.  Prefixes share their rounded products with
+// every term below them, whose signs alternate: against the double-double
+// pass, the errors of 40 matrices of n = 29 to 33, 0/1 and signed, are 0.002
+// to 0.43 of err_est, 0.18 on the quadratic mean (1/3 if err_est's model held
+// exactly).
+//
 // Bound: the latency of a step (stack, then four records at a time as scalar
 // loads) at eleven waves per compute unit (their stacks fill the LDS), 40 to
 // 100 steps per wave; the first level's 2^18..2^23 numbers are 5 to 30 us of
@@ -80,7 +88,8 @@ __device__ __forceinline__ bool complete_rows(Prefix<DDP>& p, RecordPtr records,
       const double value = __builtin_bit_cast(double, (uint64_t)r[k / 2][4 * (k % 2) + 1]);
       const double start = __builtin_bit_cast(double, (uint64_t)r[k / 2][4 * (k % 2) + 2]);
       const uint64_t set = p.set & mask;
-      const int count = __builtin_popcount((uint32_t)set) + __builtin_popcount((uint32_t)(set >> 32));
+      const int count =
+          __builtin_popcount((uint32_t)set) + __builtin_popcount((uint32_t)(set >> 32));
       if constexpr (SINGLE)
         x = __builtin_fma(value, (double)count, start);
       else
@@ -221,8 +230,9 @@ hipError_t launch_skip_tree(const SkipTreeLaunch& L, hipStream_t stream, const R
     return hipErrorInvalidValue;
   const size_t lds = (size_t)(L.n_levels - 1) * (L.mode ? 3 : 2) * kSkipLevelRoom * 8;
   const auto kernel =
-      L.mode ? L.single ? ryser_skip_tree_kernel<true, true> : ryser_skip_tree_kernel<true, false>
-             : L.single ? ryser_skip_tree_kernel<false, true> : ryser_skip_tree_kernel<false, false>;
+      L.mode ? (L.single ? ryser_skip_tree_kernel<true, true> : ryser_skip_tree_kernel<true, false>)
+             : (L.single ? ryser_skip_tree_kernel<false, true>
+                         : ryser_skip_tree_kernel<false, false>);
   kernel<<<L.waves, kWave, lds, stream>>>(L.records, L.levels, L.n_levels, L.top_bits, L.waves,
                                           L.partials, L.begin_tick);
   if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
