@@ -62,11 +62,18 @@ struct NestMenu {
   int max_k0;
   unsigned mask;
   int min_class_n;  // the class walk's smallest order for these kernels (0: none)
+  // a workgroup covers the same subsets in the class walk and in the Gray walk,
+  // also for integer matrices (for others always: their FP64 workgroups are
+  // measured by the Gray walk)
+  bool aligned;
 };
-constexpr NestMenu kMenuSingle = {kMaxDenseN, 0x1fu, kMinClassN};  // single matrices: all
+// single matrices: all
+constexpr NestMenu kMenuSingle = {kMaxDenseN, 0x1fu, kMinClassN, false};
+// and where ranges of workgroups are run by themselves or on the CPU
+constexpr NestMenu kMenuRanges = {kMaxDenseN, 0x1fu, kMinClassN, true};
 // batch and served kernels: shapes j = 0, 3, 4
-constexpr NestMenu kMenuBatch = {kMaxDenseN, 0x19u, kMinBatchClassN};
-constexpr NestMenu kMenuServe = {kMaxDenseN, 0x19u, 0};
+constexpr NestMenu kMenuBatch = {kMaxDenseN, 0x19u, kMinBatchClassN, false};
+constexpr NestMenu kMenuServe = {kMaxDenseN, 0x19u, 0, false};
 constexpr bool nest_menu_has(const NestMenu& m, int n, int k0, int j) {
   return k0 <= m.max_k0 && ((m.mask >> j) & 1u) && nest_menu_shape(n, k0, j).k0 != 0;
 }

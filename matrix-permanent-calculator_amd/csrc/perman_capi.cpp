@@ -920,14 +920,15 @@ int perm_max_n(void) { return perm::kMaxDenseN; }
 int perm_plan_dense(int dtype, const void* mat, int nov, perm_plan** plan) {
   if (!plan) return fail(PERM_ERR_ARG, "null plan");
   Prepared p;
-  if (int s = perm::prepare_dense(dtype, mat, nov, p)) return s;
+  if (int s = perm::prepare_dense(dtype, mat, nov, p, perm::kMenuRanges)) return s;
   return make_plan(nov, p, plan);
 }
 int perm_plan_sparse(int dtype, const void* mat, const int* cptrs, const int* rows,
                      const void* cvals, int nov, perm_plan** plan) {
   if (!plan) return fail(PERM_ERR_ARG, "null plan");
   Prepared p;
-  if (int s = perm::prepare_sparse(dtype, mat, cptrs, rows, cvals, nov, p)) return s;
+  if (int s = perm::prepare_sparse(dtype, mat, cptrs, rows, cvals, nov, p, perm::kMenuRanges))
+    return s;
   return make_plan(nov, p, plan);
 }
 int perm_plan_geometry(const perm_plan* P, int* walk_bits, int* high_bits,
@@ -1078,8 +1079,9 @@ int perm_chunked(int dtype, const void* mat, const int* cptrs, const int* rows,
                  int* cpu_chunks) {
   if (!out) return fail(PERM_ERR_ARG, "null result");
   Prepared p;
-  const int s = cptrs ? perm::prepare_sparse(dtype, mat, cptrs, rows, cvals, nov, p)
-                      : perm::prepare_dense(dtype, mat, nov, p);
+  const perm::NestMenu& menu = use_cpu ? perm::kMenuRanges : perm::kMenuSingle;
+  const int s = cptrs ? perm::prepare_sparse(dtype, mat, cptrs, rows, cvals, nov, p, menu)
+                      : perm::prepare_dense(dtype, mat, nov, p, menu);
   if (s) return s;
   return run_chunked(nov, p, use_cpu != 0, threads, out, cpu_chunks);
 }

@@ -461,13 +461,13 @@ static void append_search(Prepared& p) {
 }
 
 // Smallest orders at which the Gray walk of a class-walked matrix looks for its
-// first columns among all of them (6 us of host time): its passes in
-// double-double products (of integer matrices; of others only where a caller
-// asks for them) take a millisecond and more there, and the class columns,
-// chosen to overlap little, cost them up to 8 % (density 0.5, n = 32 4.65 ->
-// 4.83 ms, n = 33 8.64 -> 9.26 ms).  Below, and where that pass is a search,
-// the class columns are the candidates.
-constexpr int kMinFreeNestIntegral = 30, kMinFreeNestN = 32;
+// first columns among more than the class columns (up to 6 us of host time):
+// its passes in double-double products (of integer matrices; of others only
+// where a caller asks for them) take a millisecond and more there, and the
+// class columns, chosen to overlap little, cost them up to 8 % (density 0.5,
+// n = 32 4.65 -> 4.83 ms, n = 33 8.64 -> 9.26 ms).  Not where that pass is a
+// search.
+constexpr int kMinWideNestIntegral = 30, kMinWideNestN = 32;
 
 void finish_prepare(int n, const NestMenu& menu, std::vector<double>& cols, Prepared& p) {
   uint64_t sup[64];
@@ -487,15 +487,23 @@ void finish_prepare(int n, const NestMenu& menu, std::vector<double>& cols, Prep
   }
   const bool single = menu.mask == kMenuSingle.mask;
   if (p.classed && single && p.integral && n >= kMinTreeN) plan_search(n, sup, cols, p);
-  const bool free_nest = !p.classed || (!(p.tree_modes & 2u) &&
-                                        n >= (p.integral ? kMinFreeNestIntegral : kMinFreeNestN));
-  nest_order(n, menu, sup, free_nest ? natural : p.plan.cols, free_nest ? B : kClassBits, first,
-             rp, p.nu, p.nu1, p.nu2);
+  // the candidates: all columns, or those a workgroup of the class walk covers
+  // (class, walk and lane columns; a batch's has the lane columns at least)
+  // where one of the Gray walk has to cover the same: the cost of its shape is
+  // 1.00 to 1.03 times that of all columns' then, of the class columns' alone
+  // 1.00 to 1.07 (20 matrices of each order and density)
+  const int* cand = natural;
+  int pool = B;
+  if (p.classed && (n < (p.integral ? kMinWideNestIntegral : kMinWideNestN) || p.tree_modes & 2u)) {
+    cand = p.plan.cols;
+    pool = kClassBits;
+  } else if (p.classed && (menu.aligned || !p.integral)) {
+    cand = p.plan.cols;
+    pool = kClassBits + kClassLaneBits + (single ? class_walk_bits(n) : 0);
+  }
+  nest_order(n, menu, sup, cand, pool, first, rp, p.nu, p.nu1, p.nu2);
   const auto chosen = [&](int k) { return k == first[0] || k == first[1] || k == first[2]; };
   if (p.classed) {
-    // the Gray walk's first columns follow the class columns: both are among
-    // the first eight then, which a workgroup of either walk covers
-    std::stable_partition(p.plan.cols + kClassBits, p.plan.cols + B, chosen);
     // (a batch chooses its split later, and its tables are expanded on the
     // device)
     build_class_tables(p.plan, p.x0.data(), cols.data(), single ? class_walk_bits(n) : -1,

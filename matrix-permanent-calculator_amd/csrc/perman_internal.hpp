@@ -38,8 +38,8 @@ struct Prepared {
   bool integral = false;
   double product_bits = 1e9;  // integer_product_bits (integer matrices)
   // Class walk (the FP64 pass; see kMinClassN): its plan and tables.  The
-  // store above then has the class columns first, so
-  // the Gray kernels' workgroups cover the same subsets as the class walk's.
+  // store above then has the columns of a workgroup of it first, so the Gray
+  // kernels' workgroups cover the same subsets (NestMenu::aligned).
   bool classed = false;
   ClassPlan plan;
   ClassTables tables;
@@ -67,7 +67,8 @@ void fill_zero_result(int n, bool integral, perm_result& out);
 // log2 of the class walk's groups per lane for order n.
 int class_walk_bits(int n);
 // menu: the walk shapes the kernels that will run the matrix are compiled
-// for (kMenuSingle: single-matrix paths, kMenuBatch: batches, kMenuServe: the
+// for (kMenuSingle: single-matrix paths, kMenuRanges: those whose ranges of
+// workgroups may be run apart, kMenuBatch: batches, kMenuServe: the
 // server) and the orders prepared for the class walk.
 int prepare_dense(int dtype, const void* mat, int n, Prepared& p,
                   const NestMenu& menu = kMenuSingle);

@@ -1,7 +1,8 @@
 """Whole passes in double-double of matrices whose FP64 pass is the class walk:
-the Gray walk runs them on its own split and with the walk shape that all
-columns allow, as it does where the class walk is off (PERMAN_WALK_BITS at the
-Gray walk's own value), and ranges of workgroups keep the class walk's split."""
+the Gray walk runs them on its own split and, where a call is not cut into
+ranges of workgroups, with the walk shape that all columns allow, as it does
+where the class walk is off (PERMAN_WALK_BITS at the Gray walk's own value);
+ranges of workgroups keep the class walk's split."""
 import numpy as np
 import pytest
 
@@ -23,7 +24,7 @@ def runs(a, modes):
 @pytest.mark.parametrize("n,density,binary", [(27, 0.4, False), (27, 0.5, True), (29, 0.3, False),
                                               (31, 0.5, True), (32, 0.5, True), (32, 0.5, False),
                                               (33, 0.3, True), (33, 0.5, True)])
-def test_split_and_shape_are_the_gray_walks(monkeypatch, n, density, binary):
+def test_split_is_the_gray_walks(monkeypatch, n, density, binary):
     a = P.synthetic_matrix(n, density, 60 + n, binary=binary, full_support=True)
     if binary:
         a = a.astype(np.int32)
@@ -42,8 +43,23 @@ def test_split_and_shape_are_the_gray_walks(monkeypatch, n, density, binary):
             start = 0.0 if binary else n * 2.0 ** -106
             per_term = [(q.err_bound - start * abs(q.value)) / q.abs_sum for q in (r, w)]
             assert per_term[0] == pytest.approx(per_term[1], rel=1e-6, abs=0.0), (r, w)
-        if r.mode == 2 or n >= 31 and (binary or n >= 32):
-            assert (r.nu, r.nu1, r.nu2) == (w.nu, w.nu1, w.nu2)
+        if r.mode == 2:
+            assert (r.nu, r.nu1, r.nu2) == (n, n, n)
+
+
+@pytest.mark.parametrize("n", [30, 32, 33, 34])
+@pytest.mark.parametrize("density", [0.3, 0.5, 0.7])
+def test_shape_of_an_integer_matrix_is_the_gray_walks(monkeypatch, n, density):
+    """Dense, sparse and chunked calls (without the CPU): the shape their passes
+    with double-double products walk."""
+    a = P.synthetic_matrix(n, density, 60 + n, binary=True, full_support=True).astype(np.int32)
+    calls = [P.dense(a), P.sparse(a), P.chunked(a)[0]]
+    with monkeypatch.context() as m:
+        m.setenv("PERMAN_WALK_BITS", "10")
+        want = P.dense(a)
+    for r in calls:
+        assert (r.nu, r.nu1, r.nu2) == (want.nu, want.nu1, want.nu2), (r, want)
+        assert abs(r.value - want.value) <= r.stated + want.stated, (r, want)
 
 
 @pytest.mark.parametrize("n,density,binary", [(24, 0.5, False), (29, 0.3, False), (32, 0.5, True),
