@@ -30,17 +30,17 @@ os.environ.setdefault("OMP_PROC_BIND", "close")
 FULL_CPU_SET = os.sched_getaffinity(0)
 
 # HBM bytes per launch of the n=40 kernel on this workload: rocprofv3 FETCH_SIZE
-# + WRITE_SIZE (profiles/ryser_class.md, another n = 40 matrix of density 0.5):
-# 1708 KiB read + 65536 KiB written (2^20 workgroup records of 48 B, each one
-# 64-B line write).
-TRAFFIC_BYTES_N40 = (1707.6 + 65536.0) * 1024
+# + WRITE_SIZE (profiles/ryser_class.md): 1698 KiB read + 65536 KiB written
+# (2^20 workgroup records of 48 B, each one 64-B line write).
+TRAFFIC_BYTES_N40 = (1697.9 + 65536.0) * 1024
 FP64_PEAK_TFLOPS = 78.6
 # FP64 lane-instructions the chip issues per second (an FMA is one: half the
 # flop rate), in T/s
 FP64_ISSUE_PEAK = FP64_PEAK_TFLOPS / 2
 # FP64 instructions per subset the class walk needs for this workload's matrix
 # (its plan: row additions and products per column class, the classes' joins
-# and two FMAs per subset; all VALU instructions by counter: 21.1)
+# and two FMAs per subset; a CPU test holds it to the plan); all VALU
+# instructions by counter: 21.1 (profiles/ryser_class.md)
 FP64_INSTR_N40 = 19.34
 N = 40
 DENSITY = 0.5
